@@ -81,8 +81,19 @@ __device__ __forceinline__ int wave_entity(const Instance &I) {
   return __builtin_amdgcn_readfirstlane(block_entity0(I.n.WPB) + (int)(threadIdx.x >> 6));
 }
 __device__ __forceinline__ int lane() { return (int)(threadIdx.x & 63); }
-__device__ __forceinline__ float up1(float x) { return __shfl_up(x, 1, 64); }     // value of lane k-1
-__device__ __forceinline__ float dn1(float x) { return __shfl_down(x, 1, 64); }   // value of lane k+1
+// Value of lane k-1 (lane 0: its own) and k+1 (lane 63: its own): whole-wave
+// DPP shifts, one VALU move each.  The generic shuffles go through the LDS
+// permute unit, a round trip that also waits for every scalar load in flight
+// (four x1.40962 steps with their output: 24.41 -> 24.27 ms).
+// Call with every lane active (outside lane-dependent branches).
+__device__ __forceinline__ float up1(float x) {
+  const int v = __float_as_int(x);
+  return __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x138, 0xf, 0xf, false));  // wave_shr:1
+}
+__device__ __forceinline__ float dn1(float x) {
+  const int v = __float_as_int(x);
+  return __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x130, 0xf, 0xf, false));  // wave_shl:1
+}
 __device__ __forceinline__ float rdl(float x, int j) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), j));
 }
@@ -91,12 +102,6 @@ __device__ __forceinline__ float max0(float x) { return x > 0.0f ? x : 0.0f; }
 __device__ __forceinline__ float min0(float x) { return x < 0.0f ? x : 0.0f; }
 __device__ __forceinline__ float pmin(float a, float b) { return b < a ? b : a; }
 __device__ __forceinline__ float pmax(float a, float b) { return b > a ? b : a; }
-__device__ __forceinline__ int cl(int k) { return k < 0 ? 0 : (k > 63 ? 63 : k); }
-// Value of x held by lane cl(k + d): the same value a load of row[cl(k + d)]
-// gives, taken from the row already in registers.  Whole-wave shuffles: call
-// with every lane active (outside lane-dependent branches).
-__device__ __forceinline__ float lane_off(float x, int k, int d) { return __shfl(x, cl(k + d), 64); }
-
 // x / 12 with IEEE round-to-nearest.  For quotients in [2^-125, FLT_MAX] the
 // product by RN(1/12) plus one FMA residual correction is the correctly
 // rounded quotient (verified exhaustively over every binary32 x); zeros,
@@ -658,9 +663,9 @@ KBCOL(COLW_VC) k_vcoef(const Instance I, float dts, const float *__restrict__ ex
   __syncthreads();
   const float fzm = s_lev[0 * 64 + k], fzp = s_lev[1 * 64 + k], rdzu = s_lev[2 * 64 + k];
   const float rdzw = s_lev[3 * 64 + k], etp = s_lev[4 * 64 + k], ewp = s_lev[5 * 64 + k];
-  const float zkm = lane_off(zk, k, -1), exkm = lane_off(exk, k, -1), thkm = lane_off(thk, k, -1);
-  const float rdzwm = lane_off(rdzw, k, -1), etpm = lane_off(etp, k, -1);
-  const float ewpm = lane_off(ewp, k, -1), ewpp = lane_off(ewp, k, 1);
+  const float zkm = up1(zk), exkm = up1(exk), thkm = up1(thk);
+  const float rdzwm = up1(rdzw), etpm = up1(etp);
+  const float ewpm = up1(ewp), ewpp = dn1(ewp);
   float cofwr = 0.0f, cofwz = 0.0f, coftz = 0.0f;
   if (k >= 1 && k < L) {
     const float iz = fzm * zk + fzp * zkm;
@@ -994,8 +999,8 @@ KB k_sub_cell(const Instance I) {
   const float g = I.k.gravity;
   const float dpdz = MOIST ? (-g) * (rb * qt + rho_p * (1.0f + qt)) : (-g) * rho_p;
   // 0 - x, not -x: a zero divergence gives +0 (density_tendency_f32)
-  const float trho = (0.0f - acc) - rdzw * (lane_off(rw_k, k, 1) - rw_k);
-  const float pp_m1 = lane_off(pp_k, k, -1);
+  const float trho = (0.0f - acc) - rdzw * (dn1(rw_k) - rw_k);
+  const float pp_m1 = up1(pp_k);
   const float dpdzm = up1(dpdz);
   float erw = 0.0f;
   if (k >= 1 && k < L) {
@@ -1106,7 +1111,7 @@ __device__ __forceinline__ float tend_mom_edge(const Instance &I, int e, int k) 
   keep(u_k, rw0, rw1, pve, rho0, rho1, ke0, ke1, hd0, hd1, eru, fe, idc);
   SlotRow<NX> wt = wtr, ca = car, sa = sar;
   settle(wt, ca, sa);
-  const float u_m1 = lane_off(u_k, k, -1), u_m2 = lane_off(u_k, k, -2), u_p1 = lane_off(u_k, k, 1);
+  const float u_m1 = up1(u_k), u_m2 = up1(up1(u_k)), u_p1 = dn1(u_k);
   const float rwe = 0.5f * (rw0 + rw1);
   float wduz = 0.0f;
   if (k == 1 || k == L - 1) {
@@ -1313,10 +1318,10 @@ KB k_tend_cell(const Instance I) {
   settle(sgs);
   float sg[NE];
   slot_vals(sgs, sg);
-  const float th_m1 = lane_off(th_k, k, -1), th_m2 = lane_off(th_k, k, -2), th_p1 = lane_off(th_k, k, 1);
-  const float ths_m1 = lane_off(ths_k, k, -1), rwc_m1 = lane_off(rwc_k, k, -1);
-  const float ww_m1 = lane_off(ww_k, k, -1), ww_m2 = lane_off(ww_k, k, -2), ww_p1 = lane_off(ww_k, k, 1);
-  const float zz_m1 = lane_off(zz_k, k, -1);
+  const float th_m1 = up1(th_k), th_m2 = up1(up1(th_k)), th_p1 = dn1(th_k);
+  const float ths_m1 = up1(ths_k), rwc_m1 = up1(rwc_k);
+  const float ww_m1 = up1(ww_k), ww_m2 = up1(up1(ww_k)), ww_p1 = dn1(ww_k);
+  const float zz_m1 = up1(zz_k);
   float vf = 0.0f;
   if (k == 1) {
     vf = rwc_k * (fzm * th_k + fzp * th_m1);
@@ -1516,20 +1521,20 @@ KBCOL(COLW_AC) k_ac_cell(const Instance I, float dts, int store_old) {
       t = t - (flux * 0.5f) * (th1 + th0);
     }
   const float coftz_p = dn1(coftz);
-  const float ewm_p = lane_off(ewm, k, 1), ewp_p = lane_off(ewp, k, 1);
+  const float ewm_p = dn1(ewm), ewp_p = dn1(ewp);
   const float rwp_p = dn1(rwp);
   const float rs = ((rpp + dts * trho) + r) - (dts * rdzw) * (ewm_p * rwp_p - ewm * rwp);
   const float ts = ((rtpp + dts * trt) + t) - (dts * rdzw) * ((ewm_p * coftz_p) * rwp_p - (ewm * coftz) * rwp);
   if (k >= 1 && k < L) wwa = wwa + ewm * rwp;
   const float ts_m = up1(ts), rs_m = up1(rs), rtpp_m = up1(rtpp), rpp_m = up1(rpp), zk_m = up1(zk);
   const float cofwt_m = up1(cofwt);
-  const float etp_m = lane_off(etp, k, -1), etm_m = lane_off(etm, k, -1);
+  const float etp_m = up1(etp), etm_m = up1(etm);
   const float crho_m = up1(crho);
   // cofwr and the sub-diagonal a of the implicit w system at levels 1..L-1,
   // formed from zz, the level rows and the stored coefficients of levels k
   // and k-1 by the same operations as in k_vcoef (which stores cofwz, coftz
   // and cofwt for this kernel, and a only for export)
-  const float rdzw_m = lane_off(rdzw, k, -1), ewp_m = lane_off(ewp, k, -1), coftz_m = up1(coftz);
+  const float rdzw_m = up1(rdzw), ewp_m = up1(ewp), coftz_m = up1(coftz);
   float cofwr = 0.0f, a = 0.0f;
   if (k >= 1 && k < L) {
     cofwr = (0.5f * I.k.gravity) * (fzm * zk + fzp * zk_m);
@@ -1629,7 +1634,7 @@ __device__ __forceinline__ float recover_w_column(const Instance &I, int c, int 
   settle(sgs, sd);
   float sg[NE];
   slot_vals(sgs, sg);
-  const float zkm = lane_off(zk, k, -1);
+  const float zkm = up1(zk);
   if (hdiv_out) {
     // mass-flux divergence of the recovered ru (dynamics.py:86-121), next stage's hdiv
     float acc = 0.0f;
@@ -1941,7 +1946,7 @@ KB k_sc_cell(const Instance I, const float *__restrict__ qs, const float *__rest
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       if (sp0 + g >= NT) break;
-      const float q_m2 = lane_off(qk[g], k, -2), q_m1 = lane_off(qk[g], k, -1), q_p1 = lane_off(qk[g], k, 1);
+      const float q_m2 = up1(up1(qk[g])), q_m1 = up1(qk[g]), q_p1 = dn1(qk[g]);
       float vf = 0.0f;
       if (k >= 1 && k < L) vf = vflux(q_m2, q_m1, qk[g], q_p1, sw, k, L, fzm, fzp, I.k.coef3);
       const float vf_p = dn1(vf);
@@ -2116,7 +2121,7 @@ KB k_fct_cell1(const Instance I, const float *__restrict__ qs, float dt, const f
 #pragma unroll
     for (int s = 0; s < NE; ++s)
       if (s < n) hd = hd + (-(uh[s] * sd[s])) * ia;  // ((-csign)*uh)*dv, csign = +-1
-    const float wk_p = lane_off(wk, k, 1);
+    const float wk_p = dn1(wk);
     const float target = orho + dt * (hd - rdzw * (wk_p - wk));
     if (sp0 == 0 && k < L) {
       AT(I.b.target, c, k) = target;
@@ -2127,7 +2132,7 @@ KB k_fct_cell1(const Instance I, const float *__restrict__ qs, float dt, const f
       if (sp0 + g >= NT) break;
       const int sp = sp0 + g;
       const float qs_k = qsk[g];
-      const float qs_m2 = lane_off(qs_k, k, -2), qs_m1 = lane_off(qs_k, k, -1), qs_p1 = lane_off(qs_k, k, 1);
+      const float qs_m2 = up1(up1(qs_k)), qs_m1 = up1(qs_k), qs_p1 = dn1(qs_k);
       const float qo = qol[g] + qadd;
       const float qo_m = up1(qo), qo_p = dn1(qo);
       float a, b;
