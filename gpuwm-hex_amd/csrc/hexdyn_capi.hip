@@ -180,7 +180,6 @@ struct hexdyn_handle {
   int use_graphs = 1;
   int post_clamp = 1;  // end-of-step q < 0 -> 0 (0: scalars handed over unclamped)
   hipStream_t capture_stream = nullptr;
-  Side side{};  // the whole step's second stream and its fork/join events (created with the first step)
   struct Roles {  // host-side buffer roles and step flags
     Instance I;
     int in_step, cur_sub, start_is_pub, fresh_sub, fresh_step, exner_start, pp_pub;
@@ -289,6 +288,8 @@ Instance view(const hexdyn_handle *h, bool recovery) {
   // the whole-step sequence (step_view) stores only what a later kernel reads
   J.k.store_flux = 1;
   Work &B = J.b;
+  B.r_rho = B.c_rho; B.r_rt = B.c_rt; B.r_rw = B.c_rw; B.r_theta = B.theta; B.r_rho_p = B.rho_p;
+  B.r_rtheta_p = B.rtheta_p; B.r_exner = B.exner; B.r_pp = B.pp;
   if (h->start_is_pub) {
     B.s_rho = B.rho; B.s_rt = B.rt; B.s_ru = B.ru; B.s_rw = B.rw;
     B.s_theta = B.p_theta; B.s_exner = B.p_exner; B.s_rho_p = B.p_rho_p; B.s_rtheta_p = B.p_rtheta_p;
@@ -404,9 +405,6 @@ void hexdyn_destroy(hexdyn_handle *h) {
   if (!h) return;
   for (auto &g : h->graphs) (void)hipGraphExecDestroy(g.second.first);
   if (h->capture_stream) (void)hipStreamDestroy(h->capture_stream);
-  if (h->side.s) (void)hipStreamDestroy(h->side.s);
-  if (h->side.fork) (void)hipEventDestroy(h->side.fork);
-  if (h->side.join) (void)hipEventDestroy(h->side.join);
   for (void *p : h->allocs) (void)hipFree(p);
   delete h;
 }
@@ -1150,13 +1148,14 @@ int hexdyn_begin_subcycle(hexdyn_handle *h, int subcycle, void *stream) {
 
 int hexdyn_dyn_tend(hexdyn_handle *h, int stage, void *stream) {
   if (!h || stage < 1 || stage > 3) return HEXDYN_E_INVALID;
-  return NS_CALL(h, dyn_tend, view(h, false), stage, (hipStream_t)stream) ? HEXDYN_E_HIP : 0;
+  return NS_CALL(h, dyn_tend, view(h, false), stage, h->cur_sub, (hipStream_t)stream) ? HEXDYN_E_HIP : 0;
 }
 
 int hexdyn_acoustic_substep(hexdyn_handle *h, int stage, int small_step, void *stream) {
   if (!h || stage < 1 || stage > 3 || small_step < 1 || small_step > h->I.k.steps[stage - 1]) return HEXDYN_E_INVALID;
-  return NS_CALL(h, acoustic_substep, view(h, false), stage, small_step, 0, (hipStream_t)stream) ? HEXDYN_E_HIP
-                                                                                                   : 0;
+  return NS_CALL(h, acoustic_substep, view(h, false), stage, small_step, h->cur_sub, 0, (hipStream_t)stream)
+             ? HEXDYN_E_HIP
+             : 0;
 }
 
 int hexdyn_divergence_damping(hexdyn_handle *h, int stage, void *stream) {
@@ -1216,25 +1215,18 @@ Instance step_view(const hexdyn_handle *h, bool recovery) {
 // (begin_step's for the first stage of the first subcycle).
 int enqueue_step(hexdyn_handle *h, hipStream_t s) {
   const hexdyn_config &c = h->cfg;
-  if (!h->side.s &&
-      (hipStreamCreateWithFlags(&h->side.s, hipStreamNonBlocking) != hipSuccess ||
-       hipEventCreateWithFlags(&h->side.fork, hipEventDisableTiming) != hipSuccess ||
-       hipEventCreateWithFlags(&h->side.join, hipEventDisableTiming) != hipSuccess))
-    return HEXDYN_E_HIP;
   int rc = run_phase_begin_step(h, s, true);
-  // profiled steps stay on one stream, so each kernel's HIP-event time is its own
-  const Side *side = g_prof_on ? nullptr : &h->side;
   for (int sub = 1; rc == 0 && sub <= c.config_dynamics_split_steps; ++sub) {
     h->cur_sub = sub;
     rotate_subcycle(h, sub);
-    rc |= NS_CALL(h, begin_subcycle, step_view(h, false), sub, s, side);
+    rc |= NS_CALL(h, begin_subcycle, step_view(h, false), sub, s);
     for (int st = 1; rc == 0 && st <= 3; ++st) {
-      rc |= NS_CALL(h, dyn_tend, step_view(h, false), st, s, side);
+      rc |= NS_CALL(h, dyn_tend, step_view(h, false), st, sub, s);
       // divergence damping of substep ss is fused into the next edge pass:
       // the acoustic edge update of ss+1, or the edge recovery after the last substep
       const int dd = c.config_divergence_damping ? 1 : 0;
       for (int ss = 1; rc == 0 && ss <= h->I.k.steps[st - 1]; ++ss)
-        rc |= NS_CALL(h, acoustic_substep, step_view(h, false), st, ss, (dd && ss > 1) ? 1 : 0, s);
+        rc |= NS_CALL(h, acoustic_substep, step_view(h, false), st, ss, sub, (dd && ss > 1) ? 1 : 0, s);
       rc |= NS_CALL(h, recover, step_view(h, true), st, sub, dd, s);
       recovered(h, st);
       // the last stage's diagnostics would only feed a subcycle that does not
@@ -1367,7 +1359,7 @@ void drop_graphs(hexdyn_handle *h) {
 // block through LDS) and the edge-tiled flux pass (HX_TILE_E edges per block)
 bool column_kernel(const char *name) {
   return std::strcmp(name, "k_vcoef") == 0 || std::strcmp(name, "k_ac_cell") == 0 ||
-         std::strcmp(name, "k_diag_edge_flux_t") == 0;
+         std::strcmp(name, "k_col") == 0 || std::strcmp(name, "k_diag_edge_flux_t") == 0;
 }
 }  // namespace
 

@@ -108,6 +108,9 @@ struct Work {
   float *p_theta, *p_exner, *p_rho_p, *p_rtheta_p, *p_pp, *p_u, *p_w;
   // current state
   float *c_rho, *c_rt, *c_ru, *c_rw;
+  // where the recovery at the end of a stage writes (set per launch: until a
+  // subcycle's first recovery the current fields are read elsewhere)
+  float *r_rho, *r_rt, *r_rw, *r_theta, *r_rho_p, *r_rtheta_p, *r_exner, *r_pp;
   // subcycle start copies
   float *s_rho, *s_rt, *s_ru, *s_rw, *s_theta, *s_rho_p, *s_rtheta_p, *s_exner;
   // moist coefficients
@@ -160,7 +163,8 @@ struct Consts {
                                  // vorticity of rk 1-2; the damped ru_p of stages 1-2; atri)
   int fused;                     // whole-step launch sequence: the next stage's theta/w edge fluxes
                                  // ride on the edge diagnostics, the first acoustic edge update on
-                                 // the momentum tendency, and ru_avg is kept only where read back
+                                 // the momentum tendency, a stage's column work is one pass, and
+                                 // ru_avg is kept only where read back
   float strain_scale, ceiling;   // (c_s*len)^2, (0.01*len^2)/dt
   int ray_levels;                // Rayleigh damping of u over the top ray_levels levels (0: off)
   float ray_inverse;             // 1/(levels*(days*86400))
@@ -201,23 +205,14 @@ struct Instance {
   const LaunchTune *tune;  // host pointer to the handle's launch table
 };
 
-// A second stream (default priority) for the implicit coefficients, which
-// depend on none of the kernels launched beside them: forked from the
-// caller's stream and joined back to it with the two events, so in a
-// captured step they are a parallel branch of the graph.  Null: one stream.
-struct Side {
-  hipStream_t s;
-  hipEvent_t fork, join;
-};
-
 // Phase entry points, compiled once with strict binary32 numerics
 // (no contraction) and once with fused multiply-adds allowed.
 #define HEXDYN_PHASES(NS)                                                 \
   namespace NS {                                                          \
   int begin_step(const Instance &I, hipStream_t s);                       \
-  int begin_subcycle(const Instance &I, int sub, hipStream_t s, const Side *side = nullptr); \
-  int dyn_tend(const Instance &I, int stage, hipStream_t s, const Side *side = nullptr);     \
-  int acoustic_substep(const Instance &I, int stage, int ss, int damp_prev, hipStream_t s); \
+  int begin_subcycle(const Instance &I, int sub, hipStream_t s);          \
+  int dyn_tend(const Instance &I, int stage, int sub, hipStream_t s);     \
+  int acoustic_substep(const Instance &I, int stage, int ss, int sub, int damp_prev, hipStream_t s); \
   int divergence_damping(const Instance &I, int stage, hipStream_t s);    \
   int recover(const Instance &I, int stage, int sub, int damp, hipStream_t s); \
   int solve_diagnostics(const Instance &I, int rk, hipStream_t s);        \

@@ -14,8 +14,8 @@
  * renumbered so each XCD (hardware assigns block b to XCD b % 8) works on a
  * contiguous range of the space-filling-curve order and its L2 sees the
  * neighbour rows it needs.  Vertical neighbours come from cross-lane moves;
- * the serial column recurrences (Thomas sweep, implicit coefficients) walk
- * the lanes with readlane so their arithmetic order is the reference's.
+ * the serial column recurrences (Thomas sweep, implicit coefficients) run one
+ * column per lane out of LDS, in the reference's arithmetic order.
  *
  * Reference operators (operation order per element):
  *   solve diagnostics  cuda_horizontal_v841.py:67-200, diagnostics.py:95-306
@@ -192,6 +192,9 @@ __device__ __forceinline__ void settle(R &...rows) {
 // issued.  Without it the compiler may issue one index table's loads only
 // after waiting for another's, one more dependent round trip.
 __device__ __forceinline__ void fence(int x) { asm volatile("" ::"s"(x)); }
+// Loads after this point are issued after it (a pass in several parts holds
+// back the rows of the next part, whose registers the part before frees).
+__device__ __forceinline__ void hold_loads() { asm volatile("" ::: "memory"); }
 // A per-entity value read by a vector load (every lane the same address) for
 // the same reason; the zero offset is opaque, so the load stays a vector load.
 __device__ __forceinline__ float uni_load(const float *__restrict__ p) {
@@ -211,7 +214,7 @@ inline int nblocks(int n, int wpb) { return (n + wpb - 1) / wpb; }
 // overlap their loads with the others' sweeps: 57 -> 53 us; the
 // coefficients were 1 us slower at 8).
 constexpr int COLW_VC = 16;  // k_vcoef
-constexpr int COLW_AC = 8;   // k_ac_cell (at least 7: its waves 0-6 stage the level rows)
+constexpr int COLW_AC = 8;   // k_ac_cell and k_col (one level row staged by each wavefront)
 constexpr int COLP = 65;
 // The column blocks of a CU need every SIMD to hold 8 wavefronts: the
 // register budget is capped for that (at 7 a CU would hold one block of 16).
@@ -225,6 +228,98 @@ __device__ __forceinline__ void stage_levels(float *s_lev, const float *const (&
 #pragma unroll
   for (int j = 0; j < N; ++j)
     if (w == j) s_lev[j * 64 + k] = rows[j][k];
+}
+
+// 1 / x with IEEE round-to-nearest.  For |x| in [2^-100, 2^100] the hardware
+// reciprocal with one FMA correction is the correctly rounded quotient
+// (verified exhaustively over every binary32 x of that range); other inputs
+// take the division itself.
+__device__ __forceinline__ float recip(float x) {
+  const float a = fabsf(x);
+  if (a >= 0x1p-100f && a <= 0x1p100f) {
+    const float y0 = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, y0, 1.0f), y0, y0);
+  }
+  return 1.0f / x;
+}
+
+// A block of U levels of a column's LDS rows in registers.  Levels past the
+// column's last are read too (rows hold COLP >= 8 * ceil(L / 8) floats) and
+// used by nobody.
+template <int U>
+__device__ __forceinline__ void sweep_load(float (&r)[U], const float *p, int j) {
+#pragma unroll
+  for (int u = 0; u < U; ++u) r[u] = p[j + u];
+}
+// The serial recurrences of one column (lane = column).  Each level's step
+// waits for the one before, so the time is the chain's: the LDS reads of a
+// block of levels are issued together ahead of the block's chain, and the
+// levels left after the whole blocks form one block too (m of its U levels)
+// instead of a loop that pays the LDS latency at every level.
+// Thomas sweeps (acoustic_v841.py:296-565): forward for levels 1..L-1, back
+// substitution for levels L-1..0.
+template <bool WHOLE, int U>
+__device__ __forceinline__ float sweep_up(float *x, const float *pd, const float *pl, int j, int m, float p) {
+  float xv[U], dv[U], lv[U];
+  sweep_load(xv, x, j);
+  sweep_load(dv, pd, j);
+  sweep_load(lv, pl, j);
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (WHOLE || u < m) x[j + u] = p = (xv[u] - dv[u] * p) * lv[u];
+  return p;
+}
+template <bool WHOLE, int U>
+__device__ __forceinline__ float sweep_down(float *x, const float *pg, int j, int m, float p) {
+  float xv[U], gv[U];
+  sweep_load(xv, x, j);
+  sweep_load(gv, pg, j);
+#pragma unroll
+  for (int u = U - 1; u >= 0; --u)
+    if (WHOLE || u < m) x[j + u] = p = xv[u] - gv[u] * p;
+  return p;
+}
+__device__ __forceinline__ void thomas_sweeps(float *x, const float *pd, const float *pl, const float *pg, int L) {
+  constexpr int U = 8;
+  float p = x[0];
+  int j = 1;
+  for (; j + U <= L; j += U) p = sweep_up<true, U>(x, pd, pl, j, U, p);
+  if (j < L) sweep_up<false, U>(x, pd, pl, j, L - j, p);
+  p = x[L];
+  j = L / U * U;
+  if (j < L) p = sweep_down<false, U>(x, pg, j, L - j, p);
+  for (j -= U; j >= 0; j -= U) p = sweep_down<true, U>(x, pg, j, U, p);
+}
+// alpha/gamma recurrence up the column (acoustic_v841.py:81-233): alpha over
+// pa, gamma over pb; returns 1 where a denominator vanishes.  Blocks of 4: the
+// division dominates a level's chain, and the fused column pass has few
+// registers to spare.
+template <bool WHOLE, int U>
+__device__ __forceinline__ float sweep_coef(float *pa, float *pb, const float *pc, int j, int m, float dts2, float gm,
+                                            int &singular) {
+  float av[U], bv[U], cv[U];
+  sweep_load(av, pa, j);
+  sweep_load(bv, pb, j);
+  sweep_load(cv, pc, j);
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (WHOLE || u < m) {
+      const float den = 1.0f + dts2 * (bv[u] - av[u] * gm);
+      if (den == 0.0f) singular = 1;
+      const float al = recip(den);
+      gm = (dts2 * cv[u]) * al;
+      pa[j + u] = al;
+      pb[j + u] = gm;
+    }
+  return gm;
+}
+__device__ __forceinline__ int coef_sweep(float *pa, float *pb, const float *pc, int L, float dts2) {
+  constexpr int U = 4;
+  float gm = 0.0f;
+  int singular = 0, j = 1;
+  for (; j + U <= L; j += U) gm = sweep_coef<true, U>(pa, pb, pc, j, U, dts2, gm, singular);
+  if (j < L) sweep_coef<false, U>(pa, pb, pc, j, L - j, dts2, gm, singular);
+  return singular;
 }
 
 // Gather helpers.  Connectivity rows are padded to fixed widths (NE = maxEdges
@@ -639,6 +734,65 @@ KB k_moist_edge(const Instance I) {
 }
 
 // ------------------------------------------------------ implicit coefficients
+// The rows the coefficients of a column are formed from, and the coefficients
+// of a level.
+struct CoefIn {
+  float zk, exk, thk, cqw, qt, rtpk, rbk, rtbk, exbk;
+};
+struct CoefOut {
+  float cofwz, coftz, cofwt, a, b, cc;
+};
+__device__ __forceinline__ CoefIn coef_rows(const Instance &I, const float *__restrict__ exn,
+                                            const float *__restrict__ theta, const float *__restrict__ rtp, int c,
+                                            int k) {
+  return {AT(I.z.zz, c, k),   AT(exn, c, k),  AT(theta, c, k), AT(I.b.cqw, c, k), AT(I.b.qtot, c, k),
+          AT(rtp, c, k),      AT(I.z.rb, c, k), AT(I.z.rtb, c, k), AT(I.z.exb, c, k)};
+}
+// Level rows: fzm, fzp, rdzu, rdzw, etp, ewp of level k; neighbours by lane moves.
+__device__ __forceinline__ CoefOut coef_system(const Instance &I, const CoefIn &r, int k, float fzm, float fzp,
+                                               float rdzu, float rdzw, float etp, float ewp) {
+  const int L = I.n.L;
+  const float g = I.k.gravity, rcv = I.k.rcv, c2 = I.k.c2;
+  const float zkm = up1(r.zk), exkm = up1(r.exk), thkm = up1(r.thk);
+  const float rdzwm = up1(rdzw), etpm = up1(etp);
+  const float ewpm = up1(ewp), ewpp = dn1(ewp);
+  float cofwr = 0.0f, cofwz = 0.0f, coftz = 0.0f;
+  if (k >= 1 && k < L) {
+    const float iz = fzm * r.zk + fzp * zkm;
+    cofwr = (0.5f * g) * iz;
+    cofwz = (((c2 * iz) * rdzu) * r.cqw) * (fzm * r.exk + fzp * exkm);
+    coftz = fzm * r.thk + fzp * thkm;
+  }
+  float cofwt = 0.0f;
+  if (k < L)
+    cofwt = (((((((0.5f * rcv) * r.zk) * g) * r.rbk) / (1.0f + r.qt)) * r.exk) / ((r.rtbk + r.rtpk) * r.exbk));
+  const float coftz_m = up1(coftz), coftz_p = dn1(coftz), cofwt_m = up1(cofwt);
+  float a = 0.0f, b = 1.0f, cc = 0.0f;
+  if (k >= 1 && k < L) {
+    a = (((-cofwz) * coftz_m) * rdzwm) * zkm + cofwr * rdzwm - (cofwt_m * coftz_m) * rdzwm;
+    a = (a * etpm) * ewpm;
+    b = (cofwz * coftz) * ((etp * rdzw) * r.zk + (etpm * rdzwm) * zkm) -
+        coftz * ((etp * cofwt) * rdzw - (etpm * cofwt_m) * rdzwm) + cofwr * (etp * rdzw - etpm * rdzwm);
+    b = b * ewp;
+    cc = (((-cofwz) * coftz_p) * rdzw) * r.zk - cofwr * rdzw + (cofwt * coftz_p) * rdzw;
+    cc = (cc * etp) * ewpp;
+    if (k == L - 1) cc = 0.0f;
+  }
+  return {cofwz, coftz, cofwt, a, b, cc};
+}
+__device__ __forceinline__ void store_coefs(const Instance &I, int c, int k, float coftz, float cofwt, float cofwz,
+                                            float a, float alpha, float gamma) {
+  if (k > I.n.L) return;
+  AT(I.b.coftz, c, k) = coftz;
+  if (k < I.n.L) {
+    AT(I.b.cofwz, c, k) = cofwz;
+    AT(I.b.cofwt, c, k) = cofwt;
+    if (I.k.store_flux) AT(I.b.atri, c, k) = a;  // export only: the acoustic column update forms a itself
+    AT(I.b.alpha, c, k) = alpha;
+    AT(I.b.gamma, c, k) = gamma;
+  }
+}
+
 KBCOL(COLW_VC) k_vcoef(const Instance I, float dts, const float *__restrict__ exn, const float *__restrict__ theta,
               const float *__restrict__ rtp) {
   constexpr int COLW = COLW_VC;
@@ -650,77 +804,28 @@ KBCOL(COLW_VC) k_vcoef(const Instance I, float dts, const float *__restrict__ ex
   const int c = live ? c0 : 0;  // every wave reaches the barriers
   const int k = lane();
   const int L = I.n.L;
-  const float g = I.k.gravity, rcv = I.k.rcv, c2 = I.k.c2;
-  const float dts2 = dts * dts;
   // every load first; the level k-1 and k+1 values come from neighbouring lanes
-  const float zk = AT(I.z.zz, c, k), exk = AT(exn, c, k), thk = AT(theta, c, k);
-  const float cqw = AT(I.b.cqw, c, k), qt = AT(I.b.qtot, c, k), rtpk = AT(rtp, c, k);
-  const float rbk = AT(I.z.rb, c, k), rtbk = AT(I.z.rtb, c, k), exbk = AT(I.z.exb, c, k);
+  const CoefIn r = coef_rows(I, exn, theta, rtp, c, k);
   {
     const float *const lev[6] = {I.z.fzm, I.z.fzp, I.z.rdzu, I.z.rdzw, I.z.etp, I.z.ewp};
     stage_levels<6>(s_lev, lev, w, k);
   }
   __syncthreads();
-  const float fzm = s_lev[0 * 64 + k], fzp = s_lev[1 * 64 + k], rdzu = s_lev[2 * 64 + k];
-  const float rdzw = s_lev[3 * 64 + k], etp = s_lev[4 * 64 + k], ewp = s_lev[5 * 64 + k];
-  const float zkm = up1(zk), exkm = up1(exk), thkm = up1(thk);
-  const float rdzwm = up1(rdzw), etpm = up1(etp);
-  const float ewpm = up1(ewp), ewpp = dn1(ewp);
-  float cofwr = 0.0f, cofwz = 0.0f, coftz = 0.0f;
-  if (k >= 1 && k < L) {
-    const float iz = fzm * zk + fzp * zkm;
-    cofwr = (0.5f * g) * iz;
-    cofwz = (((c2 * iz) * rdzu) * cqw) * (fzm * exk + fzp * exkm);
-    coftz = fzm * thk + fzp * thkm;
-  }
-  float cofwt = 0.0f;
-  if (k < L) cofwt = (((((((0.5f * rcv) * zk) * g) * rbk) / (1.0f + qt)) * exk) / ((rtbk + rtpk) * exbk));
-  const float coftz_m = up1(coftz), coftz_p = dn1(coftz), cofwt_m = up1(cofwt);
-  float a = 0.0f, b = 1.0f, cc = 0.0f;
-  if (k >= 1 && k < L) {
-    a = (((-cofwz) * coftz_m) * rdzwm) * zkm + cofwr * rdzwm - (cofwt_m * coftz_m) * rdzwm;
-    a = (a * etpm) * ewpm;
-    b = (cofwz * coftz) * ((etp * rdzw) * zk + (etpm * rdzwm) * zkm) -
-        coftz * ((etp * cofwt) * rdzw - (etpm * cofwt_m) * rdzwm) + cofwr * (etp * rdzw - etpm * rdzwm);
-    b = b * ewp;
-    cc = (((-cofwz) * coftz_p) * rdzw) * zk - cofwr * rdzw + (cofwt * coftz_p) * rdzw;
-    cc = (cc * etp) * ewpp;
-    if (k == L - 1) cc = 0.0f;
-  }
-  // alpha/gamma recurrence up the column (acoustic_v841.py:81-233), lane = cell
-  s_a[w * COLP + k] = a;
-  s_b[w * COLP + k] = b;
-  s_c[w * COLP + k] = cc;
+  const CoefOut o = coef_system(I, r, k, s_lev[0 * 64 + k], s_lev[1 * 64 + k], s_lev[2 * 64 + k], s_lev[3 * 64 + k],
+                                s_lev[4 * 64 + k], s_lev[5 * 64 + k]);
+  s_a[w * COLP + k] = o.a;
+  s_b[w * COLP + k] = o.b;
+  s_c[w * COLP + k] = o.cc;
   __syncthreads();
   if (w == 0 && k < COLW) {
-    float *pa = s_a + k * COLP, *pb = s_b + k * COLP;
-    const float *pc = s_c + k * COLP;
-    float gm = 0.0f;
-    int singular = 0;
-    for (int j = 1; j < L; ++j) {
-      const float den = 1.0f + dts2 * (pb[j] - pa[j] * gm);
-      if (den == 0.0f) singular = 1;
-      const float al = 1.0f / den;
-      gm = (dts2 * pc[j]) * al;
-      pa[j] = al;
-      pb[j] = gm;
-    }
+    const int singular = coef_sweep(s_a + k * COLP, s_b + k * COLP, s_c + k * COLP, L, dts * dts);
     if (singular && block_entity0(COLW) + k < I.n.C) set_flag(I.b.flag);
   }
   __syncthreads();
   const bool inner = k >= 1 && k < L;
-  const float alpha = inner ? s_a[w * COLP + k] : 0.0f;
-  const float gamma = inner ? s_b[w * COLP + k] : 0.0f;
-  if (live && k <= L) {
-    AT(I.b.coftz, c, k) = coftz;
-    if (k < L) {
-      AT(I.b.cofwz, c, k) = cofwz;
-      AT(I.b.cofwt, c, k) = cofwt;
-      if (I.k.store_flux) AT(I.b.atri, c, k) = a;  // export only: k_ac_cell forms a itself
-      AT(I.b.alpha, c, k) = alpha;
-      AT(I.b.gamma, c, k) = gamma;
-    }
-  }
+  if (live)
+    store_coefs(I, c, k, o.coftz, o.cofwt, o.cofwz, o.a, inner ? s_a[w * COLP + k] : 0.0f,
+                inner ? s_b[w * COLP + k] : 0.0f);
 }
 
 // ------------------------------------------------------- horizontal mixing
@@ -1274,15 +1379,117 @@ KB k_tend_flux(const Instance I) {
   store_edge_flux<CORR>(I, e, k, tend_flux_values<NE, CORR>(I, e, k));
 }
 
-// CORR: stages 2 and 3 (the theta RK correction flux); MIX: horizontal
-// mixing on (its theta increment is added)
+// Theta and w tendencies of one stage in a cell's column.  CORR: stages 2 and
+// 3 (the theta RK correction flux); MIX: horizontal mixing on (its theta
+// increment is added).  The column rows are read once; vertical neighbours by
+// shuffles.
+template <int NE>
+struct ThetaIn {
+  float th, ths, rwc, rws, eth, prt;
+  float fth[NE], fco[NE];
+};
+template <int NE>
+struct WIn {
+  float ww, zz, erw;
+  float fwv[NE], tru[NE], zb[NE], zb3[NE];
+};
+template <int NE, bool CORR, bool MIX>
+__device__ __forceinline__ void theta_rows(const Instance &I, const int (&e)[NE], int c, int k, ThetaIn<NE> &t) {
+  t.th = AT(I.b.theta, c, k);
+  t.ths = AT(I.b.s_theta, c, k);
+  t.rwc = AT(I.b.c_rw, c, k);
+  t.rws = AT(I.b.s_rw, c, k);
+  t.eth = MIX ? AT(I.b.euler_theta, c, k) : 0.0f;
+#pragma unroll
+  for (int s = 0; s < NE; ++s) {
+    t.fth[s] = AT(I.b.fth, e[s], k);
+    t.fco[s] = CORR ? AT(I.b.fcorr, e[s], k) : 0.0f;
+  }
+  t.prt = I.k.physics ? AT(I.b.phys_rt, c, k) : 0.0f;  // the buffer exists with physics only
+}
+template <int NE>
+__device__ __forceinline__ void w_rows(const Instance &I, const int (&e)[NE], int c, int k, WIn<NE> &t) {
+  t.ww = AT(I.b.w, c, k);
+  t.zz = AT(I.z.zz, c, k);
+  t.erw = AT(I.b.euler_rw, c, k);
+#pragma unroll
+  for (int s = 0; s < NE; ++s) {
+    t.fwv[s] = AT(I.b.fw, e[s], k);
+    t.tru[s] = AT(I.b.tend_ru, e[s], k);
+    t.zb[s] = AT(I.z.zb, c * NE + s, k);
+    t.zb3[s] = AT(I.z.zb3, c * NE + s, k);
+  }
+}
+template <int NE, bool CORR, bool MIX>
+__device__ __forceinline__ float theta_tendency(const Instance &I, const ThetaIn<NE> &t, const float (&sg)[NE],
+                                                float ia, int n, int k, float fzm, float fzp, float rdzw) {
+  const int L = I.n.L;
+  const float coef = I.k.coef3;
+  const float th_m1 = up1(t.th), th_m2 = up1(th_m1), th_p1 = dn1(t.th), ths_m1 = up1(t.ths);
+  float vf = 0.0f;
+  if (k == 1) {
+    vf = t.rwc * (fzm * t.th + fzp * th_m1);
+    vf = vf + (t.rws - t.rwc) * (fzm * t.ths + fzp * ths_m1);
+  } else if (k >= 2 && k < L - 1) {
+    vf = flux3(th_m2, th_m1, t.th, th_p1, t.rwc, coef);
+    vf = vf + (t.rws - t.rwc) * (fzm * t.ths + fzp * ths_m1);
+  } else if (k == L - 1) {
+    vf = t.rws * (fzm * t.th + fzp * th_m1);
+  }
+  const float vf_p = dn1(vf);
+  float r = 0.0f;
+#pragma unroll
+  for (int s = 0; s < NE; ++s)
+    if (s < n) r = r - sg[s] * t.fth[s];
+  if (CORR) {
+#pragma unroll
+    for (int s = 0; s < NE; ++s)
+      if (s < n) r = r - sg[s] * t.fco[s];
+  }
+  r = r * ia;
+  const float trt = r - rdzw * (vf_p - vf);
+  const float tmix = MIX ? trt + t.eth : trt;
+  return I.k.physics ? tmix + t.prt : tmix;
+}
+template <int NE>
+__device__ __forceinline__ float w_tendency(const Instance &I, const WIn<NE> &t, float rwc, const float (&sg)[NE],
+                                            float ia, int n, int k, float fzm, float fzp, float rdzu) {
+  const int L = I.n.L;
+  const float rwc_m1 = up1(rwc);
+  const float ww_m1 = up1(t.ww), ww_m2 = up1(ww_m1), ww_p1 = dn1(t.ww), zz_m1 = up1(t.zz);
+  float wf = 0.0f;
+  if (k == 1 || k == L - 1) {
+    wf = (0.25f * (rwc + rwc_m1)) * (t.ww + ww_m1);
+  } else if (k >= 2 && k < L - 1) {
+    wf = flux3(ww_m2, ww_m1, t.ww, ww_p1, 0.5f * (rwc + rwc_m1), 1.0f);
+  }
+  const float wf_p = dn1(wf);
+  float q = 0.0f;
+#pragma unroll
+  for (int s = 0; s < NE; ++s)
+    if (s < n) q = q - sg[s] * t.fwv[s];
+  q = q * ia;
+  q = q - rdzu * (wf_p - wf);
+  q = q + t.erw;
+#pragma unroll
+  for (int s = 0; s < NE; ++s)
+    if (s < n) {
+      const float tk = t.tru[s];
+      const float flux = sg[s] * (fzm * tk + fzp * up1(tk));
+      q = q - (t.zb[s] + cs1(tk) * t.zb3[s]) * flux;
+    }
+  return k >= 1 && k < L ? q * (fzm * t.zz + fzp * zz_m1) : 0.0f;
+}
+__device__ __forceinline__ void store_tend(const Instance &I, int c, int k, float rt, float rw) {
+  if (k < I.n.L) AT(I.b.tend_rt, c, k) = rt;
+  if (k <= I.n.L) AT(I.b.tend_rw, c, k) = rw;
+}
+
 template <int NE, bool CORR, bool MIX>
 KB k_tend_cell(const Instance I) {
   const int c = wave_entity(I);
   if (c >= I.n.C) return;
   const int k = lane();
-  const int L = I.n.L;
-  const float coef = I.k.coef3;
   const int n = I.m.neoc[c];
   int e[NE];
 #pragma unroll
@@ -1291,92 +1498,19 @@ KB k_tend_cell(const Instance I) {
   const float ia = uni_load(I.m.invarea + c);
   const float fzm = AT(I.z.fzm, 0, k), fzp = AT(I.z.fzp, 0, k);
   const float rdzw = AT(I.z.rdzw, 0, k), rdzu = AT(I.z.rdzu, 0, k);
-  // the column rows, read once; vertical neighbours by shuffles
-  const float th_k = AT(I.b.theta, c, k), ths_k = AT(I.b.s_theta, c, k);
-  const float rwc_k = AT(I.b.c_rw, c, k), rws_k = AT(I.b.s_rw, c, k), ww_k = AT(I.b.w, c, k);
-  const float zz_k = AT(I.z.zz, c, k), erw_k = AT(I.b.euler_rw, c, k);
-  const float eth_k = MIX ? AT(I.b.euler_theta, c, k) : 0.0f;
-  float fth[NE], fco[NE], fwv[NE], tru[NE], zb[NE], zb3[NE];
-#pragma unroll
-  for (int s = 0; s < NE; ++s) {
-    zb[s] = AT(I.z.zb, c * NE + s, k);
-    zb3[s] = AT(I.z.zb3, c * NE + s, k);
-  }
 #pragma unroll
   for (int s = 0; s < NE; ++s) fence(e[s]);
-#pragma unroll
-  for (int s = 0; s < NE; ++s) {
-    fth[s] = AT(I.b.fth, e[s], k);
-    fwv[s] = AT(I.b.fw, e[s], k);
-    tru[s] = AT(I.b.tend_ru, e[s], k);
-    fco[s] = CORR ? AT(I.b.fcorr, e[s], k) : 0.0f;
-  }
-  const float prt_k = I.k.physics ? AT(I.b.phys_rt, c, k) : 0.0f;  // the buffer exists with physics only
-  keep(fth, fwv, tru, zb, zb3);
-  if (CORR) keep(fco);
-  SlotRow<NE> sgs = sgr;
-  settle(sgs);
+  ThetaIn<NE> t;
+  WIn<NE> v;
+  theta_rows<NE, CORR, MIX>(I, e, c, k, t);
+  w_rows<NE>(I, e, c, k, v);
+  keep(t.fth, v.fwv, v.tru, v.zb, v.zb3);
+  if (CORR) keep(t.fco);
+  settle(sgr);
   float sg[NE];
-  slot_vals(sgs, sg);
-  const float th_m1 = up1(th_k), th_m2 = up1(up1(th_k)), th_p1 = dn1(th_k);
-  const float ths_m1 = up1(ths_k), rwc_m1 = up1(rwc_k);
-  const float ww_m1 = up1(ww_k), ww_m2 = up1(up1(ww_k)), ww_p1 = dn1(ww_k);
-  const float zz_m1 = up1(zz_k);
-  float vf = 0.0f;
-  if (k == 1) {
-    vf = rwc_k * (fzm * th_k + fzp * th_m1);
-    vf = vf + (rws_k - rwc_k) * (fzm * ths_k + fzp * ths_m1);
-  } else if (k >= 2 && k < L - 1) {
-    vf = flux3(th_m2, th_m1, th_k, th_p1, rwc_k, coef);
-    vf = vf + (rws_k - rwc_k) * (fzm * ths_k + fzp * ths_m1);
-  } else if (k == L - 1) {
-    vf = rws_k * (fzm * th_k + fzp * th_m1);
-  }
-  const float vf_p = dn1(vf);
-  float wf = 0.0f;
-  if (k == 1 || k == L - 1) {
-    wf = (0.25f * (rwc_k + rwc_m1)) * (ww_k + ww_m1);
-  } else if (k >= 2 && k < L - 1) {
-    wf = flux3(ww_m2, ww_m1, ww_k, ww_p1, 0.5f * (rwc_k + rwc_m1), 1.0f);
-  }
-  const float wf_p = dn1(wf);
-  float r = 0.0f;
-#pragma unroll
-  for (int s = 0; s < NE; ++s)
-    if (s < n) r = r - sg[s] * fth[s];
-  if (CORR) {
-#pragma unroll
-    for (int s = 0; s < NE; ++s)
-      if (s < n) r = r - sg[s] * fco[s];
-  }
-  r = r * ia;
-  const float trt = r - rdzw * (vf_p - vf);
-  float tru_m[NE];
-#pragma unroll
-  for (int s = 0; s < NE; ++s) tru_m[s] = up1(tru[s]);
-  float rw_t = 0.0f;
-  if (k >= 1 && k < L) {
-    float q = 0.0f;
-#pragma unroll
-    for (int s = 0; s < NE; ++s)
-      if (s < n) q = q - sg[s] * fwv[s];
-    q = q * ia;
-    q = q - rdzu * (wf_p - wf);
-    q = q + erw_k;
-#pragma unroll
-    for (int s = 0; s < NE; ++s)
-      if (s < n) {
-        const float tk = tru[s];
-        const float flux = sg[s] * (fzm * tk + fzp * tru_m[s]);
-        q = q - (zb[s] + cs1(tk) * zb3[s]) * flux;
-      }
-    rw_t = q * (fzm * zz_k + fzp * zz_m1);
-  }
-  if (k < L) {
-    const float tmix = MIX ? trt + eth_k : trt;
-    AT(I.b.tend_rt, c, k) = I.k.physics ? tmix + prt_k : tmix;
-  }
-  if (k <= L) AT(I.b.tend_rw, c, k) = rw_t;
+  slot_vals(sgr, sg);
+  const float rt = theta_tendency<NE, CORR, MIX>(I, t, sg, ia, n, k, fzm, fzp, rdzw);
+  store_tend(I, c, k, rt, w_tendency<NE>(I, v, t.rwc, sg, ia, n, k, fzm, fzp, rdzu));
 }
 
 // ----------------------------------------------------------- acoustic substep
@@ -1443,14 +1577,187 @@ KB k_ac_edge(const Instance I, float dts, float damp_coef) {
   AT(I.b.ru_avg, e, k) = ra_old + p;
 }
 
-// FIRST: the first substep of a stage (the perturbation fields start at
-// zero).  Every global load is issued before the column sweep.
+// The acoustic column update (acoustic_v841.py:296-565) in three parts around
+// the Thomas sweeps: the right-hand side, the Rayleigh damping and new
+// perturbations, and (LAST) the recovery of the column.
+// Level rows of a column block in LDS, in this order.
+enum { LV_RDZW, LV_EWM, LV_EWP, LV_ETP, LV_ETM, LV_FZM, LV_FZP, LV_RDZU, LV_N };
+// each wavefront of the block stages LV_PER of them
+constexpr int LV_PER = LV_N / COLW_AC;
+static_assert(LV_N % COLW_AC == 0, "level rows per wavefront");
+__device__ __forceinline__ void level_rows(const Instance &I, int w, int k, float (&lv)[LV_PER]) {
+  const float *const lev[LV_N] = {I.z.rdzw, I.z.ewm, I.z.ewp, I.z.etp, I.z.etm, I.z.fzm, I.z.fzp, I.z.rdzu};
+#pragma unroll
+  for (int j = 0; j < LV_PER; ++j) lv[j] = lev[w * LV_PER + j][k];
+}
+__device__ __forceinline__ void stage_level_rows(float *s_lev, int w, int k, const float (&lv)[LV_PER]) {
+#pragma unroll
+  for (int j = 0; j < LV_PER; ++j) s_lev[(w * LV_PER + j) * 64 + k] = lv[j];
+}
+template <int NE>
+struct AcIn {
+  float rpp, rtpp, rwp, wwa;            // zero at a stage's first substep
+  float coftz, cofwt, cofwz, trho, trt, trw, zk, al, ga, srw, crw, damp, crho, wk, sthc;
+  float rup[NE], sto[NE];               // ru_p of the cell's edges; start theta of the cells across them
+};
+struct AcMid {  // what the second part needs beside the column itself
+  float rs, ts, wwa;
+};
+// returns the right-hand side and the sub-diagonal (times dts^2) of the column
 template <int NE, bool FIRST>
-KBCOL(COLW_AC) k_ac_cell(const Instance I, float dts, int store_old) {
+__device__ __forceinline__ AcMid ac_rhs(const Instance &I, const AcIn<NE> &q, const float (&sg)[NE],
+                                        const float (&sd)[NE], float ia, int n, int k, float dts, const float *lev,
+                                        float &col, float &ad) {
+  const int L = I.n.L;
+  const float rdzw = lev[LV_RDZW * 64 + k], ewm = lev[LV_EWM * 64 + k], ewp = lev[LV_EWP * 64 + k];
+  const float etp = lev[LV_ETP * 64 + k], etm = lev[LV_ETM * 64 + k], fzm = lev[LV_FZM * 64 + k];
+  const float fzp = lev[LV_FZP * 64 + k];
+  float r = 0.0f, t = 0.0f;
+#pragma unroll
+  for (int s = 0; s < NE; ++s)
+    if (s < n) {
+      // the first substep's ru_p is dts * tend_ru (the momentum pass's product)
+      const float rp = FIRST ? dts * q.rup[s] : q.rup[s];
+      const float flux = ((dts * sd[s]) * rp) * ia;  // (csign*dts)*dv, csign = +-1
+      // theta at the edge: (theta[cell1] + theta[cell0]) in that order
+      const bool first_cell = sg[s] > 0.0f;
+      const float th0 = first_cell ? q.sthc : q.sto[s];
+      const float th1 = first_cell ? q.sto[s] : q.sthc;
+      r = r - flux;
+      t = t - (flux * 0.5f) * (th1 + th0);
+    }
+  const float coftz_p = dn1(q.coftz);
+  const float ewm_p = dn1(ewm);
+  const float rwp_p = dn1(q.rwp);
+  AcMid m;
+  m.rs = ((q.rpp + dts * q.trho) + r) - (dts * rdzw) * (ewm_p * rwp_p - ewm * q.rwp);
+  m.ts = ((q.rtpp + dts * q.trt) + t) - (dts * rdzw) * ((ewm_p * coftz_p) * rwp_p - (ewm * q.coftz) * q.rwp);
+  m.wwa = q.wwa;
+  if (k >= 1 && k < L) m.wwa = m.wwa + ewm * q.rwp;
+  const float ts_m = up1(m.ts), rs_m = up1(m.rs), rtpp_m = up1(q.rtpp), rpp_m = up1(q.rpp), zk_m = up1(q.zk);
+  const float cofwt_m = up1(q.cofwt);
+  const float etp_m = up1(etp), etm_m = up1(etm);
+  // cofwr and the sub-diagonal a of the implicit w system at levels 1..L-1,
+  // formed from zz, the level rows and the coefficients of levels k and k-1
+  // by the same operations as in coef_system
+  const float rdzw_m = up1(rdzw), ewp_m = up1(ewp), coftz_m = up1(q.coftz);
+  float cofwr = 0.0f, a = 0.0f;
+  if (k >= 1 && k < L) {
+    cofwr = (0.5f * I.k.gravity) * (fzm * q.zk + fzp * zk_m);
+    a = (((-q.cofwz) * coftz_m) * rdzw_m) * zk_m + cofwr * rdzw_m - (cofwt_m * coftz_m) * rdzw_m;
+    a = (a * etp_m) * ewp_m;
+  }
+  col = q.rwp;
+  if (k >= 1 && k < L) {
+    float x = q.trw -
+              q.cofwz * (((etp * q.zk) * m.ts - (etp_m * zk_m) * ts_m) + ((etm * q.zk) * q.rtpp - (etm_m * zk_m) * rtpp_m));
+    x = x - cofwr * ((etp * m.rs + etp_m * rs_m) + (etm * q.rpp + etm_m * rpp_m));
+    x = x + q.cofwt * (etp * m.ts + etm * q.rtpp);
+    x = x + cofwt_m * (etp_m * ts_m + etm_m * rtpp_m);
+    col = col + dts * x;
+  }
+  const float dts2 = dts * dts;
+  ad = dts2 * a;
+  return m;
+}
+struct AcOut {
+  float rwp, wwa, rpp, rtpp;
+};
+// the solved column: Rayleigh damping of w, then the new perturbations
+__device__ __forceinline__ AcOut ac_update(const Instance &I, const AcMid &m, float col, float srw, float crw, float damp,
+                                           float crho, float wk, float zk, float coftz, int k, float dts,
+                                           const float *lev) {
+  const int L = I.n.L;
+  const float rdzw = lev[LV_RDZW * 64 + k], ewp = lev[LV_EWP * 64 + k];
+  const float fzm = lev[LV_FZM * 64 + k], fzp = lev[LV_FZP * 64 + k];
+  const float zk_m = up1(zk), crho_m = up1(crho), coftz_p = dn1(coftz), ewp_p = dn1(ewp);
+  if (k >= 1 && k < L) {
+    const float delta = srw - crw;
+    const float zi = fzm * zk + fzp * zk_m;
+    const float ri = fzm * crho + fzp * crho_m;
+    col = (col + delta - (((dts * damp) * zi) * ri) * wk) / (1.0f + dts * damp) - delta;
+  }
+  AcOut o;
+  o.wwa = m.wwa;
+  if (k >= 1 && k < L) o.wwa = o.wwa + ewp * col;
+  const float col_p = dn1(col);
+  o.rwp = col;
+  o.rpp = m.rs - (dts * rdzw) * (ewp_p * col_p - ewp * col);
+  o.rtpp = m.ts - (dts * rdzw) * ((ewp_p * coftz_p) * col_p - (ewp * coftz) * col);
+  return o;
+}
+
+// Recovery of a column after a stage's last substep (driver.py:3176-3290):
+// rho, theta_m, rho*theta, the perturbations and rw; at stage 3 (S3) exner, p'
+// and the split-transport sum of the vertical flux.  The column update holds
+// the perturbations and rw, so recovering here saves storing them for the
+// recovery pass and reading them back there and in the edge recovery (which
+// reads the recovered rho instead of three rows per cell).
+struct RecIn {
+  float srp, rb, srtp, rtb, exb, spw;
+};
+template <bool S3>
+__device__ __forceinline__ RecIn rec_rows(const Instance &I, int c, int k) {
+  return {AT(I.b.s_rho_p, c, k),    AT(I.z.rb, c, k),
+          AT(I.b.s_rtheta_p, c, k), AT(I.z.rtb, c, k),
+          S3 ? AT(I.z.exb, c, k) : 0.0f, S3 ? AT(I.b.split_w, c, k) : 0.0f};
+}
+template <bool S3>
+__device__ __forceinline__ void rec_column(const Instance &I, const RecIn &r, const AcOut &o, float srw, float zk, int c,
+                                           int k, int sub, float inv_steps, int store_rtp) {
+  const int L = I.n.L;
+  const bool lay = k < L, inner = k >= 1 && k < L;
+  const float dp = lay ? r.srp + o.rpp : 0.0f;
+  const float rp = lay ? r.srtp + o.rtpp : 0.0f;
+  const float rho = lay ? dp + r.rb : 1.0f;
+  const float rtv = lay ? rp + r.rtb : 1.0f;
+  int bad = (lay && (!(rho > 0.0f) || !(rtv > 0.0f))) ? 1 : 0;
+  const float th = rtv / rho;
+  float ex = 0.0f, ppv = 0.0f;
+  if (S3 && lay) {
+    const float arg = (zk * I.k.cfac) * rtv;
+    if (!(arg > 0.0f)) bad = 1;
+    ex = exner_pow(I, arg);
+    ppv = (zk * I.k.rgas) * (ex * rp + r.rtb * (ex - r.exb));
+  }
+  if (lay) {
+    AT(I.b.r_rho, c, k) = rho;
+    AT(I.b.r_theta, c, k) = th;
+    if (store_rtp) AT(I.b.r_rtheta_p, c, k) = rp;
+    if (S3) {
+      AT(I.b.r_rho_p, c, k) = dp;
+      AT(I.b.r_rt, c, k) = rtv;
+      AT(I.b.r_exner, c, k) = ex;
+      AT(I.b.r_pp, c, k) = ppv;
+    }
+  }
+  if (k <= L) {
+    AT(I.b.r_rw, c, k) = inner ? srw + o.rwp : 0.0f;
+    if (S3) {
+      const float fw = srw + o.wwa * inv_steps;
+      const float acc = sub == 1 ? fw : fw + r.spw;
+      AT(I.b.split_w, c, k) = sub == I.k.splits ? acc * I.k.split_inv : acc;
+    }
+  }
+  if (bad) set_flag(I.b.flag);
+}
+
+// Scalars of a column pass that recovers its column.
+struct RecArgs {
+  int sub;          // dynamics subcycle
+  float inv_steps;  // 1 / substeps of the stage
+  int store_rtp;    // rtheta_p has a later reader
+  int store_work;   // keep the working perturbations current (the step's last stage)
+};
+
+// FIRST: the first substep of a stage (the perturbation fields start at
+// zero).  LAST: the stage's last substep on the whole-step path, which also
+// recovers the column.  Every global load is issued before the column sweep.
+template <int NE, bool FIRST, bool LAST, bool S3>
+KBCOL(COLW_AC) k_ac_cell(const Instance I, float dts, int store_old, const RecArgs ra) {
   constexpr int COLW = COLW_AC;
-  static_assert(COLW >= 7, "waves 0-6 stage the level rows");
   __shared__ float s_x[COLW * COLP], s_d[COLW * COLP], s_l[COLW * COLP], s_g[COLW * COLP];
-  __shared__ float s_lev[7 * 64];
+  __shared__ float s_lev[LV_N * 64];
   const int w = (int)(threadIdx.x >> 6);
   const int c0 = wave_entity<COLW>();
   const bool live = c0 < I.n.C;
@@ -1466,133 +1773,226 @@ KBCOL(COLW_AC) k_ac_cell(const Instance I, float dts, int store_old) {
   }
   SlotRow<NE> sgr = slot_row<NE>(I.m.csign + c * NE), sdr = slot_row<NE>(I.m.csdv + c * NE);
   const float ia = uni_load(I.m.invarea + c);
-  // wavefront w < 7 stages level row w for the block
-  const float *const lev[7] = {I.z.rdzw, I.z.ewm, I.z.ewp, I.z.etp, I.z.etm, I.z.fzm, I.z.fzp};
-  float lv = 0.0f;
-  if (w < 7) lv = AT(lev[w], 0, k);
-  const float sthc = AT(I.b.s_theta, c, k);
-  float rpp = 0.0f, rtpp = 0.0f, rwp = 0.0f, wwa = 0.0f;
+  float lv[LV_PER];
+  level_rows(I, w, k, lv);
+  AcIn<NE> q;
+  q.sthc = AT(I.b.s_theta, c, k);
+  q.rpp = q.rtpp = q.rwp = q.wwa = 0.0f;
   if (!FIRST) {
-    rpp = AT(I.b.rho_pp, c, k);
-    rtpp = AT(I.b.rtheta_pp, c, k);
-    rwp = AT(I.b.rw_p, c, k);
-    wwa = AT(I.b.ww_avg, c, k);
+    q.rpp = AT(I.b.rho_pp, c, k);
+    q.rtpp = AT(I.b.rtheta_pp, c, k);
+    q.rwp = AT(I.b.rw_p, c, k);
+    q.wwa = AT(I.b.ww_avg, c, k);
   }
-  const float coftz = AT(I.b.coftz, c, k), cofwt = AT(I.b.cofwt, c, k);
-  const float cofwz = AT(I.b.cofwz, c, k);
-  const float trho = AT(I.b.tend_rho, c, k), trt = AT(I.b.tend_rt, c, k), trw = AT(I.b.tend_rw, c, k);
-  const float zk = AT(I.z.zz, c, k);
-  const float al = AT(I.b.alpha, c, k), ga = AT(I.b.gamma, c, k);
-  const float srw = AT(I.b.s_rw, c, k), crw = AT(I.b.c_rw, c, k), damp = AT(I.z.dss, c, k);
-  const float crho = AT(I.b.c_rho, c, k), wk = AT(I.b.w, c, k);
+  q.coftz = AT(I.b.coftz, c, k);
+  q.cofwt = AT(I.b.cofwt, c, k);
+  q.cofwz = AT(I.b.cofwz, c, k);
+  q.trho = AT(I.b.tend_rho, c, k);
+  q.trt = AT(I.b.tend_rt, c, k);
+  q.trw = AT(I.b.tend_rw, c, k);
+  q.zk = AT(I.z.zz, c, k);
+  q.al = AT(I.b.alpha, c, k);
+  q.ga = AT(I.b.gamma, c, k);
+  q.srw = AT(I.b.s_rw, c, k);
+  q.crw = AT(I.b.c_rw, c, k);
+  q.damp = AT(I.z.dss, c, k);
+  q.crho = AT(I.b.c_rho, c, k);
+  q.wk = AT(I.b.w, c, k);
 #pragma unroll
   for (int s = 0; s < NE; ++s) {
     fence(e[s]);
     fence(o[s]);
   }
-  float rup[NE], sto[NE];
 #pragma unroll
   for (int s = 0; s < NE; ++s) {
-    rup[s] = FIRST ? AT(I.b.tend_ru, e[s], k) : AT(I.b.ru_p, e[s], k);
-    sto[s] = AT(I.b.s_theta, o[s], k);
+    q.rup[s] = FIRST ? AT(I.b.tend_ru, e[s], k) : AT(I.b.ru_p, e[s], k);
+    q.sto[s] = AT(I.b.s_theta, o[s], k);
   }
-  keep(rup, sto);
-  if (w < 7) s_lev[w * 64 + k] = lv;
+  keep(q.rup, q.sto);
+  stage_level_rows(s_lev, w, k, lv);
   settle(sgr, sdr);
   float sg[NE], sd[NE];
   slot_vals(sgr, sg);
   slot_vals(sdr, sd);
   __syncthreads();
-  const float rdzw = s_lev[0 * 64 + k], ewm = s_lev[1 * 64 + k], ewp = s_lev[2 * 64 + k];
-  const float etp = s_lev[3 * 64 + k], etm = s_lev[4 * 64 + k], fzm = s_lev[5 * 64 + k], fzp = s_lev[6 * 64 + k];
-  const float rtpp_old = rtpp;
-  float r = 0.0f, t = 0.0f;
-#pragma unroll
-  for (int s = 0; s < NE; ++s)
-    if (s < n) {
-      // the first substep's ru_p is dts * tend_ru (the momentum pass's product)
-      const float rp = FIRST ? dts * rup[s] : rup[s];
-      const float flux = ((dts * sd[s]) * rp) * ia;  // (csign*dts)*dv, csign = +-1
-      // theta at the edge: (theta[cell1] + theta[cell0]) in that order
-      const bool first_cell = sg[s] > 0.0f;
-      const float th0 = first_cell ? sthc : sto[s];
-      const float th1 = first_cell ? sto[s] : sthc;
-      r = r - flux;
-      t = t - (flux * 0.5f) * (th1 + th0);
-    }
-  const float coftz_p = dn1(coftz);
-  const float ewm_p = dn1(ewm), ewp_p = dn1(ewp);
-  const float rwp_p = dn1(rwp);
-  const float rs = ((rpp + dts * trho) + r) - (dts * rdzw) * (ewm_p * rwp_p - ewm * rwp);
-  const float ts = ((rtpp + dts * trt) + t) - (dts * rdzw) * ((ewm_p * coftz_p) * rwp_p - (ewm * coftz) * rwp);
-  if (k >= 1 && k < L) wwa = wwa + ewm * rwp;
-  const float ts_m = up1(ts), rs_m = up1(rs), rtpp_m = up1(rtpp), rpp_m = up1(rpp), zk_m = up1(zk);
-  const float cofwt_m = up1(cofwt);
-  const float etp_m = up1(etp), etm_m = up1(etm);
-  const float crho_m = up1(crho);
-  // cofwr and the sub-diagonal a of the implicit w system at levels 1..L-1,
-  // formed from zz, the level rows and the stored coefficients of levels k
-  // and k-1 by the same operations as in k_vcoef (which stores cofwz, coftz
-  // and cofwt for this kernel, and a only for export)
-  const float rdzw_m = up1(rdzw), ewp_m = up1(ewp), coftz_m = up1(coftz);
-  float cofwr = 0.0f, a = 0.0f;
-  if (k >= 1 && k < L) {
-    cofwr = (0.5f * I.k.gravity) * (fzm * zk + fzp * zk_m);
-    a = (((-cofwz) * coftz_m) * rdzw_m) * zk_m + cofwr * rdzw_m - (cofwt_m * coftz_m) * rdzw_m;
-    a = (a * etp_m) * ewp_m;
-  }
-  float col = rwp;
-  if (k >= 1 && k < L) {
-    float x = trw - cofwz * (((etp * zk) * ts - (etp_m * zk_m) * ts_m) + ((etm * zk) * rtpp - (etm_m * zk_m) * rtpp_m));
-    x = x - cofwr * ((etp * rs + etp_m * rs_m) + (etm * rpp + etm_m * rpp_m));
-    x = x + cofwt * (etp * ts + etm * rtpp);
-    x = x + cofwt_m * (etp_m * ts_m + etm_m * rtpp_m);
-    col = col + dts * x;
-  }
-  const float dts2 = dts * dts;
-  const float ad = dts2 * a;
-  // Thomas sweeps (acoustic_v841.py:296-565), lane = cell: forward for
-  // levels 1..L-1, back substitution for levels L-1..0
+  float col, ad;
+  const AcMid m = ac_rhs<NE, FIRST>(I, q, sg, sd, ia, n, k, dts, s_lev, col, ad);
   s_x[w * COLP + k] = col;
   s_d[w * COLP + k] = ad;
-  s_l[w * COLP + k] = al;
-  s_g[w * COLP + k] = ga;
+  s_l[w * COLP + k] = q.al;
+  s_g[w * COLP + k] = q.ga;
+  RecIn r;
+  if (LAST) r = rec_rows<S3>(I, c, k);  // in flight during the sweeps
   __syncthreads();
-  if (w == 0 && k < COLW) {
-    float *x = s_x + k * COLP;
-    const float *pd = s_d + k * COLP, *pl = s_l + k * COLP, *pg = s_g + k * COLP;
-    float p = x[0];
-    for (int j = 1; j < L; ++j) {
-      p = (x[j] - pd[j] * p) * pl[j];
-      x[j] = p;
-    }
-    p = x[L];
-    for (int j = L - 1; j >= 0; --j) {
-      p = x[j] - pg[j] * p;
-      x[j] = p;
-    }
-  }
+  if (w == 0 && k < COLW)
+    thomas_sweeps(s_x + k * COLP, s_d + k * COLP, s_l + k * COLP, s_g + k * COLP, L);
   __syncthreads();
-  col = s_x[w * COLP + k];
-  if (k >= 1 && k < L) {
-    const float delta = srw - crw;
-    const float zi = fzm * zk + fzp * zk_m;
-    const float ri = fzm * crho + fzp * crho_m;
-    col = (col + delta - (((dts * damp) * zi) * ri) * wk) / (1.0f + dts * damp) - delta;
+  const AcOut a =
+      ac_update(I, m, s_x[w * COLP + k], q.srw, q.crw, q.damp, q.crho, q.wk, q.zk, q.coftz, k, dts, s_lev);
+  if (!live) return;
+  if (!LAST || ra.store_work) {
+    if (k <= L) {
+      AT(I.b.rw_p, c, k) = a.rwp;
+      AT(I.b.ww_avg, c, k) = a.wwa;
+    }
+    if (k < L) AT(I.b.rho_pp, c, k) = a.rpp;
   }
-  if (k >= 1 && k < L) wwa = wwa + ewp * col;
-  const float col_p = dn1(col);
-  const float rpp_new = rs - (dts * rdzw) * (ewp_p * col_p - ewp * col);
-  const float rtpp_new = ts - (dts * rdzw) * ((ewp_p * coftz_p) * col_p - (ewp * coftz) * col);
-  if (live && k <= L) {
-    AT(I.b.rw_p, c, k) = col;
-    AT(I.b.ww_avg, c, k) = wwa;
+  if (k < L) {
+    AT(I.b.rtheta_pp, c, k) = a.rtpp;  // read by the damping that follows
+    if (store_old) AT(I.b.rtheta_pp_old, c, k) = q.rtpp;
   }
-  if (live && k < L) {
-    AT(I.b.rho_pp, c, k) = rpp_new;
-    AT(I.b.rtheta_pp, c, k) = rtpp_new;
-    if (store_old) AT(I.b.rtheta_pp_old, c, k) = rtpp_old;
+  if (LAST) rec_column<S3>(I, r, a, q.srw, q.zk, c, k, ra.sub, ra.inv_steps, ra.store_rtp);
+}
+
+// A stage's column work in one pass on the whole-step path: (VC) the implicit
+// coefficients, the theta and w tendencies, the first acoustic column update
+// and (LAST, a stage of one substep) the recovery.  As passes of their own
+// each of these reads the column's rows again (theta, zz, rw, w, tend_ru of
+// the cell's edges) and hands its result over through memory (five
+// coefficient rows, two tendencies, the perturbations).  x1.40962 moist, the
+// stages of a subcycle with their recovery: 136 + 166 + 111 us against 168 +
+// 182 + 115 us in passes of their own (HBM-bound, 4.0-4.5 TB/s); x1.162, where
+// each launch costs about 5 us: a whole step 662 -> 432 us with the side
+// stream of the coefficients gone.
+// A CU holds four blocks of eight columns (blocks of four: the same times).
+// The registers of eight wavefronts per SIMD do not hold every part's rows at
+// once: the coefficients wait in LDS until the acoustic part, and its rows are
+// loaded when the theta part has freed its own (spills cost their traffic:
+// 130 MB a launch when the parts were left to overlap).  Seven-edge cells take
+// six wavefronts per SIMD.
+template <int NE, bool VC, bool CORR, bool MIX, bool LAST, bool S3>
+__global__ void __launch_bounds__(64 * COLW_AC) __attribute__((amdgpu_waves_per_eu(NE == 6 ? 8 : 6, NE == 6 ? 8 : 6)))
+k_col(const Instance I, float dts, const float *__restrict__ rtp, int store_old, int store_cof, int store_t,
+      const RecArgs ra) {
+  constexpr int COLW = COLW_AC;
+  __shared__ float s_x[COLW * COLP], s_d[COLW * COLP], s_l[COLW * COLP], s_g[COLW * COLP];
+  __shared__ float s_cof[VC ? 3 * COLW * 64 : 1];  // coftz, cofwt, cofwz
+  __shared__ float s_lev[LV_N * 64];
+  const int w = (int)(threadIdx.x >> 6);
+  const int c0 = wave_entity<COLW>();
+  const bool live = c0 < I.n.C;
+  const int c = live ? c0 : 0;  // every wave reaches the barriers
+  const int k = lane();
+  const int L = I.n.L;
+  const int n = I.m.neoc[c];
+  const bool inner = k >= 1 && k < L;
+  int e[NE], o[NE];
+#pragma unroll
+  for (int s = 0; s < NE; ++s) {
+    e[s] = I.m.eoc[c * NE + s];
+    o[s] = I.m.ocell[c * NE + s];  // the other cell of edge s
   }
+  SlotRow<NE> sgr = slot_row<NE>(I.m.csign + c * NE), sdr = slot_row<NE>(I.m.csdv + c * NE);
+  const float ia = uni_load(I.m.invarea + c);
+  float lv[LV_PER];
+  level_rows(I, w, k, lv);
+  if (VC) {
+    const CoefIn r = coef_rows(I, I.b.s_exner, I.b.theta, rtp, c, k);
+    stage_level_rows(s_lev, w, k, lv);
+    __syncthreads();
+    const CoefOut cf = coef_system(I, r, k, s_lev[LV_FZM * 64 + k], s_lev[LV_FZP * 64 + k], s_lev[LV_RDZU * 64 + k],
+                                   s_lev[LV_RDZW * 64 + k], s_lev[LV_ETP * 64 + k], s_lev[LV_EWP * 64 + k]);
+    s_l[w * COLP + k] = cf.a;
+    s_g[w * COLP + k] = cf.b;
+    s_x[w * COLP + k] = cf.cc;
+    s_cof[(0 * COLW + w) * 64 + k] = cf.coftz;
+    s_cof[(1 * COLW + w) * 64 + k] = cf.cofwt;
+    s_cof[(2 * COLW + w) * 64 + k] = cf.cofwz;
+    hold_loads();
+  } else {
+    stage_level_rows(s_lev, w, k, lv);
+  }
+#pragma unroll
+  for (int s = 0; s < NE; ++s) {
+    fence(e[s]);
+    fence(o[s]);
+  }
+  ThetaIn<NE> t;
+  WIn<NE> v;
+  AcIn<NE> q;
+  theta_rows<NE, CORR, MIX>(I, e, c, k, t);
+  if (!VC) w_rows<NE>(I, e, c, k, v);
+  __syncthreads();
+  if (VC) {
+    if (w == 0 && k < COLW) {
+      const int singular = coef_sweep(s_l + k * COLP, s_g + k * COLP, s_x + k * COLP, L, dts * dts);
+      if (singular && block_entity0(COLW) + k < I.n.C) set_flag(I.b.flag);
+    }
+    __syncthreads();
+    w_rows<NE>(I, e, c, k, v);
+    if (!inner) s_l[w * COLP + k] = s_g[w * COLP + k] = 0.0f;  // alpha and gamma of the other levels
+    if (live && store_cof)
+      store_coefs(I, c, k, s_cof[(0 * COLW + w) * 64 + k], s_cof[(1 * COLW + w) * 64 + k],
+                  s_cof[(2 * COLW + w) * 64 + k], 0.0f, s_l[w * COLP + k], s_g[w * COLP + k]);
+  }
+  keep(t.fth);
+  if (CORR) keep(t.fco);
+  settle(sgr, sdr);
+  float sg[NE], sd[NE];
+  slot_vals(sgr, sg);
+  slot_vals(sdr, sd);
+  q.trt = theta_tendency<NE, CORR, MIX>(I, t, sg, ia, n, k, s_lev[LV_FZM * 64 + k], s_lev[LV_FZP * 64 + k],
+                                        s_lev[LV_RDZW * 64 + k]);
+  keep(q.trt);
+  hold_loads();
+  q.trho = AT(I.b.tend_rho, c, k);
+  q.damp = AT(I.z.dss, c, k);
+  q.crho = AT(I.b.c_rho, c, k);
+#pragma unroll
+  for (int s = 0; s < NE; ++s) q.sto[s] = AT(I.b.s_theta, o[s], k);
+  keep(v.fwv, v.tru, v.zb, v.zb3);
+  q.trw = w_tendency<NE>(I, v, t.rwc, sg, ia, n, k, s_lev[LV_FZM * 64 + k], s_lev[LV_FZP * 64 + k],
+                         s_lev[LV_RDZU * 64 + k]);
+  keep(q.trw);
+  hold_loads();
+  if (VC) {
+    q.coftz = s_cof[(0 * COLW + w) * 64 + k];
+    q.cofwt = s_cof[(1 * COLW + w) * 64 + k];
+    q.cofwz = s_cof[(2 * COLW + w) * 64 + k];
+  } else {
+    q.coftz = AT(I.b.coftz, c, k);
+    q.cofwt = AT(I.b.cofwt, c, k);
+    q.cofwz = AT(I.b.cofwz, c, k);
+    s_l[w * COLP + k] = AT(I.b.alpha, c, k);
+    s_g[w * COLP + k] = AT(I.b.gamma, c, k);
+  }
+  if (live && store_t) store_tend(I, c, k, q.trt, q.trw);
+  q.sthc = t.ths;
+  q.rpp = q.rtpp = q.rwp = q.wwa = 0.0f;
+  if (k >= L) q.trt = 0.0f;  // levels past the top read zero, as the stored rows hold
+  q.zk = v.zz;
+  q.srw = t.rws;
+  q.crw = t.rwc;
+  q.wk = v.ww;
+#pragma unroll
+  for (int s = 0; s < NE; ++s) q.rup[s] = v.tru[s];
+  keep(q.sto);
+  float col, ad;
+  const AcMid m = ac_rhs<NE, true>(I, q, sg, sd, ia, n, k, dts, s_lev, col, ad);
+  s_x[w * COLP + k] = col;
+  s_d[w * COLP + k] = ad;
+  hold_loads();
+  RecIn r;
+  if (LAST) r = rec_rows<S3>(I, c, k);  // in flight during the sweeps
+  __syncthreads();
+  if (w == 0 && k < COLW)
+    thomas_sweeps(s_x + k * COLP, s_d + k * COLP, s_l + k * COLP, s_g + k * COLP, L);
+  __syncthreads();
+  const AcOut a =
+      ac_update(I, m, s_x[w * COLP + k], q.srw, q.crw, q.damp, q.crho, q.wk, q.zk, q.coftz, k, dts, s_lev);
+  if (!live) return;
+  if (!LAST || ra.store_work) {
+    if (k <= L) {
+      AT(I.b.rw_p, c, k) = a.rwp;
+      AT(I.b.ww_avg, c, k) = a.wwa;
+    }
+    if (k < L) AT(I.b.rho_pp, c, k) = a.rpp;
+  }
+  if (k < L) {
+    AT(I.b.rtheta_pp, c, k) = a.rtpp;
+    if (store_old) AT(I.b.rtheta_pp_old, c, k) = 0.0f;
+  }
+  if (LAST) rec_column<S3>(I, r, a, q.srw, q.zk, c, k, ra.sub, ra.inv_steps, ra.store_rtp);
 }
 
 KB k_divdamp(const Instance I, float coefficient) {
@@ -1673,11 +2073,30 @@ __device__ __forceinline__ float recover_w_column(const Instance &I, int c, int 
   return col;
 }
 
+// The part of a recovery that reads the cell's recovered edges, after a column
+// pass that recovered the column: terrain w and (HDIV) the next stage's
+// mass-flux divergence.  After stage 3 the next subcycle's opening pass forms
+// the divergence again.
+template <int NE, bool HDIV>
+KB k_rec_w(const Instance I) {
+  const int c = wave_entity(I);
+  if (c >= I.n.C) return;
+  const int k = lane();
+  const float rho = AT(I.b.c_rho, c, k), rwv = AT(I.b.c_rw, c, k);
+  const float *cru = I.b.c_ru;
+  float hd = 0.0f;
+  const float wv =
+      recover_w_column<NE>(I, c, k, rho, rwv, [&](int e) { return AT(cru, e, k); }, HDIV ? &hd : nullptr);
+  if (HDIV && k < I.n.L) AT(I.b.hdiv, c, k) = hd;
+  if (k <= I.n.L) AT(I.b.w, c, k) = wv;
+}
+
+// The whole cell recovery as a pass of its own (the phase entry points).
 // S3: the stage-3 recovery (exner, p' and the split-transport sums).  The
 // loads and the terrain w recovery come first, branch-free, so every gather
 // of the pass is in flight together; stores come last.
 template <int NE, bool S3>
-KB k_rec_cell(const Instance I, int sub, float inv_steps, int store_rtp) {
+KB k_rec_cell(const Instance I, int sub, float inv_steps) {
   const int c = wave_entity(I);
   if (c >= I.n.C) return;
   const int k = lane();
@@ -1721,13 +2140,9 @@ KB k_rec_cell(const Instance I, int sub, float inv_steps, int store_rtp) {
     split = sub == I.k.splits ? acc * I.k.split_inv : acc;
   }
   if (lay) {
-    // rho_p and rtheta_m are read only as the next subcycle's start values
-    // (stage 3) or by an export between phases
-    if (S3 || I.k.store_flux) {
-      AT(I.b.rho_p, c, k) = dp;
-      AT(I.b.c_rt, c, k) = rtv;
-    }
-    if (store_rtp) AT(I.b.rtheta_p, c, k) = rp;
+    AT(I.b.rho_p, c, k) = dp;
+    AT(I.b.c_rt, c, k) = rtv;
+    AT(I.b.rtheta_p, c, k) = rp;
     AT(I.b.c_rho, c, k) = rho;
     AT(I.b.theta, c, k) = th;
     if (S3) {
@@ -1738,7 +2153,7 @@ KB k_rec_cell(const Instance I, int sub, float inv_steps, int store_rtp) {
   }
   if (itf) {
     AT(I.b.c_rw, c, k) = rwv;
-    if (I.k.store_flux) AT(I.b.flux_w, c, k) = fw;
+    AT(I.b.flux_w, c, k) = fw;
     if (S3) AT(I.b.split_w, c, k) = split;
     AT(I.b.w, c, k) = wv;
   }
@@ -1747,9 +2162,9 @@ KB k_rec_cell(const Instance I, int sub, float inv_steps, int store_rtp) {
 
 // DAMP: apply the last substep's divergence damping to ru_p first.
 // AVGRP: one substep and ru_avg not stored, so the average is the undamped
-// ru_p of that substep.  S3: accumulate the split-transport sums.  Loads
-// first, stores last.
-template <bool S3, bool DAMP, bool AVGRP>
+// ru_p of that substep.  S3: accumulate the split-transport sums.  RHO: the
+// column pass has recovered rho.  Loads first, stores last.
+template <bool S3, bool DAMP, bool AVGRP, bool RHO>
 KB k_rec_edge(const Instance I, int sub, float inv_steps, float damp_coef, float dts) {
   const int e = wave_entity(I);
   if (e >= I.n.E) return;
@@ -1761,8 +2176,8 @@ KB k_rec_edge(const Instance I, int sub, float inv_steps, float damp_coef, float
   const float rp_ld = AVGRP ? AT(I.b.tend_ru, e, k) : AT(I.b.ru_p, e, k);
   const float avg_ld = AVGRP ? 0.0f : AT(I.b.ru_avg, e, k);
   const float spu = S3 ? AT(I.b.split_u, e, k) : 0.0f;
-  const float r0 = (AT(I.b.s_rho_p, c0, k) + AT(I.b.rho_pp, c0, k)) + AT(I.z.rb, c0, k);
-  const float r1 = (AT(I.b.s_rho_p, c1, k) + AT(I.b.rho_pp, c1, k)) + AT(I.z.rb, c1, k);
+  const float r0 = RHO ? AT(I.b.c_rho, c0, k) : (AT(I.b.s_rho_p, c0, k) + AT(I.b.rho_pp, c0, k)) + AT(I.z.rb, c0, k);
+  const float r1 = RHO ? AT(I.b.c_rho, c1, k) : (AT(I.b.s_rho_p, c1, k) + AT(I.b.rho_pp, c1, k)) + AT(I.z.rb, c1, k);
   const float rp_raw = AVGRP ? dts * rp_ld : rp_ld;
   const float avg = AVGRP ? rp_raw : avg_ld;
   const float rp = DAMP ? damped_ru_p<AVGRP>(I, e, k, rp_raw, damp_coef) : rp_raw;
@@ -2397,25 +2812,11 @@ int begin_step(const Instance &I, hipStream_t s) {
   return solve_diagnostics(I, 3, s);
 }
 
-// The side stream (or s itself): ordered after everything s has queued.
-inline hipStream_t fork_side(const Side *side, hipStream_t s, int &rc) {
-  if (!side) return s;
-  if (hipEventRecord(side->fork, s) != hipSuccess || hipStreamWaitEvent(side->s, side->fork, 0) != hipSuccess) rc = -1;
-  return side->s;
-}
-// s waits for what the side stream has queued
-inline void join_side(const Side *side, hipStream_t s, int &rc) {
-  if (!side) return;
-  if (hipEventRecord(side->join, side->s) != hipSuccess || hipStreamWaitEvent(s, side->join, 0) != hipSuccess) rc = -1;
-}
-
-int begin_subcycle(const Instance &I, int sub, hipStream_t s, const Side *side) {
+int begin_subcycle(const Instance &I, int sub, hipStream_t s) {
   (void)sub;
-  // the implicit coefficients read only the subcycle-start state, the
-  // moisture and reference rows: beside the pools and the mixing
-  int rc = 0;
-  launch_col_named<COLW_VC>("k_vcoef", k_vcoef, I.n.C, fork_side(side, s, rc), I, I.k.dts[0],
-                            (const float *)I.b.s_exner, (const float *)I.b.s_theta, (const float *)I.b.s_rtheta_p);
+  if (!I.k.fused)  // the whole step forms the implicit coefficients in the stages' column passes
+    launch_col_named<COLW_VC>("k_vcoef", k_vcoef, I.n.C, s, I, I.k.dts[0], (const float *)I.b.s_exner,
+                              (const float *)I.b.s_theta, (const float *)I.b.s_rtheta_p);
   // with mixing, kdiff rides on the cell pass and the del2 u increment on the
   // edge pass (the pool is written once)
   if (I.k.mixing) {
@@ -2449,31 +2850,58 @@ int begin_subcycle(const Instance &I, int sub, hipStream_t s, const Side *side) 
                  launch_named("k_mix_cell", k_mix_cell<7, false>, I.n.C, 1, s, I));
     if (I.k.mix4) LAUNCH_NE(I, k_mix_cell4, I.n.C, 1, s, I);
   }
-  join_side(side, s, rc);
-  return rc ? rc : check();
+  return check();
 }
 
-int dyn_tend(const Instance &I, int stage, hipStream_t s, const Side *side) {
-  // stage 2's implicit coefficients beside the stage's tendencies (which
-  // neither read nor write them); joined before the acoustic substeps
-  int rc = 0;
-  const bool vc = stage == 2 && I.k.order == 3;
-  if (vc)
-    launch_col_named<COLW_VC>("k_vcoef", k_vcoef, I.n.C, fork_side(side, s, rc), I, I.k.dts[1],
-                              (const float *)I.b.s_exner, (const float *)I.b.theta, (const float *)I.b.rtheta_p);
+// the column pass of a stage on the whole-step path
+template <int NE>
+void stage_columns(const Instance &I, int stage, int sub, hipStream_t s) {
+  const int n = I.k.steps[stage - 1];
+  const float dts = I.k.dts[stage - 1];
+  const bool order3 = I.k.order == 3, vc = stage == 1 || (stage == 2 && order3);
+  const bool corr = stage > 1, mix = I.k.mixing != 0, last = n == 1;
+  // a later substep's damping reads rtheta_pp_old; with two substeps the
+  // second takes the zero without a store and a reload
+  const int store_old = n > 2 ? 1 : 0;
+  // stage 1 of the third-order scheme is one substep, and stage 2 forms its own coefficients
+  const int store_cof = !(stage == 1 && order3 && last) ? 1 : 0;
+  const int closing = stage == 3 && sub == I.k.splits ? 1 : 0;  // the working fields the step leaves current
+  const int store_t = !last || closing ? 1 : 0;
+  const RecArgs ra{sub, I.k.inv_steps[stage - 1], stage == 3 || (stage == 1 && order3) ? 1 : 0, closing};
+#define COL(VCV, CO, MX, LA, S3V)                                                                                \
+  launch_col_named<COLW_AC>("k_col", k_col<NE, VCV, CO, MX, LA, S3V>, I.n.C, s, I, dts,                          \
+                            (const float *)I.b.rtheta_p, store_old, store_cof, store_t, ra)
+#define COL_MIX(VCV, CO, LA, S3V) (mix ? COL(VCV, CO, true, LA, S3V) : COL(VCV, CO, false, LA, S3V))
+  if (stage == 3) {
+    last ? COL_MIX(false, true, true, true) : COL_MIX(false, true, false, false);
+  } else if (vc) {
+    corr ? (last ? COL_MIX(true, true, true, false) : COL_MIX(true, true, false, false))
+         : (last ? COL_MIX(true, false, true, false) : COL_MIX(true, false, false, false));
+  } else {
+    last ? COL_MIX(false, true, true, false) : COL_MIX(false, true, false, false);
+  }
+#undef COL_MIX
+#undef COL
+}
+
+int dyn_tend(const Instance &I, int stage, int sub, hipStream_t s) {
   if (I.k.fused) {
     // the edge fluxes came with the preceding diagnostics
     LAUNCH_NE(I, k_tend_mom_ac, I.n.E, 1, s, I, I.k.dts[stage - 1], I.k.steps[stage - 1] > 2 ? 1 : 0,
               I.k.steps[stage - 1] > 1 || stage == 3 ? 1 : 0);
-  } else {
-    LAUNCH_NE(I, k_tend_mom, I.n.E, 1, s, I);
-    if (stage > 1)
-      NEDISPATCH(I, launch_named("k_tend_flux", k_tend_flux<6, true>, I.n.E, 1, s, I),
-                 launch_named("k_tend_flux", k_tend_flux<7, true>, I.n.E, 1, s, I));
-    else
-      NEDISPATCH(I, launch_named("k_tend_flux", k_tend_flux<6, false>, I.n.E, 1, s, I),
-                 launch_named("k_tend_flux", k_tend_flux<7, false>, I.n.E, 1, s, I));
+    NEDISPATCH(I, stage_columns<6>(I, stage, sub, s), stage_columns<7>(I, stage, sub, s));
+    return check();
   }
+  if (stage == 2 && I.k.order == 3)
+    launch_col_named<COLW_VC>("k_vcoef", k_vcoef, I.n.C, s, I, I.k.dts[1], (const float *)I.b.s_exner,
+                              (const float *)I.b.theta, (const float *)I.b.rtheta_p);
+  LAUNCH_NE(I, k_tend_mom, I.n.E, 1, s, I);
+  if (stage > 1)
+    NEDISPATCH(I, launch_named("k_tend_flux", k_tend_flux<6, true>, I.n.E, 1, s, I),
+               launch_named("k_tend_flux", k_tend_flux<7, true>, I.n.E, 1, s, I));
+  else
+    NEDISPATCH(I, launch_named("k_tend_flux", k_tend_flux<6, false>, I.n.E, 1, s, I),
+               launch_named("k_tend_flux", k_tend_flux<7, false>, I.n.E, 1, s, I));
   {
     const bool corr = stage > 1, mix = I.k.mixing != 0;
 #define TEND_CELL(NE, CO, MX) launch_named("k_tend_cell", k_tend_cell<NE, CO, MX>, I.n.C, 1, s, I)
@@ -2484,38 +2912,45 @@ int dyn_tend(const Instance &I, int stage, hipStream_t s, const Side *side) {
 #undef TEND_CELL_NE
 #undef TEND_CELL
   }
-  if (vc) join_side(side, s, rc);
-  return rc ? rc : check();
+  return check();
 }
 
-int acoustic_substep(const Instance &I, int stage, int ss, int damp_prev, hipStream_t s) {
+template <int NE>
+void substep_columns(const Instance &I, int stage, int ss, int sub, hipStream_t s) {
+  const float dts = I.k.dts[stage - 1];
+  const bool last = I.k.fused && ss == I.k.steps[stage - 1];
+  const RecArgs ra{sub, I.k.inv_steps[stage - 1], stage == 3 || (stage == 1 && I.k.order == 3) ? 1 : 0,
+                   stage == 3 && sub == I.k.splits ? 1 : 0};
+#define AC(FI, LA, S3V) launch_col_named<COLW_AC>("k_ac_cell", k_ac_cell<NE, FI, LA, S3V>, I.n.C, s, I, dts, 1, ra)
+  if (ss == 1)
+    AC(true, false, false);
+  else if (!last)
+    AC(false, false, false);
+  else if (stage == 3)
+    AC(false, true, true);
+  else
+    AC(false, true, false);
+#undef AC
+}
+
+int acoustic_substep(const Instance &I, int stage, int ss, int sub, int damp_prev, hipStream_t s) {
   const float dts = I.k.dts[stage - 1];
   const int n = I.k.steps[stage - 1];
-  if (!(I.k.fused && ss == 1))  // fused: the first edge update ran with the momentum tendency
-  {
-    const float coef = I.k.dts_inv_coef[stage - 1];
-    const bool avgrp = I.k.fused && n == 2;
-    if (ss == 1)
-      launch_named("k_ac_edge", k_ac_edge<true, false, false>, I.n.E, 1, s, I, dts, coef);
-    else if (damp_prev && avgrp)
-      launch_named("k_ac_edge", k_ac_edge<false, true, true>, I.n.E, 1, s, I, dts, coef);
-    else if (damp_prev)
-      launch_named("k_ac_edge", k_ac_edge<false, true, false>, I.n.E, 1, s, I, dts, coef);
-    else if (avgrp)
-      launch_named("k_ac_edge", k_ac_edge<false, false, true>, I.n.E, 1, s, I, dts, coef);
-    else
-      launch_named("k_ac_edge", k_ac_edge<false, false, false>, I.n.E, 1, s, I, dts, coef);
-  }
-  // a stage's first substep leaves rtheta_pp_old zero; on the step path the
-  // damping after it takes that zero without a store and a reload (the
-  // second of two substeps' edge update, or a one-substep stage's recovery)
-  const int store_old = I.k.fused && ss == 1 && n <= 2 ? 0 : 1;
+  // fused: the first edge update ran with the momentum tendency, the first column update with the tendencies
+  if (I.k.fused && ss == 1) return check();
+  const float coef = I.k.dts_inv_coef[stage - 1];
+  const bool avgrp = I.k.fused && n == 2;
   if (ss == 1)
-    NEDISPATCH(I, launch_col_named<COLW_AC>("k_ac_cell", k_ac_cell<6, true>, I.n.C, s, I, dts, store_old),
-               launch_col_named<COLW_AC>("k_ac_cell", k_ac_cell<7, true>, I.n.C, s, I, dts, store_old));
+    launch_named("k_ac_edge", k_ac_edge<true, false, false>, I.n.E, 1, s, I, dts, coef);
+  else if (damp_prev && avgrp)
+    launch_named("k_ac_edge", k_ac_edge<false, true, true>, I.n.E, 1, s, I, dts, coef);
+  else if (damp_prev)
+    launch_named("k_ac_edge", k_ac_edge<false, true, false>, I.n.E, 1, s, I, dts, coef);
+  else if (avgrp)
+    launch_named("k_ac_edge", k_ac_edge<false, false, true>, I.n.E, 1, s, I, dts, coef);
   else
-    NEDISPATCH(I, launch_col_named<COLW_AC>("k_ac_cell", k_ac_cell<6, false>, I.n.C, s, I, dts, store_old),
-               launch_col_named<COLW_AC>("k_ac_cell", k_ac_cell<7, false>, I.n.C, s, I, dts, store_old));
+    launch_named("k_ac_edge", k_ac_edge<false, false, false>, I.n.E, 1, s, I, dts, coef);
+  NEDISPATCH(I, substep_columns<6>(I, stage, ss, sub, s), substep_columns<7>(I, stage, ss, sub, s));
   return check();
 }
 
@@ -2527,31 +2962,36 @@ int divergence_damping(const Instance &I, int stage, hipStream_t s) {
 template <bool S3>
 void recover_edges(const Instance &I, int sub, float inv, bool damp, bool avgrp, float coef, float dts,
                    hipStream_t s) {
-  if (damp && avgrp)
-    launch_named("k_rec_edge", k_rec_edge<S3, true, true>, I.n.E, 1, s, I, sub, inv, coef, dts);
-  else if (damp)
-    launch_named("k_rec_edge", k_rec_edge<S3, true, false>, I.n.E, 1, s, I, sub, inv, coef, dts);
-  else if (avgrp)
-    launch_named("k_rec_edge", k_rec_edge<S3, false, true>, I.n.E, 1, s, I, sub, inv, coef, dts);
+#define REC(DA, AV, RH) launch_named("k_rec_edge", k_rec_edge<S3, DA, AV, RH>, I.n.E, 1, s, I, sub, inv, coef, dts)
+  if (I.k.fused)
+    damp ? (avgrp ? REC(true, true, true) : REC(true, false, true))
+         : (avgrp ? REC(false, true, true) : REC(false, false, true));
   else
-    launch_named("k_rec_edge", k_rec_edge<S3, false, false>, I.n.E, 1, s, I, sub, inv, coef, dts);
+    REC(false, false, false);  // the phase entry points damp in a pass of their own and keep ru_avg
+#undef REC
 }
 
 int recover(const Instance &I, int stage, int sub, int damp, hipStream_t s) {
   const float inv = I.k.inv_steps[stage - 1];
   const bool avgrp = I.k.fused && I.k.steps[stage - 1] == 1;
   const float coef = I.k.dts_inv_coef[stage - 1];
-  // rtheta_p is read by the implicit coefficients of stage 2 (from stage 1)
-  // and as the next subcycle's start (from stage 3)
-  const int store_rtp = stage == 3 || (stage == 1 && I.k.order == 3) || I.k.store_flux ? 1 : 0;
-  if (stage == 3) {
+  if (stage == 3)
     recover_edges<true>(I, sub, inv, damp != 0, avgrp, coef, I.k.dts[stage - 1], s);
-    NEDISPATCH(I, launch_named("k_rec_cell", k_rec_cell<6, true>, I.n.C, 1, s, I, sub, inv, store_rtp),
-               launch_named("k_rec_cell", k_rec_cell<7, true>, I.n.C, 1, s, I, sub, inv, store_rtp));
-  } else {
+  else
     recover_edges<false>(I, sub, inv, damp != 0, avgrp, coef, I.k.dts[stage - 1], s);
-    NEDISPATCH(I, launch_named("k_rec_cell", k_rec_cell<6, false>, I.n.C, 1, s, I, sub, inv, store_rtp),
-               launch_named("k_rec_cell", k_rec_cell<7, false>, I.n.C, 1, s, I, sub, inv, store_rtp));
+  if (I.k.fused) {  // the column pass recovered the rest
+    if (stage == 3)
+      NEDISPATCH(I, launch_named("k_rec_w", k_rec_w<6, false>, I.n.C, 1, s, I),
+                 launch_named("k_rec_w", k_rec_w<7, false>, I.n.C, 1, s, I));
+    else
+      NEDISPATCH(I, launch_named("k_rec_w", k_rec_w<6, true>, I.n.C, 1, s, I),
+                 launch_named("k_rec_w", k_rec_w<7, true>, I.n.C, 1, s, I));
+  } else if (stage == 3) {
+    NEDISPATCH(I, launch_named("k_rec_cell", k_rec_cell<6, true>, I.n.C, 1, s, I, sub, inv),
+               launch_named("k_rec_cell", k_rec_cell<7, true>, I.n.C, 1, s, I, sub, inv));
+  } else {
+    NEDISPATCH(I, launch_named("k_rec_cell", k_rec_cell<6, false>, I.n.C, 1, s, I, sub, inv),
+               launch_named("k_rec_cell", k_rec_cell<7, false>, I.n.C, 1, s, I, sub, inv));
   }
   return check();
 }

@@ -90,14 +90,22 @@ _K: Dict[str, List[Tuple[str, str]]] = {
                   ("C", "L"), ("C", "W"), ("C", "W"), ("C", "L"), ("C", "L"),
                   ("C", "L"), ("C", "L"), ("C", "L"), ("C", "L"), ("C", "W"), ("C", "W"), ("C", "L"),
                   ("C", "W"), ("C", "W"), ("C", "W"), ("C", "L"), ("C", "L"), ("C", "L")],
+    # a stage's whole column work with its coefficients and recovery (stage 2):
+    # k_tend_cell's reads | exner, cqw, qtot, rtheta_p, rb, rtb, exb | tend_rho, dss, c_rho | s_rho_p, s_rtheta_p |
+    # cofwz, cofwt, alpha, gamma, coftz | rho, theta, rtheta_pp, rw
+    "k_col": [("C", "L"), ("C", "L"), ("C", "W"), ("C", "W"), ("C", "W"), ("E", "L"), ("E", "L"),
+              ("E", "W"), ("C", "W"), ("E", "L"), ("CM", "W"), ("CM", "W"), ("C", "L")]
+             + [("C", "L")] * 7 + [("C", "L")] * 3 + [("C", "L")] * 2 + [("C", "L")] * 4 + [("C", "W")]
+             + [("C", "L")] * 3 + [("C", "W")],
+    # rho, rw, ru, zz, zb, zb3 | w, hdiv
+    "k_rec_w": [("C", "L"), ("C", "W"), ("E", "L"), ("C", "L"), ("CM", "W"), ("CM", "W"), ("C", "W"), ("C", "L")],
     "k_divdamp": [("C", "L"), ("C", "L"), ("C", "L"), ("E", "L"), ("E", "L")],
     # s_rho_p, rho_pp, s_rtheta_p, rtheta_pp, rb, rtb, s_rw, rw_p, ww_avg, s_ru, ru_p, zz, zb, zb3, exb |
     # rho_p, rtheta_p, c_rho, c_rt, theta, c_rw, flux_w, w, (exner, pp)
     "k_rec_cell": [("C", "L")] * 6 + [("C", "W")] * 3 + [("E", "L")] * 2 + [("C", "L"), ("CM", "W"), ("CM", "W"),
                    ("C", "L")] + [("C", "L")] * 5 + [("C", "W")] * 3 + [("C", "L")] * 2,
-    # the whole-step form after one damped substep: s_ru, ru_p, s_rho_p, rho_pp, rb, rtheta_pp,
-    # rtheta_pp_old, s_theta | ru_p, c_ru, u
-    "k_rec_edge": [("E", "L")] * 2 + [("C", "L")] * 6 + [("E", "L")] * 3,
+    # the whole-step form after one damped substep: s_ru, tend_ru, rho, rtheta_pp, s_theta | c_ru, u
+    "k_rec_edge": [("E", "L")] * 2 + [("C", "L")] * 3 + [("E", "L")] * 2,
     "k_sc_edge": [("SC", "L"), ("E", "L"), ("SE", "L")],
     "k_sc_cell": [("SC", "L"), ("C", "W"), ("E", "L"), ("SE", "L"), ("C", "L"), ("C", "L"), ("SC", "L"),
                   ("SC", "L")],
