@@ -51,198 +51,341 @@ constexpr int KIN = 6 * HX_ROW;    // 384 input features per cell
 constexpr int NOUT = 5 * HX_ROW;   // 320 outputs per cell
 enum { CH_UE = 0, CH_UN = 1, CH_W = 2, CH_TH = 3, CH_RHO = 4, CH_QV = 5 };
 enum { O_UE = 0, O_UN = 1, O_TH = 2, O_RHO = 3, O_W = 4 };
-constexpr int GPART = 128;         // blocks of the weight-gradient reductions
 
 __device__ __forceinline__ f32x4 mfma(const bf16x8 &a, const bf16x8 &b, const f32x4 &c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// ------------------------------------------------------------------ GEMM
-// out[M][N] = epi(A[M][K] . B), A = [A1 (K1 columns) | A2 (K - K1 columns)]
-// row-major bf16, B given transposed (Bt[N][K], bf16).  A block of four
-// wavefronts stages Bt in LDS once and walks 16-row tiles (one tile per
-// wavefront at a time, all N columns: N/16 MFMA accumulators).
-// MFMA operand layout (16x16x32): lane l supplies row (or column) l % 16
-// and the 8 consecutive k values 8 * (l / 16) .. +7; the accumulator lane l
-// holds column l % 16, rows 4 * (l / 16) + i.
-enum { EPI_RELU = 0, EPI_RESID_RELU = 1, EPI_F32 = 2 };
-constexpr int GEMM_WAVES = 8;  // wavefronts per block (2 per SIMD beside the block's LDS copy of B)
-constexpr int GEMM_TR = 2;     // 16-row tiles per wavefront at a time (each B fragment feeds TR MFMAs)
+// Logical block of a launch: XCD x (hardware block b runs on XCD b % 8) takes
+// a contiguous range of the curve, so the rows its gathers share meet in its L2.
+__device__ __forceinline__ int curve_block() {
+  const int nb = (int)gridDim.x, b = (int)blockIdx.x;
+  const int x = b & 7, i = b >> 3, q = nb >> 3, r = nb & 7;
+  return (x < r) ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
+}
 
-template <int K, int N, int K1, int EPI>
-__global__ void __launch_bounds__(64 * GEMM_WAVES) k_gemm(const bf16 *__restrict__ A1, const bf16 *__restrict__ A2,
-                                                          const bf16 *__restrict__ Bt, const float *__restrict__ bias,
-                                                          const bf16 *__restrict__ resid, bf16 *__restrict__ out_b,
-                                                          float *__restrict__ out_f, bf16 *__restrict__ relu_out,
-                                                          int M) {
-  static_assert(K % 32 == 0 && N % 16 == 0 && K1 % 32 == 0 && K1 <= K, "tile shape");
-  constexpr int LDK = K + 8;  // row stride in LDS (16-byte pad against bank conflicts)
-  constexpr int KA1 = K1;
-  constexpr int KA2 = K - K1;
-  constexpr int NT = N / 16;
-  extern __shared__ __align__(16) unsigned char lds_raw[];
-  bf16 *sB = (bf16 *)lds_raw;
-  for (int i = (int)threadIdx.x; i < N * (K / 8); i += 64 * GEMM_WAVES) {
-    const int n = i / (K / 8), kc = i % (K / 8);
-    *(bf16x8 *)(sB + n * LDK + kc * 8) = *(const bf16x8 *)(Bt + (size_t)n * K + kc * 8);
-  }
-  __syncthreads();
-  const int w = (int)(threadIdx.x >> 6), l = (int)(threadIdx.x & 63);
-  const int lr = l & 15, lg = l >> 4;
-  const int ngroups = (M + 16 * GEMM_TR - 1) / (16 * GEMM_TR);
-  for (int gt = (int)blockIdx.x * GEMM_WAVES + w; gt < ngroups; gt += (int)gridDim.x * GEMM_WAVES) {
-    int row[GEMM_TR];
+// s / n for a neighbour count n in 3..7, rn = RN(1/n): the product with one
+// FMA residual correction is the correctly rounded quotient for quotients in
+// [2^-120, FLT_MAX] and for +0, which a relu leaves often (verified
+// exhaustively for every binary32 s and these n); other inputs take the
+// division.
+__device__ __forceinline__ float div_count(float s, float n, float rn) {
+  const float q0 = s * rn;
+  const float a = fabsf(q0);
+  if ((a >= 0x1p-120f && a <= 0x1.fffffep127f) || __float_as_uint(s) == 0u)
+    return __builtin_fmaf(__builtin_fmaf(-q0, n, s), rn, q0);
+  return s / n;
+}
+
+// ------------------------------------------------------------------ GEMM
+// out[M][N] = epi(A[M][K] . B), A row-major bf16, B given transposed
+// (Bt[N][K], bf16).  A wavefront takes 16 rows at a time with every column of
+// the block's NC: all K/32 fragments of A are requested before the block's
+// copy of Bt (its NC rows) is staged in LDS, so one memory latency covers
+// both, and 16 rows per wavefront keep every CU busy down to a few thousand
+// rows (32 rows per wavefront and 8 wavefronts per block left 41 blocks at
+// 10 242 rows: 30 us for a layer and its mean in two passes, 17 us here).
+// The weights are the first MFMA operand and the rows of A the second: the
+// accumulator lane l then holds row l % 16 of the tile and 4 consecutive
+// columns 4 * (l / 16) + i, which store as 8 or 16 bytes (the other way round
+// they are 4 rows of one column, 2 or 4 bytes each).  Operand layout
+// (16x16x32): lane l supplies row l % 16 and the 8 consecutive k values
+// 8 * (l / 16) .. +7.
+// NE > 0: a message-passing layer.  A = [h_c | mean over cellsOnCell of h],
+// the mean formed here from the neighbours' rows (fp32 sums in slot order, one
+// rounding to bf16) instead of in a pass of its own.
+enum { EPI_RELU = 0, EPI_RESID_RELU = 1, EPI_F32 = 2, EPI_F32_MASK = 3 };
+
+struct GemmArgs {
+  const bf16 *A, *Bt;
+  const float *bias;
+  const bf16 *resid;      // EPI_RESID_RELU: added after the relu
+  const bf16 *mask;       // EPI_F32_MASK: out_b = out_f where mask > 0
+  bf16 *out_b;
+  float *out_f;
+  bf16 *relu_out;         // EPI_RESID_RELU: the relu itself (kept for backward), may be null
+  bf16 *mean_out;         // NE > 0: the neighbour mean (kept for backward), may be null
+  const int *coc, *neoc;  // NE > 0
+  int M;
+};
+
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
+template <int K, int NE>
+__device__ __forceinline__ void gemm_rows(const GemmArgs &g, int tile, int lr, int lg, bf16x8 (&a)[K / 32]) {
+  const int row = min(tile * 16 + lr, g.M - 1);
+  constexpr int KO = NE > 0 ? K / 2 : K;  // the row's own columns
+  const bf16 *own = g.A + (size_t)row * KO + lg * 8;
 #pragma unroll
-    for (int r = 0; r < GEMM_TR; ++r) row[r] = min((gt * GEMM_TR + r) * 16 + lr, M - 1);
-    f32x4 acc[GEMM_TR][NT];
+  for (int q = 0; q < KO / 32; ++q) a[q] = *(const bf16x8 *)(own + q * 32);
+  if constexpr (NE > 0) {
+    constexpr int Q = KO / 32, QH = Q / 2;
+    const int n = g.neoc[row];
+    int nb[NE];
 #pragma unroll
-    for (int r = 0; r < GEMM_TR; ++r)
+    for (int s = 0; s < NE; ++s) nb[s] = g.coc[row * NE + s];  // padded slots hold cell 0
+    const float fn = (float)n, rn = 1.0f / fn;
 #pragma unroll
-      for (int j = 0; j < NT; ++j) acc[r][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-    for (int k0 = 0; k0 < K; k0 += 32) {
-      const int kk = k0 + lg * 8;
-      bf16x8 a[GEMM_TR];
+    for (int h = 0; h < 2; ++h) {  // half the channels at a time: every neighbour's row of them in flight together
+      bf16x8 v[NE][QH];
 #pragma unroll
-      for (int r = 0; r < GEMM_TR; ++r) {
-        if (KA2 == 0 || k0 < KA1)
-          a[r] = *(const bf16x8 *)(A1 + (size_t)row[r] * KA1 + kk);
-        else
-          a[r] = *(const bf16x8 *)(A2 + (size_t)row[r] * (KA2 > 0 ? KA2 : 1) + (kk - KA1));
-      }
+      for (int s = 0; s < NE; ++s)
 #pragma unroll
-      for (int j = 0; j < NT; ++j) {
-        const bf16x8 b = *(const bf16x8 *)(sB + (j * 16 + lr) * LDK + kk);
+        for (int q = 0; q < QH; ++q)
+          v[s][q] = *(const bf16x8 *)(g.A + (size_t)nb[s] * KO + (h * QH + q) * 32 + lg * 8);
 #pragma unroll
-        for (int r = 0; r < GEMM_TR; ++r) acc[r][j] = mfma(a[r], b, acc[r][j]);
+      for (int q = 0; q < QH; ++q) {
+        bf16x8 m;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          float acc = 0.f;
+#pragma unroll
+          for (int s = 0; s < NE; ++s) acc = s < n ? acc + (float)v[s][q][j] : acc;
+          m[j] = (bf16)div_count(acc, fn, rn);
+        }
+        a[Q + h * QH + q] = m;
+        if (g.mean_out && tile * 16 + lr < g.M)
+          *(bf16x8 *)(g.mean_out + (size_t)row * KO + (h * QH + q) * 32 + lg * 8) = m;
       }
     }
+  }
+}
+
+template <int K, int N, int NC, int EPI, int NE>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) k_gemm(const GemmArgs g) {
+  static_assert(K % 32 == 0 && NC % 16 == 0 && N % NC == 0, "tile shape");
+  static_assert(NE == 0 || NC == N, "one block forms a row's neighbour mean");
+  constexpr int LDK = K + 8;  // row stride in LDS (16-byte pad against bank conflicts)
+  constexpr int NT = NC / 16;
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  bf16 *sB = (bf16 *)lds_raw;
+  const int W = (int)(blockDim.x >> 6);
+  const int w = (int)(threadIdx.x >> 6), l = (int)(threadIdx.x & 63);
+  const int lr = l & 15, lg = l >> 4;
+  const int n0 = (int)blockIdx.y * NC;
+  const int tiles = (g.M + 15) / 16;
+  int t = curve_block() * W + w;
+  bf16x8 a[K / 32];
+  if (t < tiles) gemm_rows<K, NE>(g, t, lr, lg, a);
+  for (int i = (int)threadIdx.x; i < NC * (K / 8); i += 64 * W) {
+    const int n = i / (K / 8), kc = i % (K / 8);
+    *(bf16x8 *)(sB + n * LDK + kc * 8) = *(const bf16x8 *)(g.Bt + (size_t)(n0 + n) * K + kc * 8);
+  }
+  __syncthreads();
+  while (t < tiles) {
+    asm volatile("" ::: "memory");  // the fragments of B are read from LDS per tile, not kept across tiles
+    f32x4 acc[NT];
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const int col = j * 16 + lr;
-      const float bj = bias ? bias[col] : 0.0f;
+    for (int j = 0; j < NT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int r = 0; r < GEMM_TR; ++r) {
+    for (int q = 0; q < K / 32; ++q)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int rr = (gt * GEMM_TR + r) * 16 + lg * 4 + i;
-          if (rr >= M) continue;
-          const float v = acc[r][j][i] + bj;
-          const size_t o = (size_t)rr * N + col;
-          if (EPI == EPI_RELU) {
-            out_b[o] = (bf16)fmaxf(v, 0.0f);
-          } else if (EPI == EPI_RESID_RELU) {
-            const float rl = fmaxf(v, 0.0f);
-            if (relu_out) relu_out[o] = (bf16)rl;
-            out_b[o] = (bf16)((float)resid[o] + rl);
-          } else {
-            out_f[o] = v;
+      for (int j = 0; j < NT; ++j) {
+        const bf16x8 b = *(const bf16x8 *)(sB + (j * 16 + lr) * LDK + q * 32 + lg * 8);
+        acc[j] = mfma(b, a[q], acc[j]);
+      }
+    const int row = t * 16 + lr;
+    if (row < g.M) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const int col = n0 + j * 16 + lg * 4;
+        const size_t o = (size_t)row * N + col;
+        f32x4 v = acc[j];
+        if (g.bias) v += *(const f32x4 *)(g.bias + col);
+        if (EPI == EPI_RELU) {
+          bf16x4 r;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) r[i] = (bf16)fmaxf(v[i], 0.0f);
+          *(bf16x4 *)(g.out_b + o) = r;
+        } else if (EPI == EPI_RESID_RELU) {
+          const bf16x4 h = *(const bf16x4 *)(g.resid + o);
+          bf16x4 r, y;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float rl = fmaxf(v[i], 0.0f);
+            r[i] = (bf16)rl;
+            y[i] = (bf16)((float)h[i] + rl);
+          }
+          if (g.relu_out) *(bf16x4 *)(g.relu_out + o) = r;
+          *(bf16x4 *)(g.out_b + o) = y;
+        } else {
+          *(f32x4 *)(g.out_f + o) = v;
+          if (EPI == EPI_F32_MASK) {
+            const bf16x4 m = *(const bf16x4 *)(g.mask + o);
+            bf16x4 d;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) d[i] = (bf16)((float)m[i] > 0.0f ? v[i] : 0.0f);
+            *(bf16x4 *)(g.out_b + o) = d;
           }
         }
       }
     }
+    t += (int)gridDim.x * W;
+    if (t < tiles) gemm_rows<K, NE>(g, t, lr, lg, a);
   }
 }
 
-// partial[blockIdx][KA][NB] = sum over this block's row chunks of A^T B,
-// A = [A1 (K1 cols) | A2] [M][KA], B [M][NB] (bf16).  Chunks of 64 rows are
-// staged transposed in LDS (At[k][m], Bt[n][m]) so each MFMA operand is one
-// 16-byte LDS read; eight wavefronts split the (KA/16) x (NB/16) tiles.
-template <int KA, int K1, int NB>
-__global__ void __launch_bounds__(512) k_gemm_tn(const bf16 *__restrict__ A1, const bf16 *__restrict__ A2,
-                                                 const bf16 *__restrict__ Bm, float *__restrict__ partial, int M) {
-  constexpr int MC = 64, LDM = MC + 8;
-  constexpr int TILES = (KA / 16) * (NB / 16);
-  static_assert(TILES % 8 == 0, "tiles split over 8 wavefronts");
-  constexpr int TPW = TILES / 8;
-  constexpr int KA2 = KA - K1;
-  extern __shared__ __align__(16) unsigned char lds_raw[];
-  bf16 *sA = (bf16 *)lds_raw;      // [KA][LDM]
-  bf16 *sBt = sA + KA * LDM;       // [NB][LDM]
-  const int w = (int)(threadIdx.x >> 6), l = (int)(threadIdx.x & 63);
-  const int lr = l & 15, lg = l >> 4;
-  f32x4 acc[TPW];
+// ------------------------------------------------------- weight gradients
+// Every matrix gradient A^T B (sums over the M rows) and bias gradient (column
+// sums of B) of a backward pass in one launch: block (tile, split) forms one
+// 64 x 64 tile of one matrix over its split's rows and writes a partial in the
+// layout of the flat parameter vector; k_grad_reduce sums the splits in order
+// (repeatable bits).  The matrices are small (54 tiles at four layers), so
+// splitting the rows fills the chip: 28 us at 10 242 rows and four layers
+// (one launch per matrix over 128 blocks took 23-33 us each, its own reduction
+// and column sums 80 us more).
+struct GradJob {
+  const bf16 *A1, *A2;  // [M][K1], [M][K - K1] (null when K1 == K)
+  const bf16 *B;        // [M][N]
+  int K1, K, N;
+  int tile0;            // first tile of the job
+  long long off, boff;  // offsets of the matrix and its bias in the parameter vector
+};
+constexpr int GRAD_JOBS = 10;
+struct GradArgs {
+  GradJob job[GRAD_JOBS];
+  int jobs, M, rows;    // rows of a split, a multiple of GRAD_CH
+  long long n_params;
+};
+constexpr int GRAD_T = 64;    // tile edge
+constexpr int GRAD_CH = 128;  // rows staged at a time
+
+// 8x8 bf16 transpose: r[i] row i -> o[j] column j
+__device__ __forceinline__ void transpose8(const uint4 (&r)[8], uint4 (&o)[8]) {
+  const uint32_t *x = (const uint32_t *)r;
+  uint32_t *y = (uint32_t *)o;
 #pragma unroll
-  for (int q = 0; q < TPW; ++q) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int nchunks = (M + MC - 1) / MC;
-  for (int ch = (int)blockIdx.x; ch < nchunks; ch += (int)gridDim.x) {
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t lo = x[(2 * i) * 4 + j], hi = x[(2 * i + 1) * 4 + j];
+      y[(2 * j) * 4 + i] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+      y[(2 * j + 1) * 4 + i] = __builtin_amdgcn_perm(hi, lo, 0x07060302u);
+    }
+}
+
+__global__ void __launch_bounds__(256) k_grad(const GradArgs g, float *__restrict__ partial) {
+  constexpr int LDM = GRAD_CH + 8;
+  __shared__ __align__(16) bf16 s_t[2 * GRAD_T * LDM];  // A^T then B^T, [column][row]
+  __shared__ float s_sum[GRAD_CH / 8][GRAD_T];
+  int jn = 0;
+#pragma unroll
+  for (int i = 1; i < GRAD_JOBS; ++i)
+    if (i < g.jobs && (int)blockIdx.x >= g.job[i].tile0) jn = i;
+  const GradJob jb = g.job[jn];
+  const int nt = jb.N / GRAD_T, tl = (int)blockIdx.x - jb.tile0;
+  const int ti = tl / nt, tj = tl % nt;
+  const int th = (int)threadIdx.x;
+  // this thread's 8x8 block of the chunk: rows mb*8.., columns kb*8.. of A (threads 0..127) or B
+  const bool isb = th >= 128;
+  const int mb = th & 15, kb = (th >> 4) & 7;
+  const bf16 *src;
+  int ld;
+  if (isb) {
+    src = jb.B + tj * GRAD_T;
+    ld = jb.N;
+  } else if (ti * GRAD_T < jb.K1) {
+    src = jb.A1 + ti * GRAD_T;
+    ld = jb.K1;
+  } else {
+    src = jb.A2 + (ti * GRAD_T - jb.K1);
+    ld = jb.K - jb.K1;
+  }
+  src += kb * 8;
+  bf16 *dst = s_t + (isb ? GRAD_T * LDM : 0) + (kb * 8) * LDM + mb * 8;
+  const int w = th >> 6, l = th & 63, lr = l & 15, lg = l >> 4;
+  const int kt = (w >> 1) * 32, ct = (w & 1) * 32;  // this wavefront's 32 x 32 of the tile
+  f32x4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  const int m_lo = (int)blockIdx.y * g.rows, m_hi = min(g.M, m_lo + g.rows);
+  uint4 r[8], o[8];
+  auto load = [&](int m0) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int m = m0 + mb * 8 + i;
+      r[i] = m < m_hi ? *(const uint4 *)(src + (size_t)m * ld) : uint4{0u, 0u, 0u, 0u};
+    }
+  };
+  load(m_lo);
+  for (int m0 = m_lo; m0 < m_hi; m0 += GRAD_CH) {
+    transpose8(r, o);
+    if (ti == 0 && isb) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const bf16x8 col = __builtin_bit_cast(bf16x8, o[j]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sum[j] += (float)col[i];
+      }
+    }
+    __syncthreads();  // the chunk before this one has been read
+#pragma unroll
+    for (int j = 0; j < 8; ++j) *(uint4 *)(dst + j * LDM) = o[j];
     __syncthreads();
-    for (int i = (int)threadIdx.x; i < MC * (KA / 8); i += 512) {
-      const int m = i / (KA / 8), kc = (i % (KA / 8)) * 8;
-      const int gm = ch * MC + m;
-      bf16x8 v;
-      if (gm < M) {
-        if (KA2 == 0 || kc < K1)
-          v = *(const bf16x8 *)(A1 + (size_t)gm * K1 + kc);
-        else
-          v = *(const bf16x8 *)(A2 + (size_t)gm * (KA2 > 0 ? KA2 : 1) + (kc - K1));
-      } else {
-        for (int j = 0; j < 8; ++j) v[j] = (bf16)0.0f;
+    if (m0 + GRAD_CH < m_hi) load(m0 + GRAD_CH);  // in flight under the products
+#pragma unroll
+    for (int q = 0; q < GRAD_CH / 32; ++q) {
+      bf16x8 av[2], bv[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        av[i] = *(const bf16x8 *)(s_t + (kt + i * 16 + lr) * LDM + q * 32 + lg * 8);
+        bv[i] = *(const bf16x8 *)(s_t + (GRAD_T + ct + i * 16 + lr) * LDM + q * 32 + lg * 8);
       }
 #pragma unroll
-      for (int j = 0; j < 8; ++j) sA[(kc + j) * LDM + m] = v[j];
-    }
-    for (int i = (int)threadIdx.x; i < MC * (NB / 8); i += 512) {
-      const int m = i / (NB / 8), nc = (i % (NB / 8)) * 8;
-      const int gm = ch * MC + m;
-      bf16x8 v;
-      if (gm < M) {
-        v = *(const bf16x8 *)(Bm + (size_t)gm * NB + nc);
-      } else {
-        for (int j = 0; j < 8; ++j) v[j] = (bf16)0.0f;
-      }
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) sBt[(nc + j) * LDM + m] = v[j];
+        for (int j = 0; j < 2; ++j) acc[i][j] = mfma(av[i], bv[j], acc[i][j]);
     }
+  }
+  float *out = partial + (size_t)blockIdx.y * g.n_params;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        out[jb.off + (size_t)(ti * GRAD_T + kt + i * 16 + lg * 4 + e) * jb.N + tj * GRAD_T + ct + j * 16 + lr] =
+            acc[i][j][e];
+  if (ti == 0) {
+    if (isb)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s_sum[mb][kb * 8 + j] = sum[j];
     __syncthreads();
+    if (th < GRAD_T) {
+      float s = 0.f;
 #pragma unroll
-    for (int q = 0; q < TPW; ++q) {
-      const int tile = w * TPW + q;
-      const int ti = tile / (NB / 16), tj = tile % (NB / 16);
-#pragma unroll
-      for (int m0 = 0; m0 < MC; m0 += 32) {
-        const bf16x8 a = *(const bf16x8 *)(sA + (ti * 16 + lr) * LDM + m0 + lg * 8);
-        const bf16x8 b = *(const bf16x8 *)(sBt + (tj * 16 + lr) * LDM + m0 + lg * 8);
-        acc[q] = mfma(a, b, acc[q]);
-      }
+      for (int i = 0; i < GRAD_CH / 8; ++i) s += s_sum[i][th];
+      out[jb.boff + tj * GRAD_T + th] = s;
     }
   }
-  float *out = partial + (size_t)blockIdx.x * KA * NB;
-#pragma unroll
-  for (int q = 0; q < TPW; ++q) {
-    const int tile = w * TPW + q;
-    const int ti = tile / (NB / 16), tj = tile % (NB / 16);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) out[(size_t)(ti * 16 + lg * 4 + i) * NB + tj * 16 + lr] = acc[q][i];
-  }
 }
 
-// partial[blockIdx][NB] = column sums of B over this block's row chunks
-template <int NB>
-__global__ void __launch_bounds__(512) k_colsum(const bf16 *__restrict__ Bm, float *__restrict__ partial, int M) {
-  constexpr int MC = 64;
-  const int n = (int)threadIdx.x;
-  if (n >= NB) return;
-  float s = 0.0f;
-  const int nchunks = (M + MC - 1) / MC;
-  for (int ch = (int)blockIdx.x; ch < nchunks; ch += (int)gridDim.x)
-    for (int m = ch * MC; m < min(M, ch * MC + MC); ++m) s += (float)Bm[(size_t)m * NB + n];
-  partial[(size_t)blockIdx.x * NB + n] = s;
-}
-
-// out[i] = sum_b partial[b][i], b ascending
-__global__ void __launch_bounds__(256) k_reduce(const float *__restrict__ partial, int nb, int n,
-                                                float *__restrict__ out) {
+// grads[i] = sum over splits of partial[split][i], ascending
+__global__ void __launch_bounds__(256) k_grad_reduce(const float *__restrict__ partial, int splits, int n,
+                                                     float *__restrict__ out) {
   const int i = (int)(blockIdx.x * 256 + threadIdx.x);
   if (i >= n) return;
   float s = 0.0f;
-  for (int b = 0; b < nb; ++b) s += partial[(size_t)b * n + i];
+  int b = 0;
+  for (; b + 8 <= splits; b += 8) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = partial[(size_t)(b + u) * n + i];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += v[u];
+  }
+  for (; b < splits; ++b) s += partial[(size_t)b * n + i];
   out[i] = s;
 }
 
 // ---------------------------------------------------------- mesh kernels
-// Lane k of wavefront (blockIdx*4 + w) owns row k of one cell or edge.
-__device__ __forceinline__ int ent4() { return (int)(blockIdx.x * 4 + (threadIdx.x >> 6)); }
+// Lane k of wavefront (block*4 + w) owns row k of one cell or edge.
+__device__ __forceinline__ int ent4() {
+  return __builtin_amdgcn_readfirstlane(curve_block() * 4 + (int)(threadIdx.x >> 6));
+}
 __device__ __forceinline__ int lane() { return (int)(threadIdx.x & 63); }
 // element k of row e of a dycore array (rows rs floats apart; lanes k >= rs
 // read the row's last element, as the dycore kernels do)
@@ -339,38 +482,14 @@ __global__ void __launch_bounds__(256) k_features(const Instance I, const float 
   }
 }
 
-// a_c = mean over cellsOnCell of h (128 channels: lane and lane + 64)
-template <int NE>
-__global__ void __launch_bounds__(256) k_aggregate(const Instance I, const bf16 *__restrict__ Hin,
-                                                   bf16 *__restrict__ Aout) {
-  const int c = ent4();
-  if (c >= I.n.C) return;
-  const int k = lane();
-  const int n = I.m.neoc[c];
-  // every neighbour row first (the slot table is padded), then the sums in slot order
-  float h0[NE], h1[NE];
-#pragma unroll
-  for (int s = 0; s < NE; ++s) {
-    const int j = I.m.coc[c * NE + s];
-    h0[s] = (float)Hin[(size_t)j * HID + k];
-    h1[s] = (float)Hin[(size_t)j * HID + 64 + k];
-  }
-  float s0 = 0.f, s1 = 0.f;
-#pragma unroll
-  for (int s = 0; s < NE; ++s)
-    if (s < n) {
-      s0 += h0[s];
-      s1 += h1[s];
-    }
-  Aout[(size_t)c * HID + k] = (bf16)(s0 / (float)n);
-  Aout[(size_t)c * HID + 64 + k] = (bf16)(s1 / (float)n);
-}
-
 // dH_l = dH_{l+1} + dZ[:, :128] + sum over cellsOnCell j of dZ_j[128:] / n_j
-// (the mean's adjoint; cellsOnCell is symmetric on a Voronoi mesh)
+// (the mean's adjoint; cellsOnCell is symmetric on a Voronoi mesh), and the
+// next matrix gradient's operand dP = dH_l * [mask > 0] in bf16.  The encoder
+// reads dP only (dH null).
 template <int NE>
 __global__ void __launch_bounds__(256) k_aggregate_back(const Instance I, const float *__restrict__ dHnext,
-                                                        const float *__restrict__ dZ, float *__restrict__ dH) {
+                                                        const float *__restrict__ dZ, const bf16 *__restrict__ mask,
+                                                        float *__restrict__ dH, bf16 *__restrict__ dP) {
   const int c = ent4();
   if (c >= I.n.C) return;
   const int k = lane();
@@ -383,6 +502,10 @@ __global__ void __launch_bounds__(256) k_aggregate_back(const Instance I, const 
     z0[s] = dZ[(size_t)j * 2 * HID + HID + k];
     z1[s] = dZ[(size_t)j * 2 * HID + HID + 64 + k];
   }
+  const size_t o = (size_t)c * HID;
+  const float h0 = dHnext[o + k], h1 = dHnext[o + 64 + k];
+  const float s0 = dZ[(size_t)c * 2 * HID + k], s1 = dZ[(size_t)c * 2 * HID + 64 + k];
+  const float m0 = (float)mask[o + k], m1 = (float)mask[o + 64 + k];
   float a0 = 0.f, a1 = 0.f;
 #pragma unroll
   for (int s = 0; s < NE; ++s)
@@ -391,23 +514,13 @@ __global__ void __launch_bounds__(256) k_aggregate_back(const Instance I, const 
       a0 += z0[s] * inv;
       a1 += z1[s] * inv;
     }
-  const size_t o = (size_t)c * HID;
-  dH[o + k] = (dHnext[o + k] + dZ[(size_t)c * 2 * HID + k]) + a0;
-  dH[o + 64 + k] = (dHnext[o + 64 + k] + dZ[(size_t)c * 2 * HID + 64 + k]) + a1;
-}
-
-// dP = dH * [mask > 0] (bf16 for the next MFMA)
-__global__ void __launch_bounds__(256) k_relu_back(const float *__restrict__ dH, const bf16 *__restrict__ mask,
-                                                   bf16 *__restrict__ dP, size_t n) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  dP[i] = (bf16)((float)mask[i] > 0.0f ? dH[i] : 0.0f);
-}
-
-__global__ void __launch_bounds__(256) k_f32_to_bf16(const float *__restrict__ x, bf16 *__restrict__ y, size_t n) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  y[i] = (bf16)x[i];
+  const float d0 = (h0 + s0) + a0, d1 = (h1 + s1) + a1;
+  if (dH) {
+    dH[o + k] = d0;
+    dH[o + 64 + k] = d1;
+  }
+  dP[o + k] = (bf16)(m0 > 0.0f ? d0 : 0.0f);
+  dP[o + 64 + k] = (bf16)(m1 > 0.0f ? d1 : 0.0f);
 }
 
 // Published fields of the coarse and fine handles that the target reads.
@@ -475,7 +588,7 @@ __global__ void __launch_bounds__(256) k_loss_edges(const Instance I, const floa
   d2 = wave_sum_f(d2);
   if (k == 0) s_part[threadIdx.x >> 6] = d2;
   __syncthreads();
-  if (threadIdx.x == 0) lpart[blockIdx.x] = ((s_part[0] + s_part[1]) + s_part[2]) + s_part[3];
+  if (threadIdx.x == 0) lpart[curve_block()] = ((s_part[0] + s_part[1]) + s_part[2]) + s_part[3];
 }
 
 // dY of every output channel (bf16) and the per-block partial sums of squared
@@ -526,16 +639,28 @@ __global__ void __launch_bounds__(256) k_loss_cells(const Instance I, const floa
   __syncthreads();
   if (threadIdx.x < 3) {
     const int v = (int)threadIdx.x;
-    lpart[(size_t)v * gridDim.x + blockIdx.x] = ((s_part[v][0] + s_part[v][1]) + s_part[v][2]) + s_part[v][3];
+    lpart[(size_t)v * gridDim.x + curve_block()] = ((s_part[v][0] + s_part[v][1]) + s_part[v][2]) + s_part[v][3];
   }
 }
 
-// sum of nb floats in ascending order, in binary64 (one thread)
-__global__ void k_sum_ordered(const float *__restrict__ p, int nb, double *__restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// The four loss sums (edges, then theta, rho and w of the cells) in binary64,
+// one block each: a thread's strided partials, then a fixed tree.
+__global__ void __launch_bounds__(1024) k_loss_sums(const float *__restrict__ p, int ne, int nc,
+                                                    double *__restrict__ out) {
+  __shared__ double s_sum[1024];
+  const int v = (int)blockIdx.x, t = (int)threadIdx.x;
+  const int n = v == 0 ? ne : nc;
+  if (v > 0) p += (size_t)ne + (size_t)(v - 1) * nc;
   double s = 0.0;
-  for (int b = 0; b < nb; ++b) s += (double)p[b];
-  out[0] = s;
+#pragma unroll 4
+  for (int b = t; b < n; b += 1024) s += (double)p[b];
+  s_sum[t] = s;
+  __syncthreads();
+  for (int off = 512; off >= 1; off >>= 1) {
+    if (t < off) s_sum[t] = s_sum[t] + s_sum[t + off];
+    __syncthreads();
+  }
+  if (t == 0) out[v] = s_sum[0];
 }
 
 // ---------------------------------------------------------- application
@@ -563,7 +688,7 @@ __global__ void __launch_bounds__(256) k_mass_partial(const Instance I, const fl
   }
   __syncthreads();
   if (threadIdx.x < 2)
-    part[(size_t)threadIdx.x * gridDim.x + blockIdx.x] =
+    part[(size_t)threadIdx.x * gridDim.x + curve_block()] =
         ((s_part[threadIdx.x][0] + s_part[threadIdx.x][1]) + s_part[threadIdx.x][2]) + s_part[threadIdx.x][3];
 }
 
@@ -703,9 +828,9 @@ __global__ void __launch_bounds__(256) k_checks_cells(const Instance I, float dt
   __syncthreads();
   if (threadIdx.x < 3) {
     const int v = (int)threadIdx.x;
-    fpart[(size_t)v * gridDim.x + blockIdx.x] = nanmax(nanmax(nanmax(s_f[v][0], s_f[v][1]), s_f[v][2]), s_f[v][3]);
+    fpart[(size_t)v * gridDim.x + curve_block()] = nanmax(nanmax(nanmax(s_f[v][0], s_f[v][1]), s_f[v][2]), s_f[v][3]);
   } else if (threadIdx.x == 3) {
-    mpart[blockIdx.x] = ((s_m[0] + s_m[1]) + s_m[2]) + s_m[3];
+    mpart[curve_block()] = ((s_m[0] + s_m[1]) + s_m[2]) + s_m[3];
   }
 }
 
@@ -748,10 +873,32 @@ struct Seg {
   int K, N;        // matrix shape (N = count, K = 1 for a bias)
   long long boff;  // offset in the bf16 weight buffers (matrices only, -1 for biases)
 };
+constexpr int MAX_SEGS = 2 * (8 + 2);
+struct SegTable {
+  Seg seg[MAX_SEGS];
+  int n;
+};
+
+// bf16 copies of parameter i where it belongs to a matrix: W[k][n] (backward)
+// and Wt[n][k] (forward).  A block of 256 parameters lies in one segment, or
+// in few: the table is walked with uniform reads.
+__device__ __forceinline__ void store_weight(const SegTable &t, long long i, float p, bf16 *__restrict__ W,
+                                             bf16 *__restrict__ Wt) {
+  for (int s = 0; s < t.n; ++s) {
+    const Seg sg = t.seg[s];
+    const long long j = i - sg.off;
+    if (sg.boff < 0 || j < 0 || j >= (long long)sg.K * sg.N) continue;
+    const int k = (int)j / sg.N, n = (int)j % sg.N;
+    const bf16 b = (bf16)p;
+    W[sg.boff + j] = b;
+    Wt[sg.boff + (long long)n * sg.K + k] = b;
+  }
+}
 
 __global__ void __launch_bounds__(256) k_adam(float *__restrict__ p, const float *__restrict__ g,
                                               float *__restrict__ m, float *__restrict__ v, size_t n, float lr,
-                                              float b1, float b2, float eps, float bc1, float bc2) {
+                                              float b1, float b2, float eps, float bc1, float bc2, const SegTable t,
+                                              bf16 *__restrict__ W, bf16 *__restrict__ Wt) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   const float gi = g[i];
@@ -760,18 +907,16 @@ __global__ void __launch_bounds__(256) k_adam(float *__restrict__ p, const float
   m[i] = mi;
   v[i] = vi;
   const float mh = mi / bc1, vh = vi / bc2;
-  p[i] = p[i] - lr * (mh / (sqrtf(vh) + eps));
+  const float pn = p[i] - lr * (mh / (sqrtf(vh) + eps));
+  p[i] = pn;
+  store_weight(t, (long long)i, pn, W, Wt);
 }
 
-// bf16 copies of one weight matrix: W[k][n] (backward) and Wt[n][k] (forward)
-__global__ void __launch_bounds__(256) k_to_bf16_pair(const float *__restrict__ p, int K, int N,
-                                                      bf16 *__restrict__ W, bf16 *__restrict__ Wt) {
-  const int i = (int)(blockIdx.x * 256 + threadIdx.x);
-  if (i >= K * N) return;
-  const int k = i / N, n = i % N;
-  const bf16 b = (bf16)p[i];
-  W[i] = b;
-  Wt[(size_t)n * K + k] = b;
+// bf16 copies of every weight matrix
+__global__ void __launch_bounds__(256) k_weights(const float *__restrict__ p, size_t n, const SegTable t,
+                                                 bf16 *__restrict__ W, bf16 *__restrict__ Wt) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) store_weight(t, (long long)i, p[i], W, Wt);
 }
 
 // logical (original) order export of per-cell rows of width w
@@ -799,7 +944,9 @@ inline unsigned nblk(size_t n, int per = 256) { return (unsigned)((n + per - 1) 
 // ====================================================================== Net
 struct Net {
   int C = 0, E = 0, NL = 0, NE = 6;
-  int dev_blocks = 256;  // persistent GEMM grid
+  int cus = 256;
+  SegTable table{};
+  int splits = 1, split_rows = 128;  // of the weight gradients
   std::vector<void *> allocs;
   std::vector<Seg> segs;  // W_in, b_in, (W_l, b_l) x NL, W_out, b_out
   size_t n_params = 0, n_bf = 0;
@@ -810,8 +957,9 @@ struct Net {
   std::vector<bf16 *> H, A, R;  // H: NL+1, A and R: NL
   float *Y = nullptr;
   float *Tc = nullptr, *Te = nullptr, *g = nullptr;
-  bf16 *dY = nullptr, *dP = nullptr;
-  float *dH0 = nullptr, *dH1 = nullptr, *dZ = nullptr, *dH4 = nullptr;
+  bf16 *dY = nullptr;
+  std::vector<bf16 *> dP;       // masked gradients: encoder, then the layers
+  float *dH0 = nullptr, *dH1 = nullptr, *dZ = nullptr;
   float *partial = nullptr, *lpart = nullptr;
   double *loss_out = nullptr, *mpart = nullptr;
   float *shift = nullptr, *checks = nullptr, *raw = nullptr, *cpart = nullptr;
@@ -853,44 +1001,20 @@ int set_lds(KFn fn, size_t bytes) {
              : -1;
 }
 
-template <int K, int N, int K1, int EPI>
-int gemm(const Net &n, const bf16 *A1, const bf16 *A2, const bf16 *Bt, const float *bias, const bf16 *resid,
-         bf16 *out_b, float *out_f, bf16 *relu_out, int M, hipStream_t s) {
-  const size_t lds = (size_t)N * (K + 8) * sizeof(bf16);
-  static int ready = 0;
-  if (!ready) {
-    if (set_lds(k_gemm<K, N, K1, EPI>, lds)) return -1;
-    ready = 1;
-  }
-  const int groups = (M + 16 * GEMM_TR - 1) / (16 * GEMM_TR);
-  const int grid = std::max(1, std::min(n.dev_blocks, (groups + GEMM_WAVES - 1) / GEMM_WAVES));
-  prof_mark("k_net_gemm", s, 1);
-  hipLaunchKernelGGL((k_gemm<K, N, K1, EPI>), dim3(grid), dim3(64 * GEMM_WAVES), lds, s, A1, A2, Bt, bias, resid,
-                     out_b, out_f, relu_out, M);
-  prof_mark("k_net_gemm", s, 0);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
-}
-
-template <int KA, int K1, int NB>
-int gemm_tn(const Net &n, const bf16 *A1, const bf16 *A2, const bf16 *Bm, float *dW, int M, hipStream_t s) {
-  const size_t lds = (size_t)(KA + NB) * (64 + 8) * sizeof(bf16);
-  static int ready = 0;
-  if (!ready) {
-    if (set_lds(k_gemm_tn<KA, K1, NB>, lds)) return -1;
-    ready = 1;
-  }
-  prof_mark("k_net_gemm_tn", s, 1);
-  hipLaunchKernelGGL((k_gemm_tn<KA, K1, NB>), dim3(GPART), dim3(512), lds, s, A1, A2, Bm, n.partial, M);
-  prof_mark("k_net_gemm_tn", s, 0);
-  hipLaunchKernelGGL(k_reduce, dim3(nblk((size_t)KA * NB)), dim3(256), 0, s, (const float *)n.partial, GPART, KA * NB,
-                     dW);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
-}
-
-template <int NB>
-int colsum(const Net &n, const bf16 *Bm, float *db, int M, hipStream_t s) {
-  hipLaunchKernelGGL(k_colsum<NB>, dim3(GPART), dim3(512), 0, s, Bm, n.partial, M);
-  hipLaunchKernelGGL(k_reduce, dim3(nblk(NB)), dim3(256), 0, s, (const float *)n.partial, GPART, NB, db);
+// Wavefronts per block: 4, so that a few thousand rows still reach every CU;
+// 8 (two blocks of them per CU share its LDS) once every CU has a block of 8.
+template <int K, int N, int NC, int EPI, int NE>
+int gemm(const Net &n, const GemmArgs &g, hipStream_t s) {
+  const size_t lds = (size_t)NC * (K + 8) * sizeof(bf16);
+  static const int ready = set_lds(k_gemm<K, N, NC, EPI, NE>, lds);
+  if (ready) return -1;
+  const int tiles = (g.M + 15) / 16;
+  const int W = tiles >= 8 * n.cus ? 8 : 4;
+  const int per_cu = std::max(1, (int)((size_t)160 * 1024 / lds));
+  const int grid = std::max(1, std::min((tiles + W - 1) / W, n.cus * std::min(per_cu, 4)));
+  if (g_prof_on) prof_mark("k_net_gemm", s, 1);
+  hipLaunchKernelGGL((k_gemm<K, N, NC, EPI, NE>), dim3(grid, N / NC), dim3(64 * W), lds, s, g);
+  if (g_prof_on) prof_mark("k_net_gemm", s, 0);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -905,29 +1029,42 @@ int colsum(const Net &n, const bf16 *Bm, float *db, int M, hipStream_t s) {
 }  // namespace
 
 int features(Net &n, const Instance &I, hipStream_t s, float *raw = nullptr) {
-  prof_mark("k_net_features", s, 1);
+  if (g_prof_on) prof_mark("k_net_features", s, 1);
   NE_LAUNCH(n.NE, k_features, nblk(n.C, 4), 256, s, I, (const float *)n.in_mean, (const float *)n.in_scale, n.X,
             raw);
-  prof_mark("k_net_features", s, 0);
+  if (g_prof_on) prof_mark("k_net_features", s, 0);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int forward(Net &n, const Instance &I, bool keep, hipStream_t s) {
   if (features(n, I, s)) return -1;
-  if (gemm<KIN, HID, KIN, EPI_RELU>(n, n.X, nullptr, n.Wt(n.w_in()), n.P(n.b_in()), nullptr, n.H[0], nullptr,
-                                    nullptr, n.C, s))
-    return -1;
+  GemmArgs g{};
+  g.M = n.C;
+  g.coc = I.m.coc;
+  g.neoc = I.m.neoc;
+  g.A = n.X;
+  g.Bt = n.Wt(n.w_in());
+  g.bias = n.P(n.b_in());
+  g.out_b = n.H[0];
+  if (gemm<KIN, HID, HID, EPI_RELU, 0>(n, g, s)) return -1;
   for (int l = 0; l < n.NL; ++l) {
-    prof_mark("k_net_aggregate", s, 1);
-    NE_LAUNCH(n.NE, k_aggregate, nblk(n.C, 4), 256, s, I, (const bf16 *)n.H[l], n.A[l]);
-    prof_mark("k_net_aggregate", s, 0);
-    if (gemm<2 * HID, HID, HID, EPI_RESID_RELU>(n, n.H[l], n.A[l], n.Wt(n.w_l(l)), n.P(n.b_l(l)), n.H[l],
-                                                n.H[l + 1], nullptr, keep ? n.R[l] : nullptr, n.C, s))
+    g.A = g.resid = n.H[l];
+    g.Bt = n.Wt(n.w_l(l));
+    g.bias = n.P(n.b_l(l));
+    g.out_b = n.H[l + 1];
+    g.relu_out = keep ? n.R[l] : nullptr;
+    g.mean_out = keep ? n.A[l] : nullptr;
+    if (n.NE == 6 ? gemm<2 * HID, HID, HID, EPI_RESID_RELU, 6>(n, g, s)
+                  : gemm<2 * HID, HID, HID, EPI_RESID_RELU, 7>(n, g, s))
       return -1;
   }
-  if (gemm<HID, NOUT, HID, EPI_F32>(n, n.H[n.NL], nullptr, n.Wt(n.w_out()), n.P(n.b_out()), nullptr, nullptr, n.Y,
-                                    nullptr, n.C, s))
-    return -1;
+  g = GemmArgs{};
+  g.M = n.C;
+  g.A = n.H[n.NL];
+  g.Bt = n.Wt(n.w_out());
+  g.bias = n.P(n.b_out());
+  g.out_f = n.Y;
+  if (gemm<HID, NOUT, NOUT / 4, EPI_F32, 0>(n, g, s)) return -1;
   n.have_forward = 1;
   return 0;
 }
@@ -937,13 +1074,9 @@ int loss(Net &n, const Instance &I, double *out4, hipStream_t s) {
   const unsigned ge = nblk(n.E, 4), gc = nblk(n.C, 4);
   hipLaunchKernelGGL(k_loss_edges, dim3(ge), dim3(256), 0, s, I, (const float *)n.Y, (const float *)n.Te, n.g,
                      n.lpart, 1.0f / (float)((double)n.E * L));
-  hipLaunchKernelGGL(k_sum_ordered, dim3(1), dim3(64), 0, s, (const float *)n.lpart, (int)ge, n.loss_out);
-  float *lp = n.lpart + ge;
-  NE_LAUNCH(n.NE, k_loss_cells, gc, 256, s, I, (const float *)n.Y, (const float *)n.Tc, (const float *)n.g, n.dY, lp,
-            1.0f / (float)((double)n.C * L), 1.0f / (float)((double)n.C * (L - 1)));
-  for (int v = 0; v < 3; ++v)
-    hipLaunchKernelGGL(k_sum_ordered, dim3(1), dim3(64), 0, s, (const float *)(lp + (size_t)v * gc), (int)gc,
-                       n.loss_out + 1 + v);
+  NE_LAUNCH(n.NE, k_loss_cells, gc, 256, s, I, (const float *)n.Y, (const float *)n.Tc, (const float *)n.g, n.dY,
+            n.lpart + ge, 1.0f / (float)((double)n.C * L), 1.0f / (float)((double)n.C * (L - 1)));
+  hipLaunchKernelGGL(k_loss_sums, dim3(4), dim3(1024), 0, s, (const float *)n.lpart, (int)ge, (int)gc, n.loss_out);
   if (hipGetLastError() != hipSuccess) return -1;
   double raw[4];
   if (hipMemcpyAsync(raw, n.loss_out, sizeof raw, hipMemcpyDeviceToHost, s) != hipSuccess ||
@@ -957,50 +1090,61 @@ int loss(Net &n, const Instance &I, double *out4, hipStream_t s) {
   return 0;
 }
 
+// The gradient chain first (each pass leaves the masked bf16 gradient that its
+// matrix needs), then every matrix and bias gradient in one launch.
 int backward(Net &n, const Instance &I, hipStream_t s) {
-  const int C = n.C;
-  const size_t ch = (size_t)C * HID;
-  // decoder
-  if (gemm_tn<HID, HID, NOUT>(n, n.H[n.NL], nullptr, n.dY, n.G(n.w_out()), C, s)) return -1;
-  if (colsum<NOUT>(n, n.dY, n.G(n.b_out()), C, s)) return -1;
-  if (gemm<NOUT, HID, NOUT, EPI_F32>(n, n.dY, nullptr, n.W(n.w_out()), nullptr, nullptr, nullptr, n.dH1, nullptr, C,
-                                     s))
-    return -1;
+  const int C = n.C, NL = n.NL;
+  GemmArgs g{};
+  g.M = C;
+  g.A = n.dY;
+  g.Bt = n.W(n.w_out());
+  g.out_f = n.dH1;
+  g.mask = n.R[NL - 1];
+  g.out_b = n.dP[NL];
+  if (gemm<NOUT, HID, HID, EPI_F32_MASK, 0>(n, g, s)) return -1;
   float *dHnext = n.dH1, *dHcur = n.dH0;
-  for (int l = n.NL - 1; l >= 0; --l) {
-    hipLaunchKernelGGL(k_relu_back, dim3(nblk(ch)), dim3(256), 0, s, (const float *)dHnext, (const bf16 *)n.R[l], n.dP,
-                       ch);
-    if (gemm_tn<2 * HID, HID, HID>(n, n.H[l], n.A[l], n.dP, n.G(n.w_l(l)), C, s)) return -1;
-    if (colsum<HID>(n, n.dP, n.G(n.b_l(l)), C, s)) return -1;
-    if (gemm<HID, 2 * HID, HID, EPI_F32>(n, n.dP, nullptr, n.W(n.w_l(l)), nullptr, nullptr, nullptr, n.dZ, nullptr,
-                                         C, s))
-      return -1;
-    NE_LAUNCH(n.NE, k_aggregate_back, nblk(C, 4), 256, s, I, (const float *)dHnext, (const float *)n.dZ, dHcur);
+  for (int l = NL - 1; l >= 0; --l) {
+    g = GemmArgs{};
+    g.M = C;
+    g.A = n.dP[l + 1];
+    g.Bt = n.W(n.w_l(l));
+    g.out_f = n.dZ;
+    if (gemm<HID, 2 * HID, HID, EPI_F32, 0>(n, g, s)) return -1;
+    NE_LAUNCH(n.NE, k_aggregate_back, nblk(C, 4), 256, s, I, (const float *)dHnext, (const float *)n.dZ,
+              (const bf16 *)(l > 0 ? n.R[l - 1] : n.H[0]), l > 0 ? dHcur : nullptr, n.dP[l]);
     std::swap(dHnext, dHcur);
   }
-  // encoder (dHnext holds dL/dh0)
-  hipLaunchKernelGGL(k_relu_back, dim3(nblk(ch)), dim3(256), 0, s, (const float *)dHnext, (const bf16 *)n.H[0], n.dP,
-                     ch);
-  if (gemm_tn<KIN, KIN, HID>(n, n.X, nullptr, n.dP, n.G(n.w_in()), C, s)) return -1;
-  if (colsum<HID>(n, n.dP, n.G(n.b_in()), C, s)) return -1;
+  GradArgs a{};
+  a.M = C;
+  a.rows = n.split_rows;
+  a.n_params = (long long)n.n_params;
+  int tiles = 0;
+  auto job = [&](const bf16 *A1, int K1, const bf16 *A2, const Seg &w, const Seg &b, const bf16 *B) {
+    a.job[a.jobs++] = GradJob{A1, A2, B, K1, w.K, w.N, tiles, w.off, b.off};
+    tiles += (w.K / GRAD_T) * (w.N / GRAD_T);
+  };
+  job(n.X, KIN, nullptr, n.w_in(), n.b_in(), n.dP[0]);
+  for (int l = 0; l < NL; ++l) job(n.H[l], HID, n.A[l], n.w_l(l), n.b_l(l), n.dP[l + 1]);
+  job(n.H[NL], HID, nullptr, n.w_out(), n.b_out(), n.dY);
+  if (g_prof_on) prof_mark("k_net_grad", s, 1);
+  hipLaunchKernelGGL(k_grad, dim3(tiles, n.splits), dim3(256), 0, s, a, n.partial);
+  if (g_prof_on) prof_mark("k_net_grad", s, 0);
+  hipLaunchKernelGGL(k_grad_reduce, dim3(nblk(n.n_params)), dim3(256), 0, s, (const float *)n.partial, n.splits,
+                     (int)n.n_params, n.grads);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int sync_bf16(Net &n, hipStream_t s) {
-  for (const Seg &sg : n.segs) {
-    if (sg.boff < 0) continue;
-    hipLaunchKernelGGL(k_to_bf16_pair, dim3(nblk((size_t)sg.K * sg.N)), dim3(256), 0, s,
-                       (const float *)(n.params + sg.off), sg.K, sg.N, n.w_bf + sg.boff, n.wt_bf + sg.boff);
-  }
+  hipLaunchKernelGGL(k_weights, dim3(nblk(n.n_params)), dim3(256), 0, s, (const float *)n.params, n.n_params, n.table,
+                     n.w_bf, n.wt_bf);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int adam(Net &n, float lr, float b1, float b2, float eps, int t, hipStream_t s) {
   const float bc1 = (float)(1.0 - std::pow((double)b1, t)), bc2 = (float)(1.0 - std::pow((double)b2, t));
   hipLaunchKernelGGL(k_adam, dim3(nblk(n.n_params)), dim3(256), 0, s, n.params, (const float *)n.grads, n.adam_m,
-                     n.adam_v, n.n_params, lr, b1, b2, eps, bc1, bc2);
-  if (hipGetLastError() != hipSuccess) return -1;
-  return sync_bf16(n, s);
+                     n.adam_v, n.n_params, lr, b1, b2, eps, bc1, bc2, n.table, n.w_bf, n.wt_bf);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int target(Net &n, const Instance &Ic, const Instance &If, hipStream_t s) {
@@ -1014,7 +1158,7 @@ int target(Net &n, const Instance &Ic, const Instance &If, hipStream_t s) {
 
 int apply(Net &n, const Instance &I, float gain, hipStream_t s) {
   const unsigned gc = nblk(n.C, 4);
-  prof_mark("k_net_apply", s, 1);
+  if (g_prof_on) prof_mark("k_net_apply", s, 1);
   hipLaunchKernelGGL(k_mass_partial, dim3(gc), dim3(256), 0, s, I, (const float *)n.Y, (const float *)n.out_scale,
                      n.mpart);
   hipLaunchKernelGGL(k_mass_shift, dim3(1), dim3(256), 0, s, (const double *)n.mpart, (int)gc, n.shift);
@@ -1022,17 +1166,17 @@ int apply(Net &n, const Instance &I, float gain, hipStream_t s) {
                      (const float *)n.shift, gain);
   hipLaunchKernelGGL(k_apply_edges, dim3(nblk(n.E, 4)), dim3(256), 0, s, I, (const float *)n.Y,
                      (const float *)n.out_scale, gain);
-  prof_mark("k_net_apply", s, 0);
+  if (g_prof_on) prof_mark("k_net_apply", s, 0);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int checks(Net &n, const Instance &I, float dt, float out[3], double *mass, hipStream_t s) {
   const unsigned gc = nblk(n.C, 4);
-  prof_mark("k_net_checks", s, 1);
+  if (g_prof_on) prof_mark("k_net_checks", s, 1);
   NE_LAUNCH(n.NE, k_checks_cells, gc, 256, s, I, dt, n.cpart, n.mpart);
   hipLaunchKernelGGL(k_checks_final, dim3(1), dim3(256), 0, s, (const float *)n.cpart, (const double *)n.mpart,
                      (int)gc, n.checks, n.mass_out);
-  prof_mark("k_net_checks", s, 0);
+  if (g_prof_on) prof_mark("k_net_checks", s, 0);
   if (hipGetLastError() != hipSuccess) return -1;
   // one host read: the three maxima and the binary64 mass side by side
   if (hipMemcpyAsync(n.check_host, n.checks, 4 * sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess ||
@@ -1056,7 +1200,7 @@ Net *create(const Instance &I, int layers, std::string *err) {
     if (hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0)
       cus = prop.multiProcessorCount;
   }
-  n->dev_blocks = cus;
+  n->cus = cus;
   // parameter segments
   size_t off = 0, boff = 0;
   auto mat = [&](int K, int N) {
@@ -1078,6 +1222,13 @@ Net *create(const Instance &I, int layers, std::string *err) {
   vec(NOUT);
   n->n_params = off;
   n->n_bf = boff;
+  n->table.n = (int)n->segs.size();
+  for (int i = 0; i < n->table.n; ++i) n->table.seg[i] = n->segs[i];
+  // splits of the weight gradients: about 640 rows each, at most 32 (the
+  // partials of a split are one parameter vector, 0.9 MB at four layers)
+  n->splits = std::min(32, std::max(1, (n->C + 639) / 640));
+  n->split_rows = ((n->C + n->splits - 1) / n->splits + GRAD_CH - 1) / GRAD_CH * GRAD_CH;
+  n->splits = (n->C + n->split_rows - 1) / n->split_rows;
   const size_t C = (size_t)n->C, E = (size_t)n->E;
   int rc = 0;
   rc |= n->alloc(&n->params, off);
@@ -1101,11 +1252,12 @@ Net *create(const Instance &I, int layers, std::string *err) {
   rc |= n->alloc(&n->Te, E * HX_ROW);
   rc |= n->alloc(&n->g, E * HX_ROW);
   rc |= n->alloc(&n->dY, C * NOUT);
-  rc |= n->alloc(&n->dP, C * HID);
+  n->dP.assign(layers + 1, nullptr);
+  for (auto &p : n->dP) rc |= n->alloc(&p, C * HID);
   rc |= n->alloc(&n->dH0, C * HID);
   rc |= n->alloc(&n->dH1, C * HID);
   rc |= n->alloc(&n->dZ, C * 2 * HID);
-  rc |= n->alloc(&n->partial, (size_t)GPART * KIN * NOUT);
+  rc |= n->alloc(&n->partial, (size_t)n->splits * off);
   rc |= n->alloc(&n->lpart, (size_t)nblk(E, 4) + 3 * (size_t)nblk(C, 4));
   rc |= n->alloc(&n->loss_out, 4);
   rc |= n->alloc(&n->mpart, 2 * (size_t)nblk(C, 4));

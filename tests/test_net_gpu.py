@@ -278,3 +278,44 @@ def test_ragged_mesh_forward_and_gradients_match_statement(get_case):
     net.close()
     fine.close()
     coarse.close()
+
+
+@pytest.mark.parametrize("name,layers", [("x1.162-moist", 1), ("x1.642-moist", 8), ("x1.2562-moist", 3)])
+def test_gradients_at_row_and_layer_edges(get_case, name, layers):
+    """Fewer rows than one split of the weight gradients, a ragged last tile
+    and split, one layer and the most there are, against the binary64
+    statement (tolerances as above); repeated calls give the same bits."""
+    from hexdyn import learned
+
+    print(f"[gpu] corrector gradients {name}, {layers} layers", flush=True)
+    case = get_case(name)
+    fine, coarse = learned.make_pair_drivers(case)
+    _stepped_pair(case, fine, coarse, seed=5)
+    net = learned.CorrectorNet(coarse, layers)
+    flat = learned.init_params(layers, seed=9, out_gain=0.5)
+    net.set_params(flat)
+    stats = learned.ScaleStats()
+    stats.add(net, coarse, fine)
+    net.set_scales(*stats.scales(case.n_levels))
+    net.set_target(coarse, fine)
+    got = []
+    for _ in range(2):
+        net.forward(coarse, keep=True)
+        lo = net.loss()
+        net.backward()
+        got.append(net.get_grads())
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+    g = _graph(case)
+    p = hn.unpack(flat, layers)
+    cache = hn.forward(p, net.export("X").cpu().numpy(), g, layers)
+    assert _rel(net.export("Y").cpu().numpy(), cache["Y"]) <= 2e-2
+    parts, dY = hn.loss(cache["Y"], net.export("target_cells").cpu().numpy(), net.export("target_edges").cpu().numpy(),
+                        g, case.n_levels)
+    assert abs(lo["total"] - parts["total"]) <= 2e-2 * parts["total"]
+    want = hn.backward(p, cache, dY, g, layers)
+    have = learned.unpack(got[0], layers)
+    bad = [(n, _rel(have[n], want[n])) for n, _ in hn.layout(layers) if not _rel(have[n], want[n]) <= 5e-2]
+    assert not bad, bad
+    net.close()
+    fine.close()
+    coarse.close()
