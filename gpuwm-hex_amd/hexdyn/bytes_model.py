@@ -115,7 +115,8 @@ _K: Dict[str, List[Tuple[str, str]]] = {
     "k_fct_cell1": [("SC", "L"), ("SC", "L"), ("C", "L"), ("C", "W"), ("E", "L"), ("SE", "L"), ("C", "L"),
                     ("SC", "L"), ("SC", "L"), ("SC", "L"), ("SC", "W")],
     "k_fct_edge2": [("SC", "L"), ("SC", "L"), ("SE", "L"), ("SE", "L")],
-    "k_fct_cell2": [("SC", "L"), ("SC", "L"), ("SC", "W"), ("SC", "L"), ("SE", "L"), ("C", "L"), ("SC", "L")],
+    # hres, sin, sout, vres, mass, target | q
+    "k_fct_cell2": [("SE", "L"), ("SC", "L"), ("SC", "L"), ("SC", "W"), ("SC", "L"), ("C", "L"), ("SC", "L")],
     # horizontal mixing, once per subcycle
     "k_mix_lapdiv": [("E", "L"), ("C", "L")],
     "k_mix_lapvort": [("E", "L"), ("V", "L")],
