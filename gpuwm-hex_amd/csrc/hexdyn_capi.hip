@@ -826,6 +826,14 @@ static int create_impl(const hexdyn_mesh *m, const hexdyn_vertical *vt, const he
   rc |= h->upload(&Z.ewp, pad(vt->ewp, L + 1)); rc |= h->upload(&Z.ewm, pad(vt->ewm, L + 1));
   rc |= h->upload(&Z.uinit, pad(vt->u_init, L)); rc |= h->upload(&Z.vinit, pad(vt->v_init, L));
   Z.cf1 = vt->cf1; Z.cf2 = vt->cf2; Z.cf3 = vt->cf3;
+  {
+    // the reference wind's terms are left out only where each is certainly a zero
+    auto all = [](const auto &v, auto ok) { return std::all_of(v.begin(), v.end(), ok); };
+    auto finite = [](float x) { return std::isfinite(x); };
+    bool zero = all(woe, finite) && all(ecos, finite) && all(esin, finite) && all(fedge, finite);
+    for (int k = 0; k < L; ++k) zero = zero && vt->u_init[k] == 0.0f && vt->v_init[k] == 0.0f;
+    n.REFW = zero ? 0 : 1;
+  }
   rc |= h->upload(&Z.zz, rows_cells(vt->zz, L)); rc |= h->upload(&Z.dss, rows_cells(vt->dss, L));
   rc |= h->upload(&Z.rb, rows_cells(vt->rho_base, L)); rc |= h->upload(&Z.rtb, rows_cells(vt->rtheta_base, L));
   rc |= h->upload(&Z.exb, rows_cells(vt->exner_base, L));

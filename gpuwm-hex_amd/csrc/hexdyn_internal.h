@@ -27,6 +27,7 @@ struct Sizes {
   int RS;  // floats from one level row to the next: L + 1 rounded up to 8 (at most HX_ROW)
   int TU;  // distinct advection cells per edge tile (0: the tiled flux gathers are off)
   int OCP;  // 1: in every cell, cellsOnCell slot s is the other cell of edgesOnCell slot s
+  int REFW;  // 1: a reference wind's Coriolis force enters the momentum tendency
   // wavefronts (rows) per block of the launch in flight: each launch passes
   // its own copy, so a kernel finds its tile with its other scalar arguments
   int WPB = 4;
