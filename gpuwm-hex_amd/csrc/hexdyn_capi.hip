@@ -698,6 +698,54 @@ static int create_impl(const hexdyn_mesh *m, const hexdyn_vertical *vt, const he
     }
   Mesh &M = h->I.m;
   int rc = 0;
+  // the vertices of a cell by its own edge slots (the order of MPAS meshes:
+  // vertex s between edges s - 1 and s); another order keeps the vertex passes
+  std::vector<int> vx((size_t)C * ME, 0), vcode(C, 0);
+  std::vector<int> vpos((size_t)C * ME * 3, 0);  // edgesOnVertex slots in the record's order
+  std::vector<float> vrec((size_t)C * HX_ROW, 0.0f);
+  n.VP = 1;
+  for (int nc = 0; nc < C && n.VP; ++nc)
+    for (int s = 0; s < neoc[nc] && n.VP; ++s) {
+      const size_t o = (size_t)nc * ME + s;
+      const int v = voc[o], pe_ = eoc[o], qe = eoc[(size_t)nc * ME + (s + neoc[nc] - 1) % neoc[nc]];
+      int pos[3] = {-1, -1, -1};
+      for (int j = 0; j < 3; ++j) {
+        const int e = eov[3 * v + j];
+        const int w = e == pe_ ? 0 : e == qe ? 1 : 2;
+        if (pos[w] >= 0) n.VP = 0;  // an edge twice, or one of the two missing
+        pos[w] = j;
+      }
+      if (pos[0] < 0 || pos[1] < 0 || pos[2] < 0) n.VP = 0;
+      if (!n.VP) break;
+      int owner = C;
+      for (int j = 0; j < 3; ++j) owner = std::min(owner, new_c[m->cells_on_vertex[3 * h->old_v_h[v] + j]]);
+      vx[o] = eov[3 * v + pos[2]];
+      const int last = pos[0] == 2 ? 0 : pos[1] == 2 ? 1 : 2;
+      vcode[nc] |= last << (2 * s) | (owner == nc ? 1 : 0) << (16 + s);
+      float *r = &vrec[(size_t)nc * HX_ROW + (size_t)s * HX_VREC];
+      const int adds[3] = {last == 0 ? pos[1] : pos[0], last == 2 ? pos[1] : pos[2], pos[last]};
+      for (int w = 0; w < 3; ++w) {
+        vpos[3 * o + w] = adds[w];
+        r[w] = vdc[3 * v + adds[w]];
+        r[3 + w] = vdcdv[3 * v + adds[w]];
+      }
+      r[6] = invtri[v];
+      r[7] = fvert[v];
+    }
+  // every vertex's owner must be a cell that lists it
+  if (n.VP) {
+    std::vector<char> owned(V, 0);
+    for (int nc = 0; nc < C; ++nc)
+      for (int s = 0; s < neoc[nc]; ++s)
+        if (vcode[nc] >> (16 + s) & 1) owned[voc[(size_t)nc * ME + s]] = 1;
+    for (char x : owned)
+      if (!x) n.VP = 0;
+  }
+  if (n.VP) {
+    rc |= h->upload(&M.vx, vx);
+    rc |= h->upload(&M.vcode, vcode);
+    rc |= h->upload(&M.vrec, vrec);
+  }
   rc |= h->upload(&M.csdv, csdv); rc |= h->upload(&M.cdcdv, cdcdv); rc |= h->upload(&M.ckite, ckite);
   rc |= h->upload(&M.vdc, vdc); rc |= h->upload(&M.vdcdv, vdcdv);
   rc |= h->upload(&M.ecos, ecos); rc |= h->upload(&M.esin, esin); rc |= h->upload(&M.ocell, ocell);
@@ -761,6 +809,16 @@ static int create_impl(const hexdyn_mesh *m, const hexdyn_vertical *vt, const he
     rc |= h->upload(&M.defc2, c2s); rc |= h->upload(&M.defs2, s2s); rc |= h->upload(&M.defcs, css);
     rc |= h->upload(&M.mx_fdiv, fdiv); rc |= h->upload(&M.mx_fth2, fth2); rc |= h->upload(&M.mx_fw2, fw2);
     rc |= h->upload(&M.mx_f4, f4); rc |= h->upload(&M.mx_fvort, fvort);
+    if (n.VP) {
+      std::vector<float> mrec((size_t)C * HX_ROW, 0.0f);
+      for (int nc = 0; nc < C; ++nc)
+        for (int s = 0; s < neoc[nc]; ++s)
+          for (int w = 0; w < 3; ++w) {
+            const size_t o = (size_t)nc * ME + s;
+            mrec[(size_t)nc * HX_ROW + (size_t)s * HX_VREC + w] = fvort[3 * (size_t)voc[o] + vpos[3 * o + w]];
+          }
+      rc |= h->upload(&M.mx_vrec, mrec);
+    }
     rc |= h->upload(&M.mx_idc, idc); rc |= h->upload(&M.mx_idv, idv); rc |= h->upload(&M.mx_rdc, rdc);
     rc |= h->upload(&M.mx_rdv, rdv); rc |= h->upload(&M.mx_del2, del2);
     Consts &K0 = h->I.k;

@@ -27,6 +27,7 @@ struct Sizes {
   int RS;  // floats from one level row to the next: L + 1 rounded up to 8 (at most HX_ROW)
   int TU;  // distinct advection cells per edge tile (0: the tiled flux gathers are off)
   int OCP;  // 1: in every cell, cellsOnCell slot s is the other cell of edgesOnCell slot s
+  int VP;    // 1: in every cell, vertex slot s lies between edge slots s - 1 and s (HX_VREC records built)
   int REFW;  // 1: a reference wind's Coriolis force enters the momentum tendency
   // wavefronts (rows) per block of the launch in flight: each launch passes
   // its own copy, so a kernel finds its tile with its other scalar arguments
@@ -36,6 +37,7 @@ struct Sizes {
 // Edge tiles of the staged flux gathers: HX_TILE_E edges per block, at most
 // HX_TILE_U distinct advection cells per tile (larger tiles turn the staged
 // kernels off for the mesh).
+constexpr int HX_VREC = 8;  // values of one vertex in its cell's record (Mesh::vrec)
 constexpr int HX_TILE_E = 8;
 constexpr int HX_TILE_U = 56;
 
@@ -80,6 +82,14 @@ struct Mesh {
   const float *vdcdv;   // [V][3]  dcdv[edge]
   const float *ecos, *esin;  // [E][ME2] cos/sin angle of edgesOnEdge
   const int *ocell;     // [C][ME] the other cell of the slot's edge
+  // the vertices of a cell, for the passes that form them from the cell's rows
+  // (Sizes::VP).  P, Q: the cell's edges of slots s and s - 1; X: the vertex's
+  // third edge.
+  const int *vx;        // [C][ME] X
+  const int *vcode;     // [C] bits 2s, 2s+1: which of P, Q, X (0, 1, 2) is last in edgesOnVertex;
+                        //     bit 16 + s: this cell owns the vertex (the first of its cells on the curve)
+  const float *vrec;    // [C][64] per slot: vdc and vdcdv of the three edges (the last one last), 1/areaTriangle,
+                        //     fVertex
   // horizontal mixing (binary32 factors in the reference's operation order)
   const float *defc2, *defs2, *defcs;  // [C][ME] deformation weights
   const float *mx_fdiv;   // [C][ME] ((1/area)*dv)*sign                        divergence of delsq_u
@@ -87,6 +97,7 @@ struct Mesh {
   const float *mx_fw2;    // [C][ME] (((0.5*(1/area))*sign)*dv)*(1/dc)          w del2
   const float *mx_f4;     // [C][ME] ((((del4*(h4*(1/area)))*dv)*sign)*(1/dc)   theta and w del4
   const float *mx_fvort;  // [V][3]  ((1/areaTriangle)*dc)*vertex sign          vorticity of delsq_u
+  const float *mx_vrec;   // [C][64] per slot: mx_fvort in vrec's order of edges (Sizes::VP)
   const float *mx_idc, *mx_idv, *mx_rdc, *mx_rdv, *mx_del2;  // [E]
 };
 

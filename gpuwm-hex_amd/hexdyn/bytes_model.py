@@ -52,6 +52,8 @@ def step_bytes(*, C: int, L: int, T: int, max_edges: int, n_ac: int, mix: bool =
 _K: Dict[str, List[Tuple[str, str]]] = {
     "k_diag_vertex": [("E", "L"), ("V", "L"), ("V", "L"), ("V", "L")],
     "k_diag_cell": [("E", "L"), ("V", "L"), ("V", "L"), ("C", "L"), ("C", "L"), ("C", "L")],
+    # the two together: u | ke, pv_cell, divergence, pv_vertex, vorticity
+    "k_diag_cv": [("E", "L"), ("C", "L"), ("C", "L"), ("C", "L"), ("V", "L"), ("V", "L")],
     "k_diag_edge": [("E", "L"), ("V", "L"), ("C", "L"), ("E", "L"), ("E", "L")],
     # k_diag_edge's arrays, then k_tend_flux's (the whole-step form of the pass)
     "k_diag_edge_flux": [("E", "L"), ("V", "L"), ("C", "L"), ("E", "L"), ("E", "L"),

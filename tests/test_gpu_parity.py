@@ -706,3 +706,31 @@ def test_state_transfer_round_trips_bitwise(get_case, name, nlev, species):
                                        ct.c_void_p(d.stream_ptr()))
         assert rc == 0
         assert _bits_equal(t.cpu().numpy(), d.export_field(name_f).cpu().numpy()), name_f
+
+
+@pytest.mark.parametrize("name,turn", [("x1.642-moist", 1), ("x1.642-moist", -1), ("r642-moist", 1)])
+def test_other_vertex_slot_order_step_bitwise(get_case, name, turn):
+    """verticesOnCell turned against edgesOnCell (MPAS files keep vertex slot
+    s between edge slots s - 1 and s; in another order the vertices keep a
+    pass of their own), with mixing: 2 steps bit for bit."""
+    import copy
+    import dataclasses
+
+    print(f"[gpu] {name} verticesOnCell turned by {turn}, 2 steps", flush=True)
+    base = _mixing(get_case, name)
+    mesh = copy.deepcopy(base.mesh)
+    n = mesh.arrays["nEdgesOnCell"]
+    for table in ("verticesOnCell", "kiteForCell"):
+        t = mesh.arrays[table].copy()
+        for c in range(t.shape[0]):
+            t[c, : n[c]] = np.roll(t[c, : n[c]], turn)
+        mesh.arrays[table] = t
+    case = dataclasses.replace(base, mesh=mesh)
+    o = Oracle(case, 32)
+    o.set_state(initial_state_arrays(case), rebuild=True)
+    assert o.step(2) == 0
+    d = _driver(case)
+    d.step_device(2)
+    ref, got = o.get_state(), d.get_state()
+    for k in ref:
+        assert _bits_equal(ref[k], got[k]), f"{k}: {_diff(ref[k], got[k])}"
