@@ -1325,7 +1325,7 @@ int hexdyn_recover(hexdyn_handle *h, int stage, void *stream) {
 int hexdyn_solve_diagnostics(hexdyn_handle *h, int rk_step, void *stream) {
   if (!h || rk_step < 1 || rk_step > 3) return HEXDYN_E_INVALID;
   Instance J = view(h, false);
-  return NS_CALL(h, solve_diagnostics, J, rk_step, (hipStream_t)stream) ? HEXDYN_E_HIP : 0;
+  return NS_CALL(h, solve_diagnostics, J, rk_step, 0, (hipStream_t)stream) ? HEXDYN_E_HIP : 0;
 }
 
 int hexdyn_end_subcycle(hexdyn_handle *h, int subcycle, void *stream) {
@@ -1381,7 +1381,7 @@ int enqueue_step(hexdyn_handle *h, hipStream_t s) {
       // the last stage's diagnostics would only feed a subcycle that does not
       // follow: the next step's begin_step recomputes them from the published state
       if (!(sub == c.config_dynamics_split_steps && st == 3))
-        rc |= NS_CALL(h, solve_diagnostics, step_view(h, false), st, s);
+        rc |= NS_CALL(h, solve_diagnostics, step_view(h, false), st, 1, s);
     }
   }
   if (rc == 0 && c.config_split_dynamics_transport && transported(h))

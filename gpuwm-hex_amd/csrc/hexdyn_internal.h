@@ -227,7 +227,7 @@ struct Instance {
   int acoustic_substep(const Instance &I, int stage, int ss, int sub, int damp_prev, hipStream_t s); \
   int divergence_damping(const Instance &I, int stage, hipStream_t s);    \
   int recover(const Instance &I, int stage, int sub, int damp, hipStream_t s); \
-  int solve_diagnostics(const Instance &I, int rk, hipStream_t s);        \
+  int solve_diagnostics(const Instance &I, int rk, int with_w, hipStream_t s); \
   int scalars_stage(const Instance &I, int stage, hipStream_t s);         \
   int rebuild_saved(const Instance &I, hipStream_t s);                    \
   int rebuild_cells(const Instance &I, hipStream_t s);                    \

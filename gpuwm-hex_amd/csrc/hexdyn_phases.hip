@@ -2136,59 +2136,72 @@ KB k_divdamp(const Instance I, float coefficient) {
 }
 
 // --------------------------------------------------------------------- recovery
-// w from rw and the terrain-following horizontal flux (terrain.py:491-571).
-// ru_row(e) returns lane k's value of the edge momentum row of edge e.
-template <int NE, class RU>
-__device__ __forceinline__ float recover_w_column(const Instance &I, int c, int k, float rho_k, float rw_k, RU ru_row,
-                                                  float *hdiv_out = nullptr) {
-  const int L = I.n.L;
-  const int n = I.m.neoc[c];
-  int e[NE];
-#pragma unroll
-  for (int s = 0; s < NE; ++s) e[s] = I.m.eoc[c * NE + s];
-  SlotRow<NE> sgr = slot_row<NE>(I.m.csign + c * NE);
-  SlotRow<NE> sdr = slot_row<NE>(I.m.csdv + c * NE);
-  const float ia = uni_load(I.m.invarea + c);
-  const float zk = AT(I.z.zz, c, k);
-  const float fzm = AT(I.z.fzm, 0, k), fzp = AT(I.z.fzp, 0, k);
+// w from rw and the terrain-following horizontal flux (terrain.py:491-571) of
+// the edge momentum ru, and (hdiv_out) its mass-flux divergence.
+template <int NE>
+struct RecWIn {
   float ru[NE], zb[NE], zb3[NE];
+  SlotRow<NE> sg, sd;
+  float ia, zk, fzm, fzp;
+  int n, e[NE];
+};
+template <int NE>
+__device__ __forceinline__ void rec_w_index(const Instance &I, int c, int k, RecWIn<NE> &a) {
+  a.n = I.m.neoc[c];
+#pragma unroll
+  for (int s = 0; s < NE; ++s) a.e[s] = I.m.eoc[c * NE + s];
+  a.sg = slot_row<NE>(I.m.csign + c * NE);
+  a.sd = slot_row<NE>(I.m.csdv + c * NE);
+  a.ia = uni_load(I.m.invarea + c);
+  a.zk = AT(I.z.zz, c, k);
+  a.fzm = AT(I.z.fzm, 0, k);
+  a.fzp = AT(I.z.fzp, 0, k);
 #pragma unroll
   for (int s = 0; s < NE; ++s) {
-    zb[s] = AT(I.z.zb, c * NE + s, k);
-    zb3[s] = AT(I.z.zb3, c * NE + s, k);
+    a.zb[s] = AT(I.z.zb, c * NE + s, k);
+    a.zb3[s] = AT(I.z.zb3, c * NE + s, k);
   }
+}
+template <int NE>
+__device__ __forceinline__ void rec_w_fence(const RecWIn<NE> &a) {
 #pragma unroll
-  for (int s = 0; s < NE; ++s) fence(e[s]);
+  for (int s = 0; s < NE; ++s) fence(a.e[s]);
+}
+template <int NE>
+__device__ __forceinline__ void rec_w_rows(const Instance &I, const float *ru, int k, RecWIn<NE> &a) {
 #pragma unroll
-  for (int s = 0; s < NE; ++s) ru[s] = ru_row(e[s]);
-  keep(ru, zb, zb3);
-  SlotRow<NE> sgs = sgr, sd = sdr;
-  settle(sgs, sd);
+  for (int s = 0; s < NE; ++s) a.ru[s] = AT(ru, a.e[s], k);
+}
+template <int NE, bool HDIV>
+__device__ __forceinline__ float rec_w_compute(const Instance &I, int k, const RecWIn<NE> &a, float rho_k, float rw_k,
+                                               float &hdiv) {
+  const int L = I.n.L, n = a.n;
   float sg[NE];
-  slot_vals(sgs, sg);
-  const float zkm = up1(zk);
-  if (hdiv_out) {
+#pragma unroll
+  for (int s = 0; s < NE; ++s) sg[s] = a.sg[s];
+  const float zkm = up1(a.zk);
+  if (HDIV) {
     // mass-flux divergence of the recovered ru (dynamics.py:86-121), next stage's hdiv
     float acc = 0.0f;
 #pragma unroll
     for (int s = 0; s < NE; ++s)
-      if (s < n) acc = acc + sd[s] * ru[s];
-    *hdiv_out = acc * ia;
+      if (s < n) acc = acc + a.sd[s] * a.ru[s];
+    hdiv = acc * a.ia;
   }
   float col = 0.0f;
-  if (k >= 1 && k < L) col = rw_k / (fzm * zk + fzp * zkm);
+  if (k >= 1 && k < L) col = rw_k / (a.fzm * a.zk + a.fzp * zkm);
   const float cf1 = I.z.cf1, cf2 = I.z.cf2, cf3 = I.z.cf3;
 #pragma unroll
   for (int s = 0; s < NE; ++s) {
-    const float ru_m = up1(ru[s]);
-    const float ru0 = rdl(ru[s], 0), ru1 = rdl(ru[s], 1), ru2 = rdl(ru[s], 2);
+    const float ru_m = up1(a.ru[s]);
+    const float ru0 = rdl(a.ru[s], 0), ru1 = rdl(a.ru[s], 1), ru2 = rdl(a.ru[s], 2);
     if (s < n) {
       if (k == 0) {
         const float flux = (cf1 * ru0 + cf2 * ru1) + cf3 * ru2;
-        col = col + (sg[s] * (zb[s] + cs1(flux) * zb3[s])) * flux;
+        col = col + (sg[s] * (a.zb[s] + cs1(flux) * a.zb3[s])) * flux;
       } else if (k < L) {
-        const float flux = fzm * ru[s] + fzp * ru_m;
-        col = col + (sg[s] * (zb[s] + cs1(flux) * zb3[s])) * flux;
+        const float flux = a.fzm * a.ru[s] + a.fzp * ru_m;
+        col = col + (sg[s] * (a.zb[s] + cs1(flux) * a.zb3[s])) * flux;
       }
     }
   }
@@ -2198,29 +2211,56 @@ __device__ __forceinline__ float recover_w_column(const Instance &I, int c, int 
     const float bottom = (cf1 * r0 + cf2 * r1) + cf3 * r2;
     col = col / bottom;
   } else if (k < L) {
-    col = col / (fzm * rho_k + fzp * rho_m);
+    col = col / (a.fzm * rho_k + a.fzp * rho_m);
   } else {
     col = 0.0f;
   }
   return col;
+}
+template <int NE, bool HDIV>
+__device__ __forceinline__ float recover_w_column(const Instance &I, int c, int k, float rho_k, float rw_k,
+                                                  const float *ru, float &hdiv) {
+  RecWIn<NE> a;
+  rec_w_index(I, c, k, a);
+  rec_w_fence(a);
+  rec_w_rows(I, ru, k, a);
+  keep(a.ru, a.zb, a.zb3);
+  settle(a.sg, a.sd);
+  return rec_w_compute<NE, HDIV>(I, k, a, rho_k, rw_k, hdiv);
 }
 
 // The part of a recovery that reads the cell's recovered edges, after a column
 // pass that recovered the column: terrain w and (HDIV) the next stage's
 // mass-flux divergence.  After stage 3 the next subcycle's opening pass forms
 // the divergence again.
-template <int NE, bool HDIV>
-KB k_rec_w(const Instance I) {
+// DIAG: also the cell and vertex diagnostics of the recovered u, which read
+// the same edges: one batch of loads and one launch instead of two (55 us
+// against 34 + 34 at x1.40962).
+template <int NE, bool HDIV, bool DIAG>
+KB k_rec_w(const Instance I, int store_mix) {
   const int c = wave_entity(I);
   if (c >= I.n.C) return;
   const int k = lane();
   const float rho = AT(I.b.c_rho, c, k), rwv = AT(I.b.c_rw, c, k);
-  const float *cru = I.b.c_ru;
+  RecWIn<NE> a;
+  CellVertIn<NE> d;
+  rec_w_index(I, c, k, a);
+  if (DIAG) cell_vert_index(I, c, d);
+  rec_w_fence(a);
+  if (DIAG) cell_vert_fence(d);
+  rec_w_rows(I, I.b.c_ru, k, a);
+  if (DIAG) cell_vert_rows(I, I.b.u, k, d);
+  keep(a.ru, a.zb, a.zb3);
+  settle(a.sg, a.sd);
   float hd = 0.0f;
-  const float wv =
-      recover_w_column<NE>(I, c, k, rho, rwv, [&](int e) { return AT(cru, e, k); }, HDIV ? &hd : nullptr);
+  const float wv = rec_w_compute<NE, HDIV>(I, k, a, rho, rwv, hd);
+  if (DIAG) {
+    keep(d.uo, d.ux, d.ia);
+    settle(d.sd, d.dd, d.kt, d.rec);
+  }
   if (HDIV && k < I.n.L) AT(I.b.hdiv, c, k) = hd;
   if (k <= I.n.L) AT(I.b.w, c, k) = wv;
+  if (DIAG) cell_vert_finish(I, c, k, d, store_mix);
 }
 
 // The whole cell recovery as a pass of its own (the phase entry points).
@@ -2249,11 +2289,10 @@ KB k_rec_cell(const Instance I, int sub, float inv_steps) {
   const float rho = lay ? dp + rb : 1.0f;
   const float rtv = lay ? rp + rtb : 1.0f;
   const float rwv = inner ? srw + rwp : 0.0f;
-  const float *cru = I.b.c_ru;
   float hd = 0.0f;
   // hdiv feeds the next stage's momentum tendency; after stage 3 the next
   // subcycle's opening pass forms it again
-  const float wv = recover_w_column<NE>(I, c, k, rho, rwv, [&](int e) { return AT(cru, e, k); }, S3 ? nullptr : &hd);
+  const float wv = recover_w_column<NE, !S3>(I, c, k, rho, rwv, I.b.c_ru, hd);
   int bad = (lay && (!(rho > 0.0f) || !(rtv > 0.0f))) ? 1 : 0;
   const float th = rtv / rho;
   float ex = 0.0f, ppv = 0.0f;
@@ -2342,8 +2381,8 @@ KB k_rebuild_cell(const Instance I) {
   const float rtb = AT(I.z.rtb, c, k), rb = AT(I.z.rb, c, k), exb = AT(I.z.exb, c, k);
   const float rwk = AT(I.b.rw, c, k);
   const float rho = k < L ? rho_k : 1.0f;
-  const float *ru = I.b.ru;
-  const float wv = recover_w_column<NE>(I, c, k, rho, rwk, [&](int e) { return AT(ru, e, k); });
+  float hd;
+  const float wv = recover_w_column<NE, false>(I, c, k, rho, rwk, I.b.ru, hd);
   if (k < L) {
     const float ex = exner_pow(I, (zk * I.k.cfac) * rt);
     const float rtp = rt - rtb;
@@ -2894,12 +2933,23 @@ inline bool tiled_flux_on(const Instance &I) {
   return I.n.TU > 0 && !(I.tune && I.tune->find("k_diag_edge_flux") >= 0);
 }
 
-int solve_diagnostics(const Instance &I, int rk, hipStream_t s) {
+// with_w: the whole step's recovery left w (and hdiv) to this pass over the cells
+int solve_diagnostics(const Instance &I, int rk, int with_w, hipStream_t s) {
   // divergence and vorticity are read only by the horizontal mixing, from
   // the diagnostics that open a subcycle (rk 3, and the step's first), or by
   // an export between phases
   const int store_mix = rk == 3 || I.k.store_flux ? 1 : 0;
-  if (I.n.VP) {
+  const bool whole = with_w && I.n.VP;
+  if (with_w) {
+#define REC_W(NE) \
+  (rk == 3 ? (whole ? RW(NE, false, true) : RW(NE, false, false)) : (whole ? RW(NE, true, true) : RW(NE, true, false)))
+#define RW(NE, HD, DI) launch_named("k_rec_w", k_rec_w<NE, HD, DI>, I.n.C, 1, s, I, store_mix)
+    NEDISPATCH(I, REC_W(6), REC_W(7));
+#undef RW
+#undef REC_W
+  }
+  if (whole) {
+  } else if (I.n.VP) {
     LAUNCH_NE(I, k_diag_cv, I.n.C, 1, s, I, (const float *)I.b.u, store_mix);
   } else {
     launch(k_diag_vertex, I.n.V, 1, s, I, (const float *)I.b.u, store_mix);
@@ -2935,7 +2985,7 @@ int begin_step(const Instance &I, hipStream_t s) {
     launch(k_moist_cell, I.n.C, 1, s, I);
     launch(k_moist_edge, I.n.E, 1, s, I);
   }
-  return solve_diagnostics(I, 3, s);
+  return solve_diagnostics(I, 3, 0, s);
 }
 
 int begin_subcycle(const Instance &I, int sub, hipStream_t s) {
@@ -3109,6 +3159,7 @@ void recover_edges(const Instance &I, int sub, float inv, bool damp, bool avgrp,
 }
 
 int recover(const Instance &I, int stage, int sub, int damp, hipStream_t s) {
+  const bool last = stage == 3 && sub == I.k.splits;
   const float inv = I.k.inv_steps[stage - 1];
   const bool avgrp = I.k.fused && I.k.steps[stage - 1] == 1;
   const float coef = I.k.dts_inv_coef[stage - 1];
@@ -3116,13 +3167,12 @@ int recover(const Instance &I, int stage, int sub, int damp, hipStream_t s) {
     recover_edges<true>(I, sub, inv, damp != 0, avgrp, coef, I.k.dts[stage - 1], s);
   else
     recover_edges<false>(I, sub, inv, damp != 0, avgrp, coef, I.k.dts[stage - 1], s);
-  if (I.k.fused) {  // the column pass recovered the rest
-    if (stage == 3)
-      NEDISPATCH(I, launch_named("k_rec_w", k_rec_w<6, false>, I.n.C, 1, s, I),
-                 launch_named("k_rec_w", k_rec_w<7, false>, I.n.C, 1, s, I));
-    else
-      NEDISPATCH(I, launch_named("k_rec_w", k_rec_w<6, true>, I.n.C, 1, s, I),
-                 launch_named("k_rec_w", k_rec_w<7, true>, I.n.C, 1, s, I));
+  if (I.k.fused) {
+    // the column pass recovered the rest; w and hdiv come with the diagnostics
+    // that follow, except after a step's last stage, which has none
+    if (last)
+      NEDISPATCH(I, launch_named("k_rec_w", k_rec_w<6, false, false>, I.n.C, 1, s, I, 0),
+                 launch_named("k_rec_w", k_rec_w<7, false, false>, I.n.C, 1, s, I, 0));
   } else if (stage == 3) {
     NEDISPATCH(I, launch_named("k_rec_cell", k_rec_cell<6, true>, I.n.C, 1, s, I, sub, inv),
                launch_named("k_rec_cell", k_rec_cell<7, true>, I.n.C, 1, s, I, sub, inv));

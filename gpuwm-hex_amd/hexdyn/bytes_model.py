@@ -99,8 +99,9 @@ _K: Dict[str, List[Tuple[str, str]]] = {
               ("E", "W"), ("C", "W"), ("E", "L"), ("CM", "W"), ("CM", "W"), ("C", "L")]
              + [("C", "L")] * 7 + [("C", "L")] * 3 + [("C", "L")] * 2 + [("C", "L")] * 4 + [("C", "W")]
              + [("C", "L")] * 3 + [("C", "W")],
-    # rho, rw, ru, zz, zb, zb3 | w, hdiv
-    "k_rec_w": [("C", "L"), ("C", "W"), ("E", "L"), ("C", "L"), ("CM", "W"), ("CM", "W"), ("C", "W"), ("C", "L")],
+    # rho, rw, ru, zz, zb, zb3, u | w, hdiv, ke, pv_cell, pv_vertex
+    "k_rec_w": [("C", "L"), ("C", "W"), ("E", "L"), ("C", "L"), ("CM", "W"), ("CM", "W"), ("E", "L"), ("C", "W"),
+                ("C", "L"), ("C", "L"), ("C", "L"), ("V", "L")],
     "k_divdamp": [("C", "L"), ("C", "L"), ("C", "L"), ("E", "L"), ("E", "L")],
     # s_rho_p, rho_pp, s_rtheta_p, rtheta_pp, rb, rtb, s_rw, rw_p, ww_avg, s_ru, ru_p, zz, zb, zb3, exb |
     # rho_p, rtheta_p, c_rho, c_rt, theta, c_rw, flux_w, w, (exner, pp)
