@@ -209,12 +209,11 @@ inline int nblocks(int n, int wpb) { return (n + wpb - 1) / wpb; }
 // vertical recurrences of the block's cells run together on the lanes of
 // one wavefront (lane = cell) through LDS rows padded to COLP floats, so
 // W columns cost one column's dependent chain instead of W.  The implicit
-// coefficients take 16 columns per block; the acoustic column update, whose
-// two sweeps hold the block for longer, takes 8 (four blocks per CU
-// overlap their loads with the others' sweeps: 57 -> 53 us; the
-// coefficients were 1 us slower at 8).
+// coefficients on their own take 16 columns per block; the acoustic column
+// update (8 columns: the same time, 16: 57 us for 53) and a stage's whole column
+// pass take 4, whose sweeps hold up fewer wavefronts.
 constexpr int COLW_VC = 16;  // k_vcoef
-constexpr int COLW_AC = 8;   // k_ac_cell and k_col (one level row staged by each wavefront)
+constexpr int COLW_AC = 4;   // k_ac_cell and k_col
 constexpr int COLP = 65;
 // The column blocks of a CU need every SIMD to hold 8 wavefronts: the
 // register budget is capped for that (at 7 a CU would hold one block of 16).
@@ -230,17 +229,17 @@ __device__ __forceinline__ void stage_levels(float *s_lev, const float *const (&
     if (w == j) s_lev[j * 64 + k] = rows[j][k];
 }
 
-// 1 / x with IEEE round-to-nearest.  For |x| in [2^-100, 2^100] the hardware
-// reciprocal with one FMA correction is the correctly rounded quotient
-// (verified exhaustively over every binary32 x of that range); other inputs
-// take the division itself.
-__device__ __forceinline__ float recip(float x) {
+// 1 / x with IEEE round-to-nearest for |x| in [2^-100, 2^100]: the hardware
+// reciprocal with one FMA correction is the correctly rounded quotient there
+// (verified exhaustively over every binary32 x of that range).  Callers take
+// the division outside it.
+__device__ __forceinline__ bool recip_in_range(float x) {
   const float a = fabsf(x);
-  if (a >= 0x1p-100f && a <= 0x1p100f) {
-    const float y0 = __builtin_amdgcn_rcpf(x);
-    return __builtin_fmaf(__builtin_fmaf(-x, y0, 1.0f), y0, y0);
-  }
-  return 1.0f / x;
+  return a >= 0x1p-100f && a <= 0x1p100f;
+}
+__device__ __forceinline__ float recip(float x) {
+  const float y0 = __builtin_amdgcn_rcpf(x);
+  return __builtin_fmaf(__builtin_fmaf(-x, y0, 1.0f), y0, y0);
 }
 
 // A block of U levels of a column's LDS rows in registers.  Levels past the
@@ -291,25 +290,45 @@ __device__ __forceinline__ void thomas_sweeps(float *x, const float *pd, const f
   for (j -= U; j >= 0; j -= U) p = sweep_down<true, U>(x, pg, j, U, p);
 }
 // alpha/gamma recurrence up the column (acoustic_v841.py:81-233): alpha over
-// pa, gamma over pb; returns 1 where a denominator vanishes.  Blocks of 4: the
-// division dominates a level's chain, and the fused column pass has few
-// registers to spare.
+// pa, gamma over pb; returns 1 where a denominator vanishes.  A block of levels
+// is worked with the corrected reciprocal, its range tested once for the block,
+// and again with the division where a denominator of any column left the range
+// (x1.162, a coefficient sweep: 211 cycles a level with the test at every
+// level and the division behind it, about 120 so).  Blocks of 4: the fused column pass has
+// few registers to spare.
 template <bool WHOLE, int U>
-__device__ __forceinline__ float sweep_coef(float *pa, float *pb, const float *pc, int j, int m, float dts2, float gm,
+__device__ __forceinline__ float sweep_coef(float *pa, float *pb, const float *pc, int j, int m, float dts2, float gm0,
                                             int &singular) {
-  float av[U], bv[U], cv[U];
+  float av[U], bv[U], cv[U], al[U], gv[U];
   sweep_load(av, pa, j);
   sweep_load(bv, pb, j);
   sweep_load(cv, pc, j);
+  float gm = gm0;
+  bool in_range = true;
 #pragma unroll
   for (int u = 0; u < U; ++u)
     if (WHOLE || u < m) {
       const float den = 1.0f + dts2 * (bv[u] - av[u] * gm);
-      if (den == 0.0f) singular = 1;
-      const float al = recip(den);
-      gm = (dts2 * cv[u]) * al;
-      pa[j + u] = al;
-      pb[j + u] = gm;
+      in_range = in_range && recip_in_range(den);
+      al[u] = recip(den);
+      gv[u] = gm = (dts2 * cv[u]) * al[u];
+    }
+  if (__any(!in_range)) {
+    gm = gm0;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (WHOLE || u < m) {
+        const float den = 1.0f + dts2 * (bv[u] - av[u] * gm);
+        if (den == 0.0f) singular = 1;
+        al[u] = 1.0f / den;
+        gv[u] = gm = (dts2 * cv[u]) * al[u];
+      }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (WHOLE || u < m) {
+      pa[j + u] = al[u];
+      pb[j + u] = gv[u];
     }
   return gm;
 }
@@ -1982,19 +2001,22 @@ KBCOL(COLW_AC) k_ac_cell(const Instance I, float dts, int store_old, const RecAr
 // each of these reads the column's rows again (theta, zz, rw, w, tend_ru of
 // the cell's edges) and hands its result over through memory (five
 // coefficient rows, two tendencies, the perturbations).  x1.40962 moist, the
-// stages of a subcycle with their recovery: 136 + 166 + 111 us against 168 +
-// 182 + 115 us in passes of their own (HBM-bound, 4.0-4.5 TB/s); x1.162, where
+// stages of a subcycle with their recovery: 95 + 116 + 93 us against 168 + 182
+// + 115 us in passes of their own (HBM-bound, 4.3-4.8 TB/s); x1.162, where
 // each launch costs about 5 us: a whole step 662 -> 432 us with the side
 // stream of the coefficients gone.
-// A CU holds four blocks of eight columns (blocks of four: the same times).
-// The registers of eight wavefronts per SIMD do not hold every part's rows at
-// once: the coefficients wait in LDS until the acoustic part, and its rows are
-// loaded when the theta part has freed its own (spills cost their traffic:
-// 130 MB a launch when the parts were left to overlap).  Seven-edge cells take
-// six wavefronts per SIMD.
+// The coefficients wait in LDS until the acoustic part, and its rows are loaded
+// when the theta part has freed its registers.  Wavefronts per SIMD: as many as
+// hold the pass without spills, seven (six with coefficients and correction
+// flux, or seven-edge cells); a CU then holds seven or six blocks of four
+// columns, and the sweeps of some run under the loads of the others.  At eight
+// wavefronts 3-11 registers spill, and their traffic costs more than the
+// occupancy gives: 119 + 166 + 112 us a subcycle's three stages at x1.40962
+// against 95 + 116 + 93 (blocks of eight columns at six: 103 + 120 + 93).
 template <int NE, bool VC, bool CORR, bool MIX, bool LAST, bool S3>
-__global__ void __launch_bounds__(64 * COLW_AC) __attribute__((amdgpu_waves_per_eu(NE == 6 ? 8 : 6, NE == 6 ? 8 : 6)))
-k_col(const Instance I, float dts, const float *__restrict__ rtp, int store_old, int store_cof, int store_t,
+__global__ void __launch_bounds__(64 * COLW_AC)
+    __attribute__((amdgpu_waves_per_eu(NE == 6 && !(VC && CORR) ? 7 : 6, NE == 6 && !(VC && CORR) ? 7 : 6)))
+    k_col(const Instance I, float dts, const float *__restrict__ rtp, int store_old, int store_cof, int store_t,
       const RecArgs ra) {
   constexpr int COLW = COLW_AC;
   __shared__ float s_x[COLW * COLP], s_d[COLW * COLP], s_l[COLW * COLP], s_g[COLW * COLP];
