@@ -807,18 +807,21 @@ static int create_impl(const hexdyn_mesh *m, const hexdyn_vertical *vt, const he
       rdv[ne] = scale * idv[ne];
     }
     rc |= h->upload(&M.defc2, c2s); rc |= h->upload(&M.defs2, s2s); rc |= h->upload(&M.defcs, css);
-    rc |= h->upload(&M.mx_fdiv, fdiv); rc |= h->upload(&M.mx_fth2, fth2); rc |= h->upload(&M.mx_fw2, fw2);
+    rc |= h->upload(&M.mx_fdiv, fdiv);
     rc |= h->upload(&M.mx_f4, f4); rc |= h->upload(&M.mx_fvort, fvort);
-    if (n.VP) {
-      std::vector<float> mrec((size_t)C * HX_ROW, 0.0f);
-      for (int nc = 0; nc < C; ++nc)
-        for (int s = 0; s < neoc[nc]; ++s)
-          for (int w = 0; w < 3; ++w) {
-            const size_t o = (size_t)nc * ME + s;
-            mrec[(size_t)nc * HX_ROW + (size_t)s * HX_VREC + w] = fvort[3 * (size_t)voc[o] + vpos[3 * o + w]];
-          }
-      rc |= h->upload(&M.mx_vrec, mrec);
-    }
+    std::vector<float> mrec((size_t)C * HX_ROW, 0.0f);
+    for (int nc = 0; nc < C; ++nc)
+      for (int s = 0; s < neoc[nc]; ++s) {
+        const size_t o = (size_t)nc * ME + s;
+        float *r = &mrec[(size_t)nc * HX_ROW + (size_t)s * HX_VREC];
+        for (int w = 0; w < 3 && n.VP; ++w) r[w] = fvort[3 * (size_t)voc[o] + vpos[3 * o + w]];
+        r[3] = fdiv[o];
+        r[4] = fth2[o];
+        r[5] = fw2[o];
+        r[6] = del2[eoc[o]];
+        r[7] = csign[o];
+      }
+    rc |= h->upload(&M.mx_rec, mrec);
     rc |= h->upload(&M.mx_idc, idc); rc |= h->upload(&M.mx_idv, idv); rc |= h->upload(&M.mx_rdc, rdc);
     rc |= h->upload(&M.mx_rdv, rdv); rc |= h->upload(&M.mx_del2, del2);
     Consts &K0 = h->I.k;

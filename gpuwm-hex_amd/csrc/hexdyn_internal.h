@@ -93,11 +93,11 @@ struct Mesh {
   // horizontal mixing (binary32 factors in the reference's operation order)
   const float *defc2, *defs2, *defcs;  // [C][ME] deformation weights
   const float *mx_fdiv;   // [C][ME] ((1/area)*dv)*sign                        divergence of delsq_u
-  const float *mx_fth2;   // [C][ME] (((1/area)*sign)*dv)*(1/dc)                theta del2
-  const float *mx_fw2;    // [C][ME] (((0.5*(1/area))*sign)*dv)*(1/dc)          w del2
   const float *mx_f4;     // [C][ME] ((((del4*(h4*(1/area)))*dv)*sign)*(1/dc)   theta and w del4
   const float *mx_fvort;  // [V][3]  ((1/areaTriangle)*dc)*vertex sign          vorticity of delsq_u
-  const float *mx_vrec;   // [C][64] per slot: mx_fvort in vrec's order of edges (Sizes::VP)
+  const float *mx_rec;    // [C][64] per slot: mx_fvort in vrec's order of edges (Sizes::VP), mx_fdiv,
+                          //         theta del2 (((1/area)*sign)*dv)*(1/dc), w del2 (((0.5*(1/area))*sign)*dv)*(1/dc),
+                          //         mx_del2 of the edge, csign
   const float *mx_idc, *mx_idv, *mx_rdc, *mx_rdv, *mx_del2;  // [E]
 };
 

@@ -61,13 +61,12 @@ __device__ __forceinline__ uint32_t row_off(int rs, int ent, int k) {
 // First entity of this block: blocks are renumbered so that XCD x (hardware
 // block b runs on XCD b % 8) owns a contiguous range of the curve.  wpb is
 // the number of wavefronts (entities) per block.
-__device__ __forceinline__ int block_entity0(int wpb) {
-  const int nb = gridDim.x;
-  const int b = blockIdx.x;
+__device__ __forceinline__ int block_entity0(int b, int nb, int wpb) {
   const int x = b & 7, i = b >> 3, q = nb >> 3, r = nb & 7;
   const int lb = (x < r) ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
   return lb * wpb;
 }
+__device__ __forceinline__ int block_entity0(int wpb) { return block_entity0(blockIdx.x, gridDim.x, wpb); }
 // Column kernels: WPB rows per block, fixed at compile time.
 template <int WPB>
 __device__ __forceinline__ int wave_entity() {
@@ -79,6 +78,16 @@ __device__ __forceinline__ int wave_entity() {
 // before its first row load.
 __device__ __forceinline__ int wave_entity(const Instance &I) {
   return __builtin_amdgcn_readfirstlane(block_entity0(I.n.WPB) + (int)(threadIdx.x >> 6));
+}
+// Two independent gather passes in one launch: the first nb0 blocks (a
+// multiple of 8, so that the second pass's blocks keep their XCDs) are the
+// first pass's, the others the second's.
+__device__ __forceinline__ int wave_entity_first(const Instance &I, int nb0) {
+  return __builtin_amdgcn_readfirstlane(block_entity0(blockIdx.x, nb0, I.n.WPB) + (int)(threadIdx.x >> 6));
+}
+__device__ __forceinline__ int wave_entity_second(const Instance &I, int nb0) {
+  return __builtin_amdgcn_readfirstlane(block_entity0(blockIdx.x - nb0, gridDim.x - nb0, I.n.WPB) +
+                                        (int)(threadIdx.x >> 6));
 }
 __device__ __forceinline__ int lane() { return (int)(threadIdx.x & 63); }
 // Value of lane k-1 (lane 0: its own) and k+1 (lane 63: its own): whole-wave
@@ -1035,69 +1044,85 @@ KB k_mix_lapvort(const Instance I) {
   if (k < I.n.L) AT(I.b.delsq_vort, v, k) = acc;
 }
 
-// del4 of u (momentum_filter_lap4_v841_f32): pool - rho_e*((ddiv*r_dc) - (dvort*r_dv))
-KB k_mix_edge4(const Instance I) {
-  const int e = wave_entity(I);
-  if (e >= I.n.E) return;
-  const int k = lane();
-  const int c0 = I.m.coe[2 * e], c1 = I.m.coe[2 * e + 1];
-  const int v0 = I.m.voe[2 * e], v1 = I.m.voe[2 * e + 1];
-  const float d0 = AT(I.b.delsq_div, c0, k), d1 = AT(I.b.delsq_div, c1, k);
-  const float z0 = AT(I.b.delsq_vort, v0, k), z1 = AT(I.b.delsq_vort, v1, k);
-  const float r0 = AT(I.b.c_rho, c0, k), r1 = AT(I.b.c_rho, c1, k);
-  const float eru = AT(I.b.euler_ru, e, k);
-  const float rdc = uni_load(I.m.mx_rdc + e), rdv = uni_load(I.m.mx_rdv + e);
-  const float rho_e = 0.5f * (r0 + r1);
-  const float diffusion = rho_e * ((d1 - d0) * rdc - (z1 - z0) * rdv);
-  if (k < I.n.L) AT(I.b.euler_ru, e, k) = eru - diffusion;
-}
-
 // del2 of theta and of w (theta_filter_lap2_v841_f32, w_filter_lap2_v841_f32).
 // Without the fourth-order part (MIX4 false) the results go straight to the
-// Euler pools.
-template <int NE, bool MIX4>
+// Euler pools.  LAP: also the divergence and, at the vertices the cell owns,
+// the vorticity of delsq_u, from the cell's own and outward edges as in
+// k_diag_cv; every weight of a slot comes in one record row, where a row each
+// and a scalar load per edge cost the wavefront their issue.  The three passes
+// took 30.5 + 13.4 + 16.7 us at x1.40962, this one 47.0 (126 MB counted once,
+// 2.7 TB/s: bound by the issue of its 41 row loads).
+template <int NE, bool MIX4, bool LAP>
 KB k_mix_cell(const Instance I) {
   const int c = wave_entity(I);
   if (c >= I.n.C) return;
   const int k = lane();
   const int L = I.n.L;
   const int n = I.m.neoc[c];
-  int e[NE], o[NE];
+  const int code = LAP ? I.m.vcode[c] : 0;
+  int e[NE], x[NE], o[NE];
 #pragma unroll
   for (int s = 0; s < NE; ++s) {
-    e[s] = I.m.eoc[c * NE + s];
+    e[s] = LAP ? I.m.eoc[c * NE + s] : 0;
+    x[s] = LAP ? I.m.vx[c * NE + s] : 0;
     o[s] = I.m.ocell[c * NE + s];
   }
-  SlotRow<NE> sgr = slot_row<NE>(I.m.csign + c * NE), f2r = slot_row<NE>(I.m.mx_fth2 + c * NE),
-                    fwr = slot_row<NE>(I.m.mx_fw2 + c * NE);
+  SlotRow<HX_ROW> rec = slot_row<HX_ROW>(I.m.mx_rec + c * HX_ROW);
   const float thc = AT(I.b.theta, c, k), rhc = AT(I.b.c_rho, c, k), wc = AT(I.b.w, c, k);
   const float kdc = AT(I.b.kdiff, c, k);
   const float erw = MIX4 ? 0.0f : AT(I.b.euler_rw, c, k);
+  fence(code);
 #pragma unroll
   for (int s = 0; s < NE; ++s) {
     fence(e[s]);
+    fence(x[s]);
     fence(o[s]);
   }
-  float tho[NE], rho[NE], wo[NE], kdo[NE], d2[NE];
+  float tho[NE], rho[NE], wo[NE], kdo[NE], uo[NE], ux[NE];
 #pragma unroll
   for (int s = 0; s < NE; ++s) {
     tho[s] = AT(I.b.theta, o[s], k);
     rho[s] = AT(I.b.c_rho, o[s], k);
     wo[s] = AT(I.b.w, o[s], k);
     kdo[s] = AT(I.b.kdiff, o[s], k);
-    d2[s] = uni_load(I.m.mx_del2 + e[s]);
+    uo[s] = LAP ? AT(I.b.delsq_u, e[s], k) : 0.0f;
+    ux[s] = LAP ? AT(I.b.delsq_u, x[s], k) : 0.0f;
   }
-  keep(tho, rho, wo, kdo, d2);
-  settle(sgr, f2r, fwr);
-  float sg[NE], f2[NE], fw[NE];
-  slot_vals(sgr, sg);
-  slot_vals(f2r, f2);
-  slot_vals(fwr, fw);
+  keep(tho, rho, wo, kdo);
+  if (LAP) keep(uo, ux);
+  settle(rec);
+  if (LAP) {
+    float acc = 0.0f;
+    float uq = uo[2];  // the edge row of slot s - 1: of the last slot for s = 0
+#pragma unroll
+    for (int s = 3; s < NE; ++s) uq = s < n ? uo[s] : uq;
+#pragma unroll
+    for (int s = 0; s < NE; ++s)
+      if (s < n) {
+        const float up = uo[s];
+        const int r = s * HX_VREC;
+        acc = acc + rec[r + 3] * up;
+        if (code >> (16 + s) & 1) {
+          const int last = code >> (2 * s) & 3;
+          const float u0 = last == 0 ? uq : up, u1 = last == 2 ? uq : ux[s],
+                      u2 = last == 2 ? ux[s] : last == 1 ? uq : up;
+          float z = 0.0f + rec[r] * u0;
+          z = z + rec[r + 1] * u1;
+          z = z + rec[r + 2] * u2;
+          const int v = I.m.voc[c * NE + s];
+          if (k < L) AT(I.b.delsq_vort, v, k) = z;
+        }
+        uq = up;
+      }
+    if (k < L) AT(I.b.delsq_div, c, k) = acc;
+  }
   float lap = 0.0f, tend = 0.0f, lapw = 0.0f, tendw = 0.0f;
 #pragma unroll
   for (int s = 0; s < NE; ++s) {
     // cell0/cell1 of edge s in cellsOnEdge order
-    const bool first = sg[s] > 0.0f;
+    const int r = s * HX_VREC;
+    const float f2 = rec[r + 4], fw = rec[r + 5], d2 = rec[r + 6];
+    const bool first = rec[r + 7] > 0.0f;
     const float th0 = first ? thc : tho[s], th1 = first ? tho[s] : thc;
     const float r0 = first ? rhc : rho[s], r1 = first ? rho[s] : rhc;
     const float w0 = first ? wc : wo[s], w1 = first ? wo[s] : wc;
@@ -1106,13 +1131,13 @@ KB k_mix_cell(const Instance I) {
     const float rho_em = up1(rho_e);
     const float k0m = up1(k0), k1m = up1(k1);
     if (s < n) {
-      const float flux = (f2[s] * (th1 - th0)) * rho_e;
+      const float flux = (f2 * (th1 - th0)) * rho_e;
       lap = lap + flux;
-      tend = tend + ((flux * 0.5f) * (k0 + k1)) * d2[s];
-      const float fluxw = (fw[s] * (rho_e + rho_em)) * (w1 - w0);
+      tend = tend + ((flux * 0.5f) * (k0 + k1)) * d2;
+      const float fluxw = (fw * (rho_e + rho_em)) * (w1 - w0);
       lapw = lapw + fluxw;
       const float sum_k = ((k0 + k1) + k0m) + k1m;
-      tendw = tendw + ((fluxw * d2[s]) * 0.25f) * sum_k;
+      tendw = tendw + ((fluxw * d2) * 0.25f) * sum_k;
     }
   }
   if (k == 0 || k >= L) {
@@ -1133,10 +1158,7 @@ KB k_mix_cell(const Instance I) {
 
 // del4 of theta and of w (theta_filter_lap4_v841_f32, w_filter_lap4_v841_f32), then the w pool
 template <int NE>
-KB k_mix_cell4(const Instance I) {
-  const int c = wave_entity(I);
-  if (c >= I.n.C) return;
-  const int k = lane();
+__device__ __forceinline__ void mix_cell4(const Instance &I, int c, int k) {
   const int L = I.n.L;
   const int n = I.m.neoc[c];
   int o[NE];
@@ -1172,6 +1194,36 @@ KB k_mix_cell4(const Instance I) {
     }
   if (k < L) AT(I.b.euler_theta, c, k) = tend;
   if (k <= L) AT(I.b.euler_rw, c, k) = erw + tendw;
+}
+
+// del4 of u (momentum_filter_lap4_v841_f32): pool - rho_e*((ddiv*r_dc) - (dvort*r_dv))
+__device__ __forceinline__ void mix_edge4(const Instance &I, int e, int k) {
+  const int c0 = I.m.coe[2 * e], c1 = I.m.coe[2 * e + 1];
+  const int v0 = I.m.voe[2 * e], v1 = I.m.voe[2 * e + 1];
+  const float d0 = AT(I.b.delsq_div, c0, k), d1 = AT(I.b.delsq_div, c1, k);
+  const float z0 = AT(I.b.delsq_vort, v0, k), z1 = AT(I.b.delsq_vort, v1, k);
+  const float r0 = AT(I.b.c_rho, c0, k), r1 = AT(I.b.c_rho, c1, k);
+  const float eru = AT(I.b.euler_ru, e, k);
+  const float rdc = uni_load(I.m.mx_rdc + e), rdv = uni_load(I.m.mx_rdv + e);
+  const float rho_e = 0.5f * (r0 + r1);
+  const float diffusion = rho_e * ((d1 - d0) * rdc - (z1 - z0) * rdv);
+  if (k < I.n.L) AT(I.b.euler_ru, e, k) = eru - diffusion;
+}
+
+// the fourth-order part, after k_mix_cell: edges of the momentum pool in the
+// first nb0 blocks, cells of the theta and w pools in the others: 29.9 +
+// 18.1 us as two launches at x1.40962, 47.4 as one; on small meshes the launch
+// (4 to 5 us) is most of either.
+template <int NE>
+KB k_mix4(const Instance I, int nb0) {
+  const int k = lane();
+  if ((int)blockIdx.x < nb0) {
+    const int e = wave_entity_first(I, nb0);
+    if (e < I.n.E) mix_edge4(I, e, k);
+  } else {
+    const int c = wave_entity_second(I, nb0);
+    if (c < I.n.C) mix_cell4<NE>(I, c, k);
+  }
 }
 
 // ------------------------------------------------------------ subcycle start
@@ -2919,6 +2971,17 @@ inline void launch_named(const char *name, K kernel, int n, int gy, hipStream_t 
 }
 #define launch(kernel, ...) launch_named(#kernel, kernel, __VA_ARGS__)
 
+// two gather passes in one launch, n0 rows of the first and n1 of the second
+template <typename K>
+inline void launch_pair(const char *name, K kernel, int n0, int n1, hipStream_t s, Instance I) {
+  const int wpb = wpb_from(name, I);
+  I.n.WPB = wpb;
+  const int nb0 = (nblocks(n0, wpb) + 7) & ~7;
+  if (g_prof_on) prof_mark(name, s, 1);
+  hipLaunchKernelGGL(kernel, dim3(nb0 + nblocks(n1, wpb)), dim3(64 * wpb), 0, s, I, nb0);
+  if (g_prof_on) prof_mark(name, s, 0);
+}
+
 // column kernels: W cells per block of 64*W threads
 template <int W, class K, class... A>
 inline void launch_col_named(const char *name, K kernel, int n, hipStream_t s, A... args) {
@@ -3035,18 +3098,19 @@ int begin_subcycle(const Instance &I, int sub, hipStream_t s) {
     launch_named("k_sub_edge", k_sub_edge<false>, I.n.E, 1, s, I);
   }
   if (I.k.mixing) {
-    if (I.k.mix4) {
+    const bool mix4 = I.k.mix4 != 0, lap = mix4 && I.n.VP;
+    if (mix4 && !lap) {
       LAUNCH_NE(I, k_mix_lapdiv, I.n.C, 1, s, I);
       launch(k_mix_lapvort, I.n.V, 1, s, I);
-      launch(k_mix_edge4, I.n.E, 1, s, I);
     }
-    if (I.k.mix4)
-      NEDISPATCH(I, launch_named("k_mix_cell", k_mix_cell<6, true>, I.n.C, 1, s, I),
-                 launch_named("k_mix_cell", k_mix_cell<7, true>, I.n.C, 1, s, I));
-    else
-      NEDISPATCH(I, launch_named("k_mix_cell", k_mix_cell<6, false>, I.n.C, 1, s, I),
-                 launch_named("k_mix_cell", k_mix_cell<7, false>, I.n.C, 1, s, I));
-    if (I.k.mix4) LAUNCH_NE(I, k_mix_cell4, I.n.C, 1, s, I);
+#define MIX(NE, M4, LA) launch_named("k_mix_cell", k_mix_cell<NE, M4, LA>, I.n.C, 1, s, I)
+#define MIX_NE(NE) (lap ? MIX(NE, true, true) : mix4 ? MIX(NE, true, false) : MIX(NE, false, false))
+    NEDISPATCH(I, MIX_NE(6), MIX_NE(7));
+#undef MIX_NE
+#undef MIX
+    if (mix4)
+      NEDISPATCH(I, launch_pair("k_mix4", k_mix4<6>, I.n.E, I.n.C, s, I),
+                 launch_pair("k_mix4", k_mix4<7>, I.n.E, I.n.C, s, I));
   }
   return check();
 }

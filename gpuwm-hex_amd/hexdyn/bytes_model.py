@@ -125,8 +125,12 @@ _K: Dict[str, List[Tuple[str, str]]] = {
     "k_mix_lapvort": [("E", "L"), ("V", "L")],
     # delsq_div, delsq_vort, c_rho, euler_ru | euler_ru
     "k_mix_edge4": [("C", "L"), ("V", "L"), ("C", "L"), ("E", "L"), ("E", "L")],
-    # theta, c_rho, w, kdiff | delsq_theta, euler_theta, delsq_w, tend_w
-    "k_mix_cell": [("C", "L"), ("C", "L"), ("C", "W"), ("C", "L"), ("C", "L"), ("C", "L"), ("C", "L"), ("C", "W")],
+    # theta, c_rho, w, kdiff, delsq_u | delsq_theta, euler_theta, delsq_w, tend_w, delsq_div, delsq_vort
+    "k_mix_cell": [("C", "L"), ("C", "L"), ("C", "W"), ("C", "L"), ("E", "L"), ("C", "L"), ("C", "L"), ("C", "L"),
+                   ("C", "W"), ("C", "L"), ("V", "L")],
+    # k_mix_edge4's and k_mix_cell4's arrays
+    "k_mix4": [("C", "L"), ("V", "L"), ("C", "L"), ("E", "L"), ("E", "L"), ("C", "L"), ("C", "L"), ("C", "L"),
+               ("C", "W"), ("C", "W"), ("C", "L"), ("C", "W")],
     # delsq_theta, delsq_w, euler_theta, tend_w, euler_rw | euler_theta, euler_rw
     "k_mix_cell4": [("C", "L"), ("C", "L"), ("C", "L"), ("C", "W"), ("C", "W"), ("C", "L"), ("C", "W")],
 }

@@ -734,3 +734,23 @@ def test_other_vertex_slot_order_step_bitwise(get_case, name, turn):
     ref, got = o.get_state(), d.get_state()
     for k in ref:
         assert _bits_equal(ref[k], got[k]), f"{k}: {_diff(ref[k], got[k])}"
+
+
+@pytest.mark.parametrize("waves", [4, 16])
+def test_paired_launches_bitwise(get_case, waves):
+    """Passes that share a launch: at 16 wavefronts a block the 480 edges of
+    x1.162 fill 30 blocks, which the launch rounds up to a multiple of the 8
+    XCDs; the cells' blocks follow.  2 steps bit for bit."""
+    from hexdyn import autotune
+
+    print(f"[gpu] x1.162-moist mixing, {waves} wavefronts a block, 2 steps", flush=True)
+    case = _mixing(get_case, "x1.162-moist")
+    o = Oracle(case, 32)
+    o.set_state(initial_state_arrays(case), rebuild=True)
+    assert o.step(2) == 0
+    d = _driver(case)
+    autotune.set_launch(d, "*", waves)
+    d.step_device(2)
+    ref, got = o.get_state(), d.get_state()
+    for k in ref:
+        assert _bits_equal(ref[k], got[k]), f"{k}: {_diff(ref[k], got[k])}"
