@@ -14,8 +14,8 @@
  * renumbered so each XCD (hardware assigns block b to XCD b % 8) works on a
  * contiguous range of the space-filling-curve order and its L2 sees the
  * neighbour rows it needs.  Vertical neighbours come from cross-lane moves;
- * the serial column recurrences (Thomas sweep, implicit coefficients) run one
- * column per lane out of LDS, in the reference's arithmetic order.
+ * the serial column recurrences (Thomas sweep, implicit coefficients) pass
+ * from lane to lane, in the reference's arithmetic order.
  *
  * Reference operators (operation order per element):
  *   solve diagnostics  cuda_horizontal_v841.py:67-200, diagnostics.py:95-306
@@ -214,16 +214,12 @@ __device__ __forceinline__ float uni_load(const float *__restrict__ p) {
 
 inline int nblocks(int n, int wpb) { return (n + wpb - 1) / wpb; }
 
-// Column kernels: W cells (one wavefront each) per block.  The serial
-// vertical recurrences of the block's cells run together on the lanes of
-// one wavefront (lane = cell) through LDS rows padded to COLP floats, so
-// W columns cost one column's dependent chain instead of W.  The implicit
-// coefficients on their own take 16 columns per block; the acoustic column
-// update (8 columns: the same time, 16: 57 us for 53) and a stage's whole column
-// pass take 4, whose sweeps hold up fewer wavefronts.
+// Column kernels: W cells (one wavefront each) per block, which share the
+// per-level coefficient rows in LDS.  The implicit coefficients on their own
+// take 16 columns per block, the acoustic column update (8 columns: the same
+// time, 16: 57 us for 53) and a stage's whole column pass 4.
 constexpr int COLW_VC = 16;  // k_vcoef
 constexpr int COLW_AC = 4;   // k_ac_cell and k_col
-constexpr int COLP = 65;
 // The column blocks of a CU need every SIMD to hold 8 wavefronts: the
 // register budget is capped for that (at 7 a CU would hold one block of 16).
 #define KBCOL(W) __global__ void __launch_bounds__(64 * (W)) __attribute__((amdgpu_waves_per_eu(8, 8)))
@@ -251,102 +247,80 @@ __device__ __forceinline__ float recip(float x) {
   return __builtin_fmaf(__builtin_fmaf(-x, y0, 1.0f), y0, y0);
 }
 
-// A block of U levels of a column's LDS rows in registers.  Levels past the
-// column's last are read too (rows hold COLP >= 8 * ceil(L / 8) floats) and
-// used by nobody.
-template <int U>
-__device__ __forceinline__ void sweep_load(float (&r)[U], const float *p, int j) {
-#pragma unroll
-  for (int u = 0; u < U; ++u) r[u] = p[j + u];
+// Value of lane k-1 (lane 0: zero) and k+1 (lane 63: zero): whole-wave DPP
+// shifts that the compiler folds into the multiplication that reads them.
+__device__ __forceinline__ float up0(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x138, 0xf, 0xf, true));
 }
-// The serial recurrences of one column (lane = column).  Each level's step
-// waits for the one before, so the time is the chain's: the LDS reads of a
-// block of levels are issued together ahead of the block's chain, and the
-// levels left after the whole blocks form one block too (m of its U levels)
-// instead of a loop that pays the LDS latency at every level.
-// Thomas sweeps (acoustic_v841.py:296-565): forward for levels 1..L-1, back
-// substitution for levels L-1..0.
-template <bool WHOLE, int U>
-__device__ __forceinline__ float sweep_up(float *x, const float *pd, const float *pl, int j, int m, float p) {
-  float xv[U], dv[U], lv[U];
-  sweep_load(xv, x, j);
-  sweep_load(dv, pd, j);
-  sweep_load(lv, pl, j);
+__device__ __forceinline__ float dn0(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x130, 0xf, 0xf, true));
+}
+
+// The serial recurrences of a column, lane k being level k: every lane repeats
+// its level's step from its neighbour's last value, so after i steps the first
+// i levels are final, and a further step gives them the same bits (the count
+// rounds up to whole unrolled blocks; a lane exchange keeps the compiler from
+// unrolling a loop with a remainder).  The dependent chain of a level is what
+// one lane per column would run, which bounds the pass on small meshes; with
+// one wavefront sweeping the columns of its block out of LDS the chain also
+// waited for LDS reads and two block barriers, and the block's other
+// wavefronts for it.  The issue slots are about the same, one column's steps
+// on a whole wavefront against four columns' LDS reads and writes.  k_col with
+// coefficients 12.1 -> 9.2 us and without 8.4 -> 6.9 at x1.162, k_ac_cell 8.8
+// -> 8.1; at x1.40962, where other columns hide the chain, 96 + 115 + 94 -> 95
+// + 112 + 93 us the stages of a subcycle.
+// Thomas sweeps (acoustic_v841.py:296-565): forward for levels 1..L-1 with
+// the sub-diagonal d and 1/denominator l, back substitution with g for levels
+// L-1..0.  Levels past L give zero.
+__device__ __forceinline__ float thomas_sweeps(float x, float d, float l, float g, int k, int L) {
+  const bool inner = k >= 1 && k < L;
+  d = inner ? d : 0.0f;
+  l = inner ? l : 1.0f;
+  g = inner ? g : 0.0f;
+  x = k <= L ? x : 0.0f;
+  float p = x;
+  for (int i = 1; i < L; i += 8) {
 #pragma unroll
-  for (int u = 0; u < U; ++u)
-    if (WHOLE || u < m) x[j + u] = p = (xv[u] - dv[u] * p) * lv[u];
+    for (int u = 0; u < 8; ++u) p = (x - d * up0(p)) * l;
+  }
+  x = p;
+  for (int i = 0; i < L; i += 8) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) p = x - g * dn0(p);
+  }
   return p;
-}
-template <bool WHOLE, int U>
-__device__ __forceinline__ float sweep_down(float *x, const float *pg, int j, int m, float p) {
-  float xv[U], gv[U];
-  sweep_load(xv, x, j);
-  sweep_load(gv, pg, j);
-#pragma unroll
-  for (int u = U - 1; u >= 0; --u)
-    if (WHOLE || u < m) x[j + u] = p = xv[u] - gv[u] * p;
-  return p;
-}
-__device__ __forceinline__ void thomas_sweeps(float *x, const float *pd, const float *pl, const float *pg, int L) {
-  constexpr int U = 8;
-  float p = x[0];
-  int j = 1;
-  for (; j + U <= L; j += U) p = sweep_up<true, U>(x, pd, pl, j, U, p);
-  if (j < L) sweep_up<false, U>(x, pd, pl, j, L - j, p);
-  p = x[L];
-  j = L / U * U;
-  if (j < L) p = sweep_down<false, U>(x, pg, j, L - j, p);
-  for (j -= U; j >= 0; j -= U) p = sweep_down<true, U>(x, pg, j, U, p);
 }
 // alpha/gamma recurrence up the column (acoustic_v841.py:81-233): alpha over
-// pa, gamma over pb; returns 1 where a denominator vanishes.  A block of levels
-// is worked with the corrected reciprocal, its range tested once for the block,
-// and again with the division where a denominator of any column left the range
-// (x1.162, a coefficient sweep: 211 cycles a level with the test at every
-// level and the division behind it, about 120 so).  Blocks of 4: the fused column pass has
-// few registers to spare.
-template <bool WHOLE, int U>
-__device__ __forceinline__ float sweep_coef(float *pa, float *pb, const float *pc, int j, int m, float dts2, float gm0,
-                                            int &singular) {
-  float av[U], bv[U], cv[U], al[U], gv[U];
-  sweep_load(av, pa, j);
-  sweep_load(bv, pb, j);
-  sweep_load(cv, pc, j);
-  float gm = gm0;
-  bool in_range = true;
+// a, gamma over b, zero at the levels that have no equation; returns 1 where
+// this level's denominator vanishes.  With the corrected reciprocal, and where
+// one of the column's final denominators left that one's range again with the
+// division.
+__device__ __forceinline__ int coef_sweep(float &a, float &b, float c, int k, int L, float dts2) {
+  const bool inner = k >= 1 && k < L;
+  a = inner ? a : 0.0f;
+  b = inner ? b : 0.0f;
+  c = inner ? dts2 * c : 0.0f;
+  float gm = 0.0f, al = 1.0f, den = 1.0f;
+  for (int i = 1; i < L; i += 8) {  // L - 1 steps in whole blocks
 #pragma unroll
-  for (int u = 0; u < U; ++u)
-    if (WHOLE || u < m) {
-      const float den = 1.0f + dts2 * (bv[u] - av[u] * gm);
-      in_range = in_range && recip_in_range(den);
-      al[u] = recip(den);
-      gv[u] = gm = (dts2 * cv[u]) * al[u];
+    for (int u = 0; u < 8; ++u) {
+      den = 1.0f + dts2 * (b - a * up0(gm));
+      al = recip(den);
+      gm = c * al;
     }
-  if (__any(!in_range)) {
-    gm = gm0;
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (WHOLE || u < m) {
-        const float den = 1.0f + dts2 * (bv[u] - av[u] * gm);
-        if (den == 0.0f) singular = 1;
-        al[u] = 1.0f / den;
-        gv[u] = gm = (dts2 * cv[u]) * al[u];
-      }
   }
-#pragma unroll
-  for (int u = 0; u < U; ++u)
-    if (WHOLE || u < m) {
-      pa[j + u] = al[u];
-      pb[j + u] = gv[u];
+  int singular = 0;
+  if (__any(!recip_in_range(den))) {
+    gm = 0.0f;
+    for (int i = 1; i < L; ++i) {
+      den = 1.0f + dts2 * (b - a * up0(gm));
+      al = 1.0f / den;
+      gm = c * al;
     }
-  return gm;
-}
-__device__ __forceinline__ int coef_sweep(float *pa, float *pb, const float *pc, int L, float dts2) {
-  constexpr int U = 4;
-  float gm = 0.0f;
-  int singular = 0, j = 1;
-  for (; j + U <= L; j += U) gm = sweep_coef<true, U>(pa, pb, pc, j, U, dts2, gm, singular);
-  if (j < L) sweep_coef<false, U>(pa, pb, pc, j, L - j, dts2, gm, singular);
+    singular = den == 0.0f ? 1 : 0;
+  }
+  a = inner ? al : 0.0f;
+  b = gm;
   return singular;
 }
 
@@ -938,7 +912,6 @@ __device__ __forceinline__ void store_coefs(const Instance &I, int c, int k, flo
 KBCOL(COLW_VC) k_vcoef(const Instance I, float dts, const float *__restrict__ exn, const float *__restrict__ theta,
               const float *__restrict__ rtp) {
   constexpr int COLW = COLW_VC;
-  __shared__ float s_a[COLW * COLP], s_b[COLW * COLP], s_c[COLW * COLP];
   __shared__ float s_lev[6 * 64];
   const int w = (int)(threadIdx.x >> 6);
   const int c0 = wave_entity<COLW>();
@@ -955,19 +928,9 @@ KBCOL(COLW_VC) k_vcoef(const Instance I, float dts, const float *__restrict__ ex
   __syncthreads();
   const CoefOut o = coef_system(I, r, k, s_lev[0 * 64 + k], s_lev[1 * 64 + k], s_lev[2 * 64 + k], s_lev[3 * 64 + k],
                                 s_lev[4 * 64 + k], s_lev[5 * 64 + k]);
-  s_a[w * COLP + k] = o.a;
-  s_b[w * COLP + k] = o.b;
-  s_c[w * COLP + k] = o.cc;
-  __syncthreads();
-  if (w == 0 && k < COLW) {
-    const int singular = coef_sweep(s_a + k * COLP, s_b + k * COLP, s_c + k * COLP, L, dts * dts);
-    if (singular && block_entity0(COLW) + k < I.n.C) set_flag(I.b.flag);
-  }
-  __syncthreads();
-  const bool inner = k >= 1 && k < L;
-  if (live)
-    store_coefs(I, c, k, o.coftz, o.cofwt, o.cofwz, o.a, inner ? s_a[w * COLP + k] : 0.0f,
-                inner ? s_b[w * COLP + k] : 0.0f);
+  float a = o.a, b = o.b;
+  if (coef_sweep(a, b, o.cc, k, L, dts * dts) && live) set_flag(I.b.flag);
+  if (live) store_coefs(I, c, k, o.coftz, o.cofwt, o.cofwz, o.a, a, b);
 }
 
 // ------------------------------------------------------- horizontal mixing
@@ -1959,7 +1922,6 @@ struct RecArgs {
 template <int NE, bool FIRST, bool LAST, bool S3>
 KBCOL(COLW_AC) k_ac_cell(const Instance I, float dts, int store_old, const RecArgs ra) {
   constexpr int COLW = COLW_AC;
-  __shared__ float s_x[COLW * COLP], s_d[COLW * COLP], s_l[COLW * COLP], s_g[COLW * COLP];
   __shared__ float s_lev[LV_N * 64];
   const int w = (int)(threadIdx.x >> 6);
   const int c0 = wave_entity<COLW>();
@@ -2020,18 +1982,11 @@ KBCOL(COLW_AC) k_ac_cell(const Instance I, float dts, int store_old, const RecAr
   __syncthreads();
   float col, ad;
   const AcMid m = ac_rhs<NE, FIRST>(I, q, sg, sd, ia, n, k, dts, s_lev, col, ad);
-  s_x[w * COLP + k] = col;
-  s_d[w * COLP + k] = ad;
-  s_l[w * COLP + k] = q.al;
-  s_g[w * COLP + k] = q.ga;
   RecIn r;
   if (LAST) r = rec_rows<S3>(I, c, k);  // in flight during the sweeps
-  __syncthreads();
-  if (w == 0 && k < COLW)
-    thomas_sweeps(s_x + k * COLP, s_d + k * COLP, s_l + k * COLP, s_g + k * COLP, L);
-  __syncthreads();
+  col = thomas_sweeps(col, ad, q.al, q.ga, k, L);
   const AcOut a =
-      ac_update(I, m, s_x[w * COLP + k], q.srw, q.crw, q.damp, q.crho, q.wk, q.zk, q.coftz, k, dts, s_lev);
+      ac_update(I, m, col, q.srw, q.crw, q.damp, q.crho, q.wk, q.zk, q.coftz, k, dts, s_lev);
   if (!live) return;
   if (!LAST || ra.store_work) {
     if (k <= L) {
@@ -2053,7 +2008,7 @@ KBCOL(COLW_AC) k_ac_cell(const Instance I, float dts, int store_old, const RecAr
 // each of these reads the column's rows again (theta, zz, rw, w, tend_ru of
 // the cell's edges) and hands its result over through memory (five
 // coefficient rows, two tendencies, the perturbations).  x1.40962 moist, the
-// stages of a subcycle with their recovery: 95 + 116 + 93 us against 168 + 182
+// stages of a subcycle with their recovery: 95 + 112 + 93 us against 168 + 182
 // + 115 us in passes of their own (HBM-bound, 4.3-4.8 TB/s); x1.162, where
 // each launch costs about 5 us: a whole step 662 -> 432 us with the side
 // stream of the coefficients gone.
@@ -2061,17 +2016,18 @@ KBCOL(COLW_AC) k_ac_cell(const Instance I, float dts, int store_old, const RecAr
 // when the theta part has freed its registers.  Wavefronts per SIMD: as many as
 // hold the pass without spills, seven (six with coefficients and correction
 // flux, or seven-edge cells); a CU then holds seven or six blocks of four
-// columns, and the sweeps of some run under the loads of the others.  At eight
+// columns, and the chains of some run under the loads of the others.  At eight
 // wavefronts 3-11 registers spill, and their traffic costs more than the
 // occupancy gives: 119 + 166 + 112 us a subcycle's three stages at x1.40962
-// against 95 + 116 + 93 (blocks of eight columns at six: 103 + 120 + 93).
+// against 95 + 116 + 93, both with the columns swept out of LDS (blocks of eight
+// columns at six: 103 + 120 + 93).
 template <int NE, bool VC, bool CORR, bool MIX, bool LAST, bool S3>
 __global__ void __launch_bounds__(64 * COLW_AC)
     __attribute__((amdgpu_waves_per_eu(NE == 6 && !(VC && CORR) ? 7 : 6, NE == 6 && !(VC && CORR) ? 7 : 6)))
     k_col(const Instance I, float dts, const float *__restrict__ rtp, int store_old, int store_cof, int store_t,
       const RecArgs ra) {
   constexpr int COLW = COLW_AC;
-  __shared__ float s_x[COLW * COLP], s_d[COLW * COLP], s_l[COLW * COLP], s_g[COLW * COLP];
+  __shared__ float s_x[VC ? COLW * 64 : 1], s_l[COLW * 64], s_g[COLW * 64];
   __shared__ float s_cof[VC ? 3 * COLW * 64 : 1];  // coftz, cofwt, cofwz
   __shared__ float s_lev[LV_N * 64];
   const int w = (int)(threadIdx.x >> 6);
@@ -2098,9 +2054,9 @@ __global__ void __launch_bounds__(64 * COLW_AC)
     __syncthreads();
     const CoefOut cf = coef_system(I, r, k, s_lev[LV_FZM * 64 + k], s_lev[LV_FZP * 64 + k], s_lev[LV_RDZU * 64 + k],
                                    s_lev[LV_RDZW * 64 + k], s_lev[LV_ETP * 64 + k], s_lev[LV_EWP * 64 + k]);
-    s_l[w * COLP + k] = cf.a;
-    s_g[w * COLP + k] = cf.b;
-    s_x[w * COLP + k] = cf.cc;
+    s_l[w * 64 + k] = cf.a;
+    s_g[w * 64 + k] = cf.b;
+    s_x[w * 64 + k] = cf.cc;
     s_cof[(0 * COLW + w) * 64 + k] = cf.coftz;
     s_cof[(1 * COLW + w) * 64 + k] = cf.cofwt;
     s_cof[(2 * COLW + w) * 64 + k] = cf.cofwz;
@@ -2118,18 +2074,17 @@ __global__ void __launch_bounds__(64 * COLW_AC)
   AcIn<NE> q;
   theta_rows<NE, CORR, MIX>(I, e, c, k, t);
   if (!VC) w_rows<NE>(I, e, c, k, v);
-  __syncthreads();
-  if (VC) {
-    if (w == 0 && k < COLW) {
-      const int singular = coef_sweep(s_l + k * COLP, s_g + k * COLP, s_x + k * COLP, L, dts * dts);
-      if (singular && block_entity0(COLW) + k < I.n.C) set_flag(I.b.flag);
-    }
+  if (!VC) {
     __syncthreads();
+  } else {
+    float ca = s_l[w * 64 + k], cb = s_g[w * 64 + k];
+    if (coef_sweep(ca, cb, s_x[w * 64 + k], k, L, dts * dts) && live) set_flag(I.b.flag);
+    s_l[w * 64 + k] = ca;
+    s_g[w * 64 + k] = cb;
     w_rows<NE>(I, e, c, k, v);
-    if (!inner) s_l[w * COLP + k] = s_g[w * COLP + k] = 0.0f;  // alpha and gamma of the other levels
     if (live && store_cof)
       store_coefs(I, c, k, s_cof[(0 * COLW + w) * 64 + k], s_cof[(1 * COLW + w) * 64 + k],
-                  s_cof[(2 * COLW + w) * 64 + k], 0.0f, s_l[w * COLP + k], s_g[w * COLP + k]);
+                  s_cof[(2 * COLW + w) * 64 + k], 0.0f, ca, cb);
   }
   keep(t.fth);
   if (CORR) keep(t.fco);
@@ -2159,8 +2114,8 @@ __global__ void __launch_bounds__(64 * COLW_AC)
     q.coftz = AT(I.b.coftz, c, k);
     q.cofwt = AT(I.b.cofwt, c, k);
     q.cofwz = AT(I.b.cofwz, c, k);
-    s_l[w * COLP + k] = AT(I.b.alpha, c, k);
-    s_g[w * COLP + k] = AT(I.b.gamma, c, k);
+    s_l[w * 64 + k] = AT(I.b.alpha, c, k);
+    s_g[w * 64 + k] = AT(I.b.gamma, c, k);
   }
   if (live && store_t) store_tend(I, c, k, q.trt, q.trw);
   q.sthc = t.ths;
@@ -2175,17 +2130,12 @@ __global__ void __launch_bounds__(64 * COLW_AC)
   keep(q.sto);
   float col, ad;
   const AcMid m = ac_rhs<NE, true>(I, q, sg, sd, ia, n, k, dts, s_lev, col, ad);
-  s_x[w * COLP + k] = col;
-  s_d[w * COLP + k] = ad;
   hold_loads();
   RecIn r;
   if (LAST) r = rec_rows<S3>(I, c, k);  // in flight during the sweeps
-  __syncthreads();
-  if (w == 0 && k < COLW)
-    thomas_sweeps(s_x + k * COLP, s_d + k * COLP, s_l + k * COLP, s_g + k * COLP, L);
-  __syncthreads();
+  col = thomas_sweeps(col, ad, s_l[w * 64 + k], s_g[w * 64 + k], k, L);
   const AcOut a =
-      ac_update(I, m, s_x[w * COLP + k], q.srw, q.crw, q.damp, q.crho, q.wk, q.zk, q.coftz, k, dts, s_lev);
+      ac_update(I, m, col, q.srw, q.crw, q.damp, q.crho, q.wk, q.zk, q.coftz, k, dts, s_lev);
   if (!live) return;
   if (!LAST || ra.store_work) {
     if (k <= L) {

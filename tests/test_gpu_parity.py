@@ -754,3 +754,27 @@ def test_paired_launches_bitwise(get_case, waves):
     ref, got = o.get_state(), d.get_state()
     for k in ref:
         assert _bits_equal(ref[k], got[k]), f"{k}: {_diff(ref[k], got[k])}"
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e30])
+def test_implicit_coefficients_out_of_reciprocal_range(get_case, scale):
+    """Every third column with exner scaled so that the denominators of its
+    implicit system leave the range of the corrected reciprocal (above
+    2**100): those columns take the division.  Coefficients bit for bit."""
+    print(f"[gpu] implicit coefficients x1.162-moist, exner x {scale:g} in every third column", flush=True)
+    case = get_case("x1.162-moist")
+    o = Oracle(case, 32)
+    o.set_state(initial_state_arrays(case), rebuild=True)
+    a = o.get_state()
+    a["exner"][:, ::3] *= np.float32(scale)
+    o.set_state(a, rebuild=False)
+    d = _driver(case)
+    d.set_state(a, saved=a)
+    o.begin_step(); d.phase("begin_step")
+    o.begin_subcycle(1); d.phase("begin_subcycle", 1)
+    alpha = o.export_field("ALPHA_TRI")
+    small = (alpha != 0.0) & (np.abs(alpha) < 2.0 ** -100)
+    assert bool(small.any()) == (scale > 1.0) and np.isfinite(alpha).all()
+    for f in ("A_TRI", "ALPHA_TRI", "GAMMA_TRI", "COFWZ", "COFWT", "COFTZ"):
+        x, y = o.export_field(f), d.export_field(f).cpu().numpy()
+        assert _bits_equal(x, y), f"{f}: {_diff(x, y)}"
