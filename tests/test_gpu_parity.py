@@ -778,3 +778,49 @@ def test_implicit_coefficients_out_of_reciprocal_range(get_case, scale):
     for f in ("A_TRI", "ALPHA_TRI", "GAMMA_TRI", "COFWZ", "COFWT", "COFTZ"):
         x, y = o.export_field(f), d.export_field(f).cpu().numpy()
         assert _bits_equal(x, y), f"{f}: {_diff(x, y)}"
+
+
+@pytest.mark.parametrize("species", [0, 1, 6, 7, 13])
+def test_integrals_by_species_count(get_case, species):
+    """Species are summed in groups of six, cells in blocks of four (162
+    leave the last block half empty): host sums in binary64."""
+    print(f"[gpu] FP64 integrals x1.162, {species} species", flush=True)
+    case = get_case("x1.162-moist", n_scalars=species, moist=species > 0)
+    d = _driver(case)
+    st, a = d.get_state(), d.integrals()
+    wgt = (1.0 / case.inv_area_cell.astype(np.float64))[None, :] * (1.0 / case.grid.rdzw.astype(np.float64))[:, None]
+    rho = st["rho_zz"].astype(np.float64)
+    assert len(a) == 3 + species
+    assert abs(a["dry_mass"] / (wgt * rho).sum() - 1) < 1e-13
+    assert abs(a["rho_theta"] / (wgt * st["rtheta_m"].astype(np.float64)).sum() - 1) < 1e-13
+    for s in range(species):
+        ref = (wgt * rho * st["scalars"][s].astype(np.float64)).sum()
+        assert abs(a[f"tracer_mass_{s}"] - ref) <= 1e-12 * abs(ref) + 1e-300
+
+
+@pytest.mark.parametrize("by_phases", [False, True])
+def test_step_after_a_flagged_one(get_case, by_phases):
+    """A step whose validation flag was set (a negative rho*theta), refused by
+    the whole step or left unpublished by its phases: the next whole step
+    starts from a clear flag and gives the oracle's bits."""
+    print(f"[gpu] x1.162-moist step after a flagged one, by phases {by_phases}", flush=True)
+    case = get_case("x1.162-moist")
+    good = initial_state_arrays(case)
+    o = Oracle(case, 32)
+    o.set_state(good, rebuild=True)
+    assert o.step(2) == 0
+    d = _driver(case)
+    d.step_device(1)
+    bad = dict(good, rtheta_m=-good["rtheta_m"])
+    d.set_state(bad)
+    if by_phases:
+        d.phase("begin_step"); d.phase("begin_subcycle", 1); d.phase("dyn_tend", 1)
+        d.phase("acoustic_substep", 1, 1); d.phase("divergence_damping", 1); d.phase("recover", 1)
+    else:
+        with pytest.raises(Exception, match="validation flag"):
+            d.step_device(1)
+    d.set_state(good)
+    d.step_device(2)
+    ref, got = o.get_state(), d.get_state()
+    for k in ref:
+        assert _bits_equal(ref[k], got[k]), f"{k}: {_diff(ref[k], got[k])}"
