@@ -61,6 +61,9 @@ _K: Dict[str, List[Tuple[str, str]]] = {
                          ("E", "L"), ("E", "L"), ("E", "W")],
     "k_moist_cell": [("SC", "L"), ("C", "L"), ("C", "L")],
     "k_moist_edge": [("SC", "L"), ("E", "L")],
+    # the step's opening pass: k_moist_edge's, k_moist_cell's and k_diag_cv's arrays
+    "k_begin": [("SC", "L"), ("E", "L"), ("C", "L"), ("C", "L"), ("E", "L"), ("C", "L"), ("C", "L"), ("C", "L"),
+                ("V", "L"), ("V", "L")],
     # zz, exner, theta, cqw, qtot, rtheta_p, rb, rtb, exb | cofwz, cofwt, atri, alpha, gamma, coftz
     "k_vcoef": [("C", "L")] * 14 + [("C", "W")],
     # with 2-D Smagorinsky mixing (the default): + u, v | kdiff
