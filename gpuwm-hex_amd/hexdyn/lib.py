@@ -49,6 +49,7 @@ def lib() -> ct.CDLL:
     L.hexdyn_graph_count.argtypes = [vp]
     L.hexdyn_set_state.argtypes = [vp, ct.POINTER(capi.HexdynStateView), ct.c_int, vp]
     L.hexdyn_get_state.argtypes = [vp, ct.POINTER(capi.HexdynStateView), vp]
+    L.hexdyn_download.argtypes = [vp, ct.c_int, ct.POINTER(vp), ct.POINTER(vp), ct.POINTER(ct.c_int64), vp]
     L.hexdyn_export_field.argtypes = [vp, ct.c_int, vp, vp]
     L.hexdyn_import_field.argtypes = [vp, ct.c_int, vp, vp]
     L.hexdyn_field_shape.argtypes = [vp, ct.c_int, ct.POINTER(ct.c_int64), ct.POINTER(ct.c_int64)]
@@ -109,7 +110,7 @@ EXPORTED = [
     "hexdyn_profile_kernels", "hexdyn_powf", "hexdyn_integrals", "hexdyn_set_graphs",
     "hexdyn_set_physics_tendencies", "hexdyn_set_post_transport_clamp", "hexdyn_last_create_error",
     "hexdyn_graph_count", "hexdyn_integrals_noalloc", "hexdyn_copy_state", "hexdyn_set_launch",
-    "hexdyn_get_launch",
+    "hexdyn_get_launch", "hexdyn_download",
     "hexdyn_net_create", "hexdyn_net_destroy", "hexdyn_net_param_count", "hexdyn_net_set_params",
     "hexdyn_net_get_params", "hexdyn_net_get_grads", "hexdyn_net_set_scales", "hexdyn_net_forward",
     "hexdyn_net_set_target", "hexdyn_net_loss", "hexdyn_net_backward", "hexdyn_net_adam", "hexdyn_net_apply",

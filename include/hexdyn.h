@@ -224,6 +224,11 @@ int hexdyn_last_create_error(char *buf, size_t len);
  * pointers are ignored. */
 int hexdyn_set_state(hexdyn_handle *h, const hexdyn_state_view *state, int rebuild, void *stream);
 int hexdyn_get_state(hexdyn_handle *h, const hexdyn_state_view *state, void *stream);
+/* n device arrays to host arrays of count[i] floats, after the work on stream;
+ * the host arrays hold them when the call returns.  Calls on one handle take
+ * turns (they share its pinned staging). */
+int hexdyn_download(hexdyn_handle *h, int n, float *const *host, const float *const *dev, const int64_t *count,
+                    void *stream);
 int hexdyn_export_field(hexdyn_handle *h, int field, float *dst, void *stream);
 int hexdyn_import_field(hexdyn_handle *h, int field, const float *src, void *stream);
 int hexdyn_field_shape(const hexdyn_handle *h, int field, int64_t *rows, int64_t *cols);

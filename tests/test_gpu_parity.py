@@ -824,3 +824,82 @@ def test_step_after_a_flagged_one(get_case, by_phases):
     ref, got = o.get_state(), d.get_state()
     for k in ref:
         assert _bits_equal(ref[k], got[k]), f"{k}: {_diff(ref[k], got[k])}"
+
+
+@pytest.mark.parametrize("counts", [[1], [0, 7, 0, 1029], [1 << 19, (1 << 19) + 1, 3], [2097149, 5, 2097152, 4194311, 1]])
+def test_download_sizes(get_case, counts):
+    """Host copies through the pinned staging: empty and tiny arrays, and
+    arrays that end before, at and after a thread's share (2 MiB) and a half of
+    the staging (8 MiB), into host arrays at odd offsets."""
+    import ctypes as ct
+
+    from hexdyn.lib import lib
+
+    print(f"[gpu] download {counts}", flush=True)
+    d = _driver(get_case("x1.162-moist"))
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    dev = [torch.rand(n, device="cuda", generator=gen) for n in counts]
+    host = [np.full(n + 3, -1.0, dtype=np.float32) for n in counts]
+    n = len(counts)
+    for _ in range(2):  # the second call finds the staging of the first
+        rc = lib().hexdyn_download(
+            d.handle, n, (ct.c_void_p * n)(*(h.ctypes.data + 4 for h in host)),
+            (ct.c_void_p * n)(*(x.data_ptr() for x in dev)), (ct.c_int64 * n)(*counts), ct.c_void_p(d.stream_ptr()))
+        assert rc == 0
+        for h, x, m in zip(host, dev, counts):
+            assert np.array_equal(h[1:1 + m], x.cpu().numpy()) and h[0] == -1.0 and (h[1 + m:] == -1.0).all()
+            h[1:1 + m] = 0.0
+    assert lib().hexdyn_download(d.handle, 1, (ct.c_void_p * 1)(None), (ct.c_void_p * 1)(dev[0].data_ptr()),
+                                 (ct.c_int64 * 1)(1), ct.c_void_p(d.stream_ptr())) != 0
+
+
+@pytest.mark.parametrize("device_checks", [False, True])
+def test_state_arrays_in_any_memory_order(get_case, device_checks, monkeypatch):
+    """Prognostic arrays in C, Fortran, sliced, reversed, read-only and
+    binary64 form upload the same values, and the refusals name the first
+    array that fails, checked on the host or on the device."""
+    import hexdyn.driver as driver
+
+    print(f"[gpu] state upload orders, device checks {device_checks}", flush=True)
+    monkeypatch.setattr(driver, "_CHECK_ON_DEVICE", 1 if device_checks else 1 << 60)
+    case = get_case("x1.162-moist")
+    a = {k: np.ascontiguousarray(v) for k, v in initial_state_arrays(case).items()}
+    d = _driver(case)
+    ref = d.get_state()
+
+    def sliced(x):
+        big = np.zeros(tuple(2 * n for n in x.shape), dtype=x.dtype)
+        big[tuple(slice(None, None, 2) for _ in x.shape)] = x
+        return big[tuple(slice(None, None, 2) for _ in x.shape)]
+
+    def read_only(x):
+        y = np.asfortranarray(x)
+        y.flags.writeable = False
+        return y
+
+    forms = [np.asfortranarray, sliced, lambda x: x[::-1].copy()[::-1], read_only, lambda x: x.astype(np.float64),
+             lambda x: np.moveaxis(np.ascontiguousarray(np.moveaxis(x, 0, -1)), -1, 0)]
+    for f in forms:
+        d.set_state({k: f(v) for k, v in a.items()})
+        got = d.get_state()
+        for k in ref:
+            assert _bits_equal(ref[k], got[k]), k
+    for names, first in ((("ru",), "ru"), (("scalars", "rtheta_m"), "rtheta_m")):
+        for value in (np.nan, np.inf, -np.inf):
+            bad = {k: v.copy() for k, v in a.items()}
+            for k in names:
+                bad[k].reshape(-1)[-1] = value
+            with pytest.raises(FloatingPointError, match=f"^{first} contains"):
+                d.set_state(bad)
+            with pytest.raises(FloatingPointError, match=f"^{first} contains"):  # before a later array's shape
+                d.set_state(dict(bad, rw=a["rw"][:-1]) if first != "ru" else dict(bad, scalars=a["scalars"][:-1]))
+    for value in (0.0, -1.0):
+        bad = dict(a, rho_zz=a["rho_zz"].copy())
+        bad["rho_zz"][3, 5] = value
+        with pytest.raises(ValueError, match="strictly positive"):
+            d.set_state(bad)
+    with pytest.raises(ValueError, match="rw shape"):
+        d.set_state(dict(a, rw=a["rw"][:-1]))
+    got = d.get_state()  # refused states leave the driver's as it was
+    for k in ref:
+        assert _bits_equal(ref[k], got[k]), k
