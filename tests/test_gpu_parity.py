@@ -903,3 +903,26 @@ def test_state_arrays_in_any_memory_order(get_case, device_checks, monkeypatch):
     got = d.get_state()  # refused states leave the driver's as it was
     for k in ref:
         assert _bits_equal(ref[k], got[k]), k
+
+
+@pytest.mark.parametrize("species", [1, 2, 4, 7])
+def test_species_batches_side_by_side_bitwise(get_case, species):
+    """Small meshes run the transport passes with a grid row per batch of
+    species (batches of 2, 3 and 6, the last one partly filled): 2 steps bit
+    for bit, monotonic and not."""
+    import dataclasses
+
+    for mono in (True, False):
+        print(f"[gpu] x1.162, {species} species, monotonic {mono}, 2 steps", flush=True)
+        base = get_case("x1.162-moist", n_scalars=species, moist=True)
+        case = get_case("x1.162-moist", config=dataclasses.replace(base.config, config_monotonic=mono),
+                        n_scalars=species, moist=True)
+        o = Oracle(case, 32)
+        o.set_state(initial_state_arrays(case), rebuild=True)
+        assert o.step(2) == 0
+        d = _driver(case)
+        d.step_device(2)
+        ref, got = o.get_state(), d.get_state()
+        for k in ref:
+            assert _bits_equal(ref[k], got[k]), f"{k}: {_diff(ref[k], got[k])}"
+        d.close()
