@@ -462,7 +462,7 @@ struct CellVertIn {
   SlotRow<NE> sd, dd, kt;
   SlotRow<HX_ROW> rec;
   float ia;
-  int n, code, e[NE], x[NE];
+  int n, code, e[NE], x[NE], v[NE];
 };
 template <int NE>
 __device__ __forceinline__ void cell_vert_index(const Instance &I, int c, CellVertIn<NE> &a) {
@@ -472,6 +472,7 @@ __device__ __forceinline__ void cell_vert_index(const Instance &I, int c, CellVe
   for (int s = 0; s < NE; ++s) {
     a.e[s] = I.m.eoc[c * NE + s];
     a.x[s] = I.m.vx[c * NE + s];
+    a.v[s] = I.m.voc[c * NE + s];
   }
   a.sd = slot_row<NE>(I.m.csdv + c * NE);
   a.dd = slot_row<NE>(I.m.cdcdv + c * NE);
@@ -486,6 +487,7 @@ __device__ __forceinline__ void cell_vert_fence(const CellVertIn<NE> &a) {
   for (int s = 0; s < NE; ++s) {
     fence(a.e[s]);
     fence(a.x[s]);
+    fence(a.v[s]);
   }
 }
 template <int NE>
@@ -537,7 +539,7 @@ __device__ __forceinline__ void cell_vert_finish(const Instance &I, int c, int k
       kc = kc + corr;
       pvc = pvc + (kite * pvv) * a.ia;
       if (a.code >> (16 + s) & 1) {
-        const int v = I.m.voc[c * NE + s];
+        const int v = a.v[s];
         if (k < L) {
           AT(I.b.pv_vertex, v, k) = pvv;
           if (store_mix) AT(I.b.vorticity, v, k) = vort;
@@ -1043,9 +1045,10 @@ KB k_mix_cell(const Instance I) {
   const int L = I.n.L;
   const int n = I.m.neoc[c];
   const int code = LAP ? I.m.vcode[c] : 0;
-  int e[NE], x[NE], o[NE];
+  int e[NE], x[NE], o[NE], vo[NE];
 #pragma unroll
   for (int s = 0; s < NE; ++s) {
+    vo[s] = LAP ? I.m.voc[c * NE + s] : 0;
     e[s] = LAP ? I.m.eoc[c * NE + s] : 0;
     x[s] = LAP ? I.m.vx[c * NE + s] : 0;
     o[s] = I.m.ocell[c * NE + s];
@@ -1060,6 +1063,7 @@ KB k_mix_cell(const Instance I) {
     fence(e[s]);
     fence(x[s]);
     fence(o[s]);
+    fence(vo[s]);
   }
   float tho[NE], rho[NE], wo[NE], kdo[NE], uo[NE], ux[NE];
 #pragma unroll
@@ -1092,8 +1096,7 @@ KB k_mix_cell(const Instance I) {
           float z = 0.0f + rec[r] * u0;
           z = z + rec[r + 1] * u1;
           z = z + rec[r + 2] * u2;
-          const int v = I.m.voc[c * NE + s];
-          if (k < L) AT(I.b.delsq_vort, v, k) = z;
+          if (k < L) AT(I.b.delsq_vort, vo[s], k) = z;
         }
         uq = up;
       }
