@@ -1915,7 +1915,7 @@ __device__ __forceinline__ void rec_column(const Instance &I, const RecIn &r, co
     if (store_rtp) AT(I.b.r_rtheta_p, c, k) = rp;
     if (S3) {
       AT(I.b.r_rho_p, c, k) = dp;
-      AT(I.b.r_rt, c, k) = rtv;
+      if (sub == I.k.splits) AT(I.b.r_rt, c, k) = rtv;  // read where the step publishes it only
       AT(I.b.r_exner, c, k) = ex;
       AT(I.b.r_pp, c, k) = ppv;
     }
