@@ -1240,6 +1240,15 @@ int end_step_publish(hexdyn_handle *h, hipStream_t s) {
   return 0;
 }
 
+// with_w: the whole step left the recovery of w to the first stage
+int transport_stage(hexdyn_handle *h, int stage, int with_w, hipStream_t s) {
+  Work &B = h->I.b;
+  // stage 1 reads the published scalars in place; stages 2-3 read the previous stage's result
+  if (NS_CALL(h, scalars_stage, view(h, false), stage, with_w, s)) return HEXDYN_E_HIP;
+  std::swap(B.q_stage, B.q_next);
+  return 0;
+}
+
 int run_end_step(hexdyn_handle *h, hipStream_t s) {
   if (end_step_device(h, s)) return HEXDYN_E_HIP;
   return end_step_publish(h, s);
@@ -1363,7 +1372,7 @@ int hexdyn_recover(hexdyn_handle *h, int stage, void *stream) {
   // At stage 3 the recovered fluxes are also accumulated into the split-transport
   // sums (copy on the first subcycle, add afterwards: integration.py:27-56).
   Instance J = view(h, true);
-  const int rc = NS_CALL(h, recover, J, stage, h->cur_sub, 0, (hipStream_t)stream);
+  const int rc = NS_CALL(h, recover, J, stage, h->cur_sub, 0, 0, (hipStream_t)stream);
   recovered(h, stage);
   return rc ? HEXDYN_E_HIP : 0;
 }
@@ -1382,12 +1391,7 @@ int hexdyn_end_subcycle(hexdyn_handle *h, int subcycle, void *stream) {
 
 int hexdyn_scalars(hexdyn_handle *h, int stage, void *stream) {
   if (!h || stage < 1 || stage > 3) return HEXDYN_E_INVALID;
-  hipStream_t s = (hipStream_t)stream;
-  Work &B = h->I.b;
-  // stage 1 reads the published scalars in place; stages 2-3 read the previous stage's result
-  if (NS_CALL(h, scalars_stage, view(h, false), stage, s)) return HEXDYN_E_HIP;
-  std::swap(B.q_stage, B.q_next);
-  return 0;
+  return transport_stage(h, stage, 0, (hipStream_t)stream);
 }
 
 int hexdyn_end_step(hexdyn_handle *h, void *stream) {
@@ -1410,6 +1414,8 @@ Instance step_view(const hexdyn_handle *h, bool recovery) {
 // (begin_step's for the first stage of the first subcycle).
 int enqueue_step(hexdyn_handle *h, hipStream_t s) {
   const hexdyn_config &c = h->cfg;
+  const bool transport = c.config_split_dynamics_transport && transported(h);
+  const int w_later = transport && h->I.n.E + h->I.n.C <= HX_RESIDENT ? 1 : 0;  // see k_sc_edge_w
   int rc = run_phase_begin_step(h, s, true);
   for (int sub = 1; rc == 0 && sub <= c.config_dynamics_split_steps; ++sub) {
     h->cur_sub = sub;
@@ -1422,7 +1428,7 @@ int enqueue_step(hexdyn_handle *h, hipStream_t s) {
       const int dd = c.config_divergence_damping ? 1 : 0;
       for (int ss = 1; rc == 0 && ss <= h->I.k.steps[st - 1]; ++ss)
         rc |= NS_CALL(h, acoustic_substep, step_view(h, false), st, ss, sub, (dd && ss > 1) ? 1 : 0, s);
-      rc |= NS_CALL(h, recover, step_view(h, true), st, sub, dd, s);
+      rc |= NS_CALL(h, recover, step_view(h, true), st, sub, dd, w_later, s);
       recovered(h, st);
       // the last stage's diagnostics would only feed a subcycle that does not
       // follow: the next step's begin_step recomputes them from the published state
@@ -1430,8 +1436,7 @@ int enqueue_step(hexdyn_handle *h, hipStream_t s) {
         rc |= NS_CALL(h, solve_diagnostics, step_view(h, false), st, 1, s);
     }
   }
-  if (rc == 0 && c.config_split_dynamics_transport && transported(h))
-    for (int st = 1; rc == 0 && st <= 3; ++st) rc |= hexdyn_scalars(h, st, s);
+  for (int st = 1; rc == 0 && transport && st <= 3; ++st) rc |= transport_stage(h, st, st == 1 ? w_later : 0, s);
   if (rc == 0) rc = end_step_device(h, s);
   return rc;
 }

@@ -37,6 +37,7 @@ struct Sizes {
 // Edge tiles of the staged flux gathers: HX_TILE_E edges per block, at most
 // HX_TILE_U distinct advection cells per tile (larger tiles turn the staged
 // kernels off for the mesh).
+constexpr int HX_RESIDENT = 256 * 32;  // wavefronts the chip holds at once, 32 on each of 256 CUs
 constexpr int HX_VREC = 8;  // values of one vertex in its cell's record (Mesh::vrec)
 constexpr int HX_TILE_E = 8;
 constexpr int HX_TILE_U = 56;
@@ -226,9 +227,9 @@ struct Instance {
   int dyn_tend(const Instance &I, int stage, int sub, hipStream_t s);     \
   int acoustic_substep(const Instance &I, int stage, int ss, int sub, int damp_prev, hipStream_t s); \
   int divergence_damping(const Instance &I, int stage, hipStream_t s);    \
-  int recover(const Instance &I, int stage, int sub, int damp, hipStream_t s); \
+  int recover(const Instance &I, int stage, int sub, int damp, int w_later, hipStream_t s); \
   int solve_diagnostics(const Instance &I, int rk, int with_w, hipStream_t s); \
-  int scalars_stage(const Instance &I, int stage, hipStream_t s);         \
+  int scalars_stage(const Instance &I, int stage, int with_w, hipStream_t s); \
   int rebuild_saved(const Instance &I, hipStream_t s);                    \
   int rebuild_cells(const Instance &I, hipStream_t s);                    \
   int clamp_scalars(const Instance &I, const float *src, float *dst, hipStream_t s); \

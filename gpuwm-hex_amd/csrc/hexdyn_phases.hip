@@ -2284,10 +2284,7 @@ __device__ __forceinline__ float recover_w_column(const Instance &I, int c, int 
 // the same edges: one batch of loads and one launch instead of two (55 us
 // against 34 + 34 at x1.40962).
 template <int NE, bool HDIV, bool DIAG>
-KB k_rec_w(const Instance I, int store_mix) {
-  const int c = wave_entity(I);
-  if (c >= I.n.C) return;
-  const int k = lane();
+__device__ __forceinline__ void rec_w_cell(const Instance &I, int c, int k, int store_mix) {
   const float rho = AT(I.b.c_rho, c, k), rwv = AT(I.b.c_rw, c, k);
   RecWIn<NE> a;
   CellVertIn<NE> d;
@@ -2308,6 +2305,11 @@ KB k_rec_w(const Instance I, int store_mix) {
   if (HDIV && k < I.n.L) AT(I.b.hdiv, c, k) = hd;
   if (k <= I.n.L) AT(I.b.w, c, k) = wv;
   if (DIAG) cell_vert_finish(I, c, k, d, store_mix);
+}
+template <int NE, bool HDIV, bool DIAG>
+KB k_rec_w(const Instance I, int store_mix) {
+  const int c = wave_entity(I);
+  if (c < I.n.C) rec_w_cell<NE, HDIV, DIAG>(I, c, lane(), store_mix);
 }
 
 // The whole cell recovery as a pass of its own (the phase entry points).
@@ -2486,11 +2488,9 @@ __device__ __forceinline__ float vflux(float q0, float q1, float q2, float q3, f
 __device__ __forceinline__ int clamp_sp(int sp, int nt) { return sp < nt ? sp : nt - 1; }
 
 template <int NE>
-KB k_sc_edge(const Instance I, const float *__restrict__ qs, float *__restrict__ ev) {
+__device__ __forceinline__ void sc_edge(const Instance &I, int e, int k, const float *__restrict__ qs,
+                                        float *__restrict__ ev) {
   constexpr int NX = 2 * NE - 2, G = HEXDYN_G_SC_EDGE;
-  const int e = wave_entity(I);
-  if (e >= I.n.E) return;
-  const int k = lane();
   const int NT = I.n.NT;
   int ac[NX];
 #pragma unroll
@@ -2528,6 +2528,27 @@ KB k_sc_edge(const Instance I, const float *__restrict__ qs, float *__restrict__
         if (s < na) r = r + wt[s] * v[g][s];
       if (k < I.n.L) AT(ev, (sp0 + g) * I.n.E + e, k) = r;
     }
+  }
+}
+
+template <int NE>
+KB k_sc_edge(const Instance I, const float *__restrict__ qs, float *__restrict__ ev) {
+  const int e = wave_entity(I);
+  if (e < I.n.E) sc_edge<NE>(I, e, lane(), qs, ev);
+}
+// The transport's first edge pass and the recovery of w that ends the dynamics,
+// neither of which reads what the other writes, in one launch where the
+// wavefronts of both are resident at once: a x1.162 step 288 -> 281 us.  Above,
+// the shared launch is slower than the two (174.5 us against 122.2 + 36.8 at
+// x1.40962, 40.6 against 29.5 + 10.2 at x1.10242).
+template <int NE>
+KB k_sc_edge_w(const Instance I, int nb0, const float *__restrict__ qs, float *__restrict__ ev) {
+  if ((int)blockIdx.x < nb0) {
+    const int e = wave_entity_first(I, nb0);
+    if (e < I.n.E) sc_edge<NE>(I, e, lane(), qs, ev);
+  } else if (blockIdx.y == 0) {
+    const int c = wave_entity_second(I, nb0);
+    if (c < I.n.C) rec_w_cell<NE, false, false>(I, c, lane(), 0);
   }
 }
 
@@ -2945,13 +2966,13 @@ inline void launch_named(const char *name, K kernel, int n, int gy, hipStream_t 
 #define launch(kernel, ...) launch_named(#kernel, kernel, __VA_ARGS__)
 
 // two gather passes in one launch, n0 rows of the first and n1 of the second
-template <typename K>
-inline void launch_pair(const char *name, K kernel, int n0, int n1, hipStream_t s, Instance I) {
+template <typename K, typename... A>
+inline void launch_pair(const char *name, K kernel, int n0, int n1, int gy, hipStream_t s, Instance I, A... args) {
   const int wpb = wpb_from(name, I);
   I.n.WPB = wpb;
   const int nb0 = (nblocks(n0, wpb) + 7) & ~7;
   if (g_prof_on) prof_mark(name, s, 1);
-  hipLaunchKernelGGL(kernel, dim3(nb0 + nblocks(n1, wpb)), dim3(64 * wpb), 0, s, I, nb0);
+  hipLaunchKernelGGL(kernel, dim3(nb0 + nblocks(n1, wpb), gy), dim3(64 * wpb), 0, s, I, nb0, args...);
   if (g_prof_on) prof_mark(name, s, 0);
 }
 
@@ -3045,7 +3066,7 @@ int solve_diagnostics(const Instance &I, int rk, int with_w, hipStream_t s) {
 
 int begin_step(const Instance &I, hipStream_t s) {
   if (I.n.NM > 0) {
-#define BEGIN(NE, DI) launch_pair("k_begin", k_begin<NE, DI>, I.n.E, I.n.C, s, I)
+#define BEGIN(NE, DI) launch_pair("k_begin", k_begin<NE, DI>, I.n.E, I.n.C, 1, s, I)
     NEDISPATCH(I, I.n.VP ? BEGIN(6, true) : BEGIN(6, false), I.n.VP ? BEGIN(7, true) : BEGIN(7, false));
 #undef BEGIN
   }
@@ -3088,8 +3109,8 @@ int begin_subcycle(const Instance &I, int sub, hipStream_t s) {
 #undef MIX_NE
 #undef MIX
     if (mix4)
-      NEDISPATCH(I, launch_pair("k_mix4", k_mix4<6>, I.n.E, I.n.C, s, I),
-                 launch_pair("k_mix4", k_mix4<7>, I.n.E, I.n.C, s, I));
+      NEDISPATCH(I, launch_pair("k_mix4", k_mix4<6>, I.n.E, I.n.C, 1, s, I),
+                 launch_pair("k_mix4", k_mix4<7>, I.n.E, I.n.C, 1, s, I));
   }
   return check();
 }
@@ -3223,7 +3244,8 @@ void recover_edges(const Instance &I, int sub, float inv, bool damp, bool avgrp,
 #undef REC
 }
 
-int recover(const Instance &I, int stage, int sub, int damp, hipStream_t s) {
+// w_later: the transport's first pass recovers the last stage's w
+int recover(const Instance &I, int stage, int sub, int damp, int w_later, hipStream_t s) {
   const bool last = stage == 3 && sub == I.k.splits;
   const float inv = I.k.inv_steps[stage - 1];
   const bool avgrp = I.k.fused && I.k.steps[stage - 1] == 1;
@@ -3235,7 +3257,7 @@ int recover(const Instance &I, int stage, int sub, int damp, hipStream_t s) {
   if (I.k.fused) {
     // the column pass recovered the rest; w and hdiv come with the diagnostics
     // that follow, except after a step's last stage, which has none
-    if (last)
+    if (last && !w_later)
       NEDISPATCH(I, launch_named("k_rec_w", k_rec_w<6, false, false>, I.n.C, 1, s, I, 0),
                  launch_named("k_rec_w", k_rec_w<7, false, false>, I.n.C, 1, s, I, 0));
   } else if (stage == 3) {
@@ -3255,17 +3277,21 @@ int recover(const Instance &I, int stage, int sub, int damp, hipStream_t s) {
 // x1.642, 470 -> 465 at x1.2562.  Above, the batches fill the chip as well one
 // after the other and share the species-independent rows: 1177 us at x1.10242,
 // 1183 with a row a batch.
-constexpr int kResident = 256 * 32;
 inline int species_rows(const Instance &I, int n, int g) {
   const int batches = (I.n.NT + g - 1) / g;
-  return (long long)n * batches <= kResident ? batches : 1;
+  return (long long)n * batches <= HX_RESIDENT ? batches : 1;
 }
 
-int scalars_stage(const Instance &I, int stage, hipStream_t s) {
+int scalars_stage(const Instance &I, int stage, int with_w, hipStream_t s) {
   const float dt = I.k.sca_dt[stage - 1];
   const float *qin = stage == 1 ? I.b.q : I.b.q_stage;  // stage 1 starts from the published scalars
   if (stage < 3 || !I.k.monotonic) {
-    LAUNCH_NE(I, k_sc_edge, I.n.E, species_rows(I, I.n.E, HEXDYN_G_SC_EDGE), s, I, qin, I.b.ev);
+    const int rows = species_rows(I, I.n.E, HEXDYN_G_SC_EDGE);
+    if (with_w)
+      NEDISPATCH(I, launch_pair("k_sc_edge_w", k_sc_edge_w<6>, I.n.E, I.n.C, rows, s, I, qin, I.b.ev),
+                 launch_pair("k_sc_edge_w", k_sc_edge_w<7>, I.n.E, I.n.C, rows, s, I, qin, I.b.ev));
+    else
+      LAUNCH_NE(I, k_sc_edge, I.n.E, rows, s, I, qin, I.b.ev);
     LAUNCH_NE(I, k_sc_cell, I.n.C, species_rows(I, I.n.C, HEXDYN_G_SC_CELL), s, I, qin, (const float *)I.b.ev,
               I.b.q_next, dt,
               I.k.wn[stage - 1], (const float *)(I.k.physics_q ? I.b.phys_q : nullptr));

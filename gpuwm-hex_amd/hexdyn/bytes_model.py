@@ -113,6 +113,9 @@ _K: Dict[str, List[Tuple[str, str]]] = {
     # the whole-step form after one damped substep: s_ru, tend_ru, rho, rtheta_pp, s_theta | c_ru, u
     "k_rec_edge": [("E", "L")] * 2 + [("C", "L")] * 3 + [("E", "L")] * 2,
     "k_sc_edge": [("SC", "L"), ("E", "L"), ("SE", "L")],
+    # k_sc_edge's arrays, then rho, rw, ru, zz, zb, zb3 | w
+    "k_sc_edge_w": [("SC", "L"), ("E", "L"), ("SE", "L"), ("C", "L"), ("C", "W"), ("E", "L"), ("C", "L"),
+                    ("CM", "W"), ("CM", "W"), ("C", "W")],
     "k_sc_cell": [("SC", "L"), ("C", "W"), ("E", "L"), ("SE", "L"), ("C", "L"), ("C", "L"), ("SC", "L"),
                   ("SC", "L")],
     # qs, qold, split_u | hres
