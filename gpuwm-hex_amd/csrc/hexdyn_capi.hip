@@ -762,6 +762,7 @@ static int create_impl(const hexdyn_mesh *m, const hexdyn_vertical *vt, const he
   rc |= h->upload(&M.vdc, vdc); rc |= h->upload(&M.vdcdv, vdcdv);
   rc |= h->upload(&M.ecos, ecos); rc |= h->upload(&M.esin, esin); rc |= h->upload(&M.ocell, ocell);
   n.OCP = ocp;
+  h->tune.large = n.E > 4 * HX_RESIDENT;
   if (mixing) {
     // binary32 scalars staged as the reference host does (cuda_horizontal_v841.py:1336-1350)
     const float len = c->config_len_disp, csm = c->config_smagorinsky_coef;
@@ -1558,8 +1559,8 @@ void drop_graphs(hexdyn_handle *h) {
   for (auto &kv : h->graphs) (void)hipGraphExecDestroy(kv.second.first);
   h->graphs.clear();
 }
-// kernels with a fixed block shape: the column kernels (16 or 8 columns per
-// block through LDS) and the edge-tiled flux pass (HX_TILE_E edges per block)
+// kernels with a fixed block shape: the column kernels (16 or 4 columns per
+// block) and the edge-tiled flux pass (HX_TILE_E edges per block)
 bool column_kernel(const char *name) {
   return std::strcmp(name, "k_vcoef") == 0 || std::strcmp(name, "k_ac_cell") == 0 ||
          std::strcmp(name, "k_col") == 0 || std::strcmp(name, "k_diag_edge_flux_t") == 0;

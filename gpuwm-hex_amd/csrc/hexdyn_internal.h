@@ -195,7 +195,8 @@ extern int g_prof_on;
 struct LaunchTune {
   static constexpr int kMax = 64;
   int n = 0;
-  int def = 4;  // kernels not listed
+  int def = 0;  // kernels not listed; 0: default_wpb
+  bool large = false;  // a mesh of more edges than four times the wavefronts the chip holds
   char names[kMax][32];
   int wpb[kMax];
   int find(const char *name) const {
@@ -205,7 +206,20 @@ struct LaunchTune {
   }
   int waves_per_block(const char *name) const {
     const int i = find(name);
-    return i < 0 ? def : wpb[i];
+    return i >= 0 ? wpb[i] : def ? def : default_wpb(name);
+  }
+  // On large meshes the edge passes whose gathers gain from more of a
+  // neighbourhood in one block: k_tend_mom_ac 66.1 us at 4 wavefronts a block and
+  // 62.7 at 8 (x1.40962), k_sc_edge 122.7 and 119.0, k_rec_edge 48.2 and 47.4; a
+  // step 5101 -> 5053 us, x1.163842 18.30 -> 18.20 ms, 8 x x1.2562 2492 -> 2469 us.
+  // The others lose or are even (k_fct_edge1 158 and 171, k_sub_edge 59.2 and
+  // 61.2), as do all on meshes that fit the chip a few times over (x1.2562 403
+  // and 408 us a step, x1.10242 the same).
+  int default_wpb(const char *name) const {
+    if (large)
+      for (const char *k : {"k_tend_mom_ac", "k_sc_edge", "k_rec_edge"})
+        if (std::strcmp(name, k) == 0) return 8;
+    return 4;
   }
 };
 

@@ -109,7 +109,7 @@ def tune(drv, steps: int = 2, check_steps: int = 10) -> dict:
     apply(drv, table)
     tuned_ms = _step_ms(drv, check_steps)
     if tuned_ms > default_ms:
-        # the whole step decides: keep the default when the per-kernel picks lose
+        # the whole step decides: 4 everywhere when the per-kernel picks lose
         table = {}
         apply(drv, table)
     return {"table": table, "per_kernel_ms": per_kernel, "default_ms_per_step": round(default_ms, 4),

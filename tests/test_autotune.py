@@ -76,3 +76,26 @@ def test_tuner_is_not_slower_and_keeps_bits(get_case, tmp_path, monkeypatch):
     d2.close()
     for k in want:
         assert _bits(got[k], want[k]), k
+
+
+@pytest.mark.parametrize("name,waves", [("x1.2562-moist", 4), ("x1.10242-moist", 4), ("x1.40962-dry", 8)])
+def test_default_launch_shapes(get_case, name, waves):
+    """Three edge passes take larger blocks from 32 768 edges on; a reset sets
+    every kernel alike, and the bits stay."""
+    from hexdyn import autotune
+    from hexdyn.driver import HexDycoreDriver
+
+    print(f"[gpu] default launch shapes {name}", flush=True)
+    runs = []
+    for reset in (None, 4):
+        d = HexDycoreDriver.from_host(get_case(name))
+        if reset:
+            autotune.set_launch(d, "*", reset)
+        for k in ("k_tend_mom_ac", "k_sc_edge", "k_rec_edge"):
+            assert autotune.get_launch(d, k) == (reset or waves)
+        assert autotune.get_launch(d, "k_sub_edge") == 4
+        d.step_device(1)
+        runs.append(d.get_state())
+        d.close()
+    for k in runs[0]:
+        assert _bits(runs[0][k], runs[1][k]), k
