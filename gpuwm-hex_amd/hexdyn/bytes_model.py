@@ -59,9 +59,7 @@ _K: Dict[str, List[Tuple[str, str]]] = {
     "k_diag_edge_flux": [("E", "L"), ("V", "L"), ("C", "L"), ("E", "L"), ("E", "L"),
                          ("E", "L"), ("C", "L"), ("C", "W"), ("E", "L"), ("C", "L"),
                          ("E", "L"), ("E", "L"), ("E", "W")],
-    "k_moist_cell": [("SC", "L"), ("C", "L"), ("C", "L")],
-    "k_moist_edge": [("SC", "L"), ("E", "L")],
-    # the step's opening pass: k_moist_edge's, k_moist_cell's and k_diag_cv's arrays
+    # a step's opening pass: q | cqu, qtot, cqw, then k_diag_cv's arrays
     "k_begin": [("SC", "L"), ("E", "L"), ("C", "L"), ("C", "L"), ("E", "L"), ("C", "L"), ("C", "L"), ("C", "L"),
                 ("V", "L"), ("V", "L")],
     # zz, exner, theta, cqw, qtot, rtheta_p, rb, rtb, exb | cofwz, cofwt, atri, alpha, gamma, coftz
@@ -123,22 +121,18 @@ _K: Dict[str, List[Tuple[str, str]]] = {
     # qs, qold, rho, split_w, split_u, hres | target, mass, sin, sout, vres
     "k_fct_cell1": [("SC", "L"), ("SC", "L"), ("C", "L"), ("C", "W"), ("E", "L"), ("SE", "L"), ("C", "L"),
                     ("SC", "L"), ("SC", "L"), ("SC", "L"), ("SC", "W")],
-    "k_fct_edge2": [("SC", "L"), ("SC", "L"), ("SE", "L"), ("SE", "L")],
     # hres, sin, sout, vres, mass, target | q
     "k_fct_cell2": [("SE", "L"), ("SC", "L"), ("SC", "L"), ("SC", "W"), ("SC", "L"), ("C", "L"), ("SC", "L")],
     # horizontal mixing, once per subcycle
     "k_mix_lapdiv": [("E", "L"), ("C", "L")],
     "k_mix_lapvort": [("E", "L"), ("V", "L")],
-    # delsq_div, delsq_vort, c_rho, euler_ru | euler_ru
-    "k_mix_edge4": [("C", "L"), ("V", "L"), ("C", "L"), ("E", "L"), ("E", "L")],
     # theta, c_rho, w, kdiff, delsq_u | delsq_theta, euler_theta, delsq_w, tend_w, delsq_div, delsq_vort
     "k_mix_cell": [("C", "L"), ("C", "L"), ("C", "W"), ("C", "L"), ("E", "L"), ("C", "L"), ("C", "L"), ("C", "L"),
                    ("C", "W"), ("C", "L"), ("V", "L")],
-    # k_mix_edge4's and k_mix_cell4's arrays
+    # edges: delsq_div, delsq_vort, c_rho, euler_ru | euler_ru; cells: delsq_theta, delsq_w,
+    # euler_theta, tend_w, euler_rw | euler_theta, euler_rw
     "k_mix4": [("C", "L"), ("V", "L"), ("C", "L"), ("E", "L"), ("E", "L"), ("C", "L"), ("C", "L"), ("C", "L"),
                ("C", "W"), ("C", "W"), ("C", "L"), ("C", "W")],
-    # delsq_theta, delsq_w, euler_theta, tend_w, euler_rw | euler_theta, euler_rw
-    "k_mix_cell4": [("C", "L"), ("C", "L"), ("C", "L"), ("C", "W"), ("C", "W"), ("C", "L"), ("C", "W")],
 }
 # state rebuild (after a state is set): rho, rtheta_m, zz, rtb, rb, exb, rw, ru, zb, zb3 |
 # theta, exner, rho_p, rtheta_p, p', w

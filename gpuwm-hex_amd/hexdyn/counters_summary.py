@@ -37,7 +37,7 @@ def main() -> None:
         return sum(v) / len(v) if v else float("nan")
 
     lines = [f"# Memory-pipeline counters of the gather kernels, {a.workload} (plain step, strict numerics)", "",
-             "Commands (repository root on the GPU box, TMPDIR=/tmp), one pass each:", ""]
+             "Commands (repository root on an MI355X machine, TMPDIR=/tmp), one pass each:", ""]
     lines += ["    " + c for c in a.command]
     lines += ["", f"Per launch (mean over launches; per-CU figures divide block counters by {CUS} CUs).", "",
               "| kernel | waves | vmem rd / wave | vmem wr / wave | L2 hit % | L1 accesses / vmem instr | "

@@ -89,7 +89,7 @@ def main() -> None:
         m[1] += float(r["TotalDurationNs"])
     total = sum(v[1] for v in merged.values())
     lines = [f"# Per-kernel time and HBM traffic, {a.workload}", "",
-             "Commands (repository root on the GPU box, TMPDIR=/tmp):", ""]
+             "Commands (repository root on an MI355X machine, TMPDIR=/tmp):", ""]
     lines += [f"    {c}" for c in a.command]
     lines += ["", f"Large steps in the kernel-trace run: {a.steps:g}.",
               f"Counter calibration: FETCH_SIZE x {ff:.3f} and WRITE_SIZE x {fw:.3f} give bytes "
