@@ -283,7 +283,7 @@ __device__ __forceinline__ float thomas_sweeps(float x, float d, float l, float 
 #pragma unroll
     for (int u = 0; u < 8; ++u) p = (x - d * up0(p)) * l;
   }
-  x = p;
+  p = x = inner ? p : x;  // level L's 0 * (a value that is not finite) stays out
   for (int i = 0; i < L; i += 8) {
 #pragma unroll
     for (int u = 0; u < 8; ++u) p = x - g * dn0(p);
@@ -320,7 +320,7 @@ __device__ __forceinline__ int coef_sweep(float &a, float &b, float c, int k, in
     singular = den == 0.0f ? 1 : 0;
   }
   a = inner ? al : 0.0f;
-  b = gm;
+  b = inner ? gm : 0.0f;
   return singular;
 }
 

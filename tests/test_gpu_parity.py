@@ -926,3 +926,30 @@ def test_species_batches_side_by_side_bitwise(get_case, species):
         for k in ref:
             assert _bits_equal(ref[k], got[k]), f"{k}: {_diff(ref[k], got[k])}"
         d.close()
+
+
+@pytest.mark.parametrize("field,scale", [("exner", 1e37), ("exner", np.inf), ("w", np.inf), ("w", np.nan)])
+def test_columns_that_are_not_finite(get_case, field, scale):
+    """Every third column with a field scaled out of range at its upper half:
+    the recurrences carry infinities and NaN to the levels the serial sweeps
+    carry them to, and to no other column's (phases of a first stage, values
+    equal with NaN where NaN is)."""
+    print(f"[gpu] x1.162-moist, {field} x {scale} in every third column", flush=True)
+    case = get_case("x1.162-moist")
+    o = Oracle(case, 32)
+    o.set_state(initial_state_arrays(case), rebuild=True)
+    a = o.get_state()
+    a[field][30:, ::3] = (a[field][30:, ::3] + np.float32(1e-3)) * np.float32(scale)
+    o.set_state(a, rebuild=False)
+    d = _driver(case)
+    d.set_state(a, saved=a)
+    o.begin_step(); d.phase("begin_step")
+    o.begin_subcycle(1); d.phase("begin_subcycle", 1)
+    o.dyn_tend(1); d.phase("dyn_tend", 1)
+    o.acoustic_substep(1, 1); d.phase("acoustic_substep", 1, 1)
+    seen = False
+    for f in ("ALPHA_TRI", "GAMMA_TRI", "RW_P", "WW_AVG", "RHO_PP", "RTHETA_PP"):
+        x, y = o.export_field(f), d.export_field(f).cpu().numpy().ravel()
+        seen |= not np.isfinite(x).all()
+        assert np.array_equal(x, y, equal_nan=True), f"{f}: {np.sum(~((x == y) | (np.isnan(x) & np.isnan(y))))} differ"
+    assert seen or scale == 1e37
