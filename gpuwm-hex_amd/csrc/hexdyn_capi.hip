@@ -247,7 +247,7 @@ struct hexdyn_handle {
   double *int_partial = nullptr;                              // integral partials
   double *int_host = nullptr;                                 // integrals, in host memory the device writes
   int *flag_host = nullptr;                                   // a closed step's validation flag, likewise
-  int flag_open = 0;                                          // a step may have set the device's flag since
+  int flag_open = 0;                                          // the device's flag may be set
   // pinned staging of hexdyn_download, made on its first call
   std::mutex stage_mutex;
   char *stage = nullptr;
@@ -1157,22 +1157,18 @@ __global__ void k_clear_flag(int *flag) {
   if (threadIdx.x == 0) flag[0] = 0;
 }
 
-// hands the validation flag to the host word and leaves it clear for the next
-// step.  A step waits for this store and no copy: reading the flag with a copy
-// into pageable memory is a launch of its own behind the step, and the copy's
-// staging runs after the device has finished (an x1.162 step 319 -> 309 us, its
-// integrals 38.7 -> 22; x1.10242 1337 -> 1324).
-__global__ void k_publish_flag(int *flag, int *host) {
-  if (threadIdx.x == 0) {
-    const int v = flag[0];
-    flag[0] = 0;
-    __hip_atomic_store(host, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  }
+// hands the validation flag to the host word.  A step waits for this store and
+// no copy: reading the flag with a copy into pageable memory is a launch of its
+// own behind the step, and the copy's staging runs after the device has finished
+// (an x1.162 step 319 -> 309 us, its integrals 38.7 -> 22; x1.10242 1337 -> 1324).
+// The device's flag stays as it is: the end of a refused step asked for again is
+// refused again.
+__global__ void k_publish_flag(const int *flag, int *host) {
+  if (threadIdx.x == 0) __hip_atomic_store(host, flag[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// the phase entry points clear the flag at their start; a whole step starts
-// from the flag as the last published step left it (hexdyn_step clears it
-// where a step was left unpublished)
+// a step by phases clears the flag at its start, a whole step where the flag may
+// have been set since a step was last published (flag_open)
 int clear_flag(hexdyn_handle *h, hipStream_t s) {
   hipLaunchKernelGGL(k_clear_flag, dim3(1), dim3(64), 0, s, h->I.b.flag);
   return hipGetLastError() == hipSuccess ? 0 : HEXDYN_E_HIP;
@@ -1214,7 +1210,7 @@ int end_step_device(hexdyn_handle *h, hipStream_t s) {
       return HEXDYN_E_HIP;
     }
   }
-  hipLaunchKernelGGL(k_publish_flag, dim3(1), dim3(64), 0, s, h->I.b.flag, h->flag_host);
+  hipLaunchKernelGGL(k_publish_flag, dim3(1), dim3(64), 0, s, (const int *)h->I.b.flag, h->flag_host);
   return hipGetLastError() == hipSuccess ? 0 : HEXDYN_E_HIP;
 }
 
@@ -1226,7 +1222,7 @@ int end_step_publish(hexdyn_handle *h, hipStream_t s) {
   Work &B = h->I.b;
   if (hipStreamSynchronize(s) != hipSuccess) return HEXDYN_E_HIP;
   const int flag = *(volatile int *)h->flag_host;
-  h->flag_open = 0;
+  h->flag_open = flag;
   h->in_step = 0;
   h->start_is_pub = h->fresh_sub = h->fresh_step = h->exner_start = h->pp_pub = 0;
   if (flag) {

@@ -953,3 +953,44 @@ def test_columns_that_are_not_finite(get_case, field, scale):
         seen |= not np.isfinite(x).all()
         assert np.array_equal(x, y, equal_nan=True), f"{f}: {np.sum(~((x == y) | (np.isnan(x) & np.isnan(y))))} differ"
     assert seen or scale == 1e37
+
+
+def _refused_by_phases(d):
+    """A step by phases up to its first recovery, then its end, which refuses it."""
+    d.phase("begin_step"); d.phase("begin_subcycle", 1); d.phase("dyn_tend", 1)
+    d.phase("acoustic_substep", 1, 1); d.phase("divergence_damping", 1); d.phase("recover", 1)
+    with pytest.raises(FloatingPointError, match="validation flag"):
+        d.phase("end_step")
+
+
+@pytest.mark.parametrize("by_phases", [False, True])
+def test_a_refused_step_stays_refused(get_case, by_phases):
+    """The end of a step asked for again after it was refused is refused again
+    and publishes nothing, whether the whole step or its phases were refused;
+    the next step is judged by its own flag."""
+    print(f"[gpu] x1.162-moist end of a refused step, by phases {by_phases}", flush=True)
+    case = get_case("x1.162-moist")
+    good = initial_state_arrays(case)
+    o = Oracle(case, 32)
+    o.set_state(good, rebuild=True)
+    assert o.step(1) == 0
+    d = _driver(case)
+    d.set_state(dict(good, rtheta_m=-good["rtheta_m"]))
+    before, t = d.get_state(), d.model_time()
+    if by_phases:
+        _refused_by_phases(d)
+    else:
+        with pytest.raises(FloatingPointError, match="validation flag"):
+            d.step_device(1)
+    for _ in range(2):
+        with pytest.raises(FloatingPointError, match="validation flag"):
+            d.phase("end_step")
+    assert d.model_time() == t
+    got = d.get_state()
+    for k in before:
+        assert _bits_equal(before[k], got[k]), k
+    d.set_state(good)
+    d.step_device(1)
+    ref, got = o.get_state(), d.get_state()
+    for k in ref:
+        assert _bits_equal(ref[k], got[k]), f"{k}: {_diff(ref[k], got[k])}"
