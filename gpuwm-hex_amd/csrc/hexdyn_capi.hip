@@ -1168,7 +1168,8 @@ __global__ void k_publish_flag(const int *flag, int *host) {
 }
 
 // a step by phases clears the flag at its start, a whole step where the flag may
-// have been set since a step was last published (flag_open)
+// have been set since a step was last published (flag_open: by the step's own
+// passes or by a phase, which may be called outside a step too)
 int clear_flag(hexdyn_handle *h, hipStream_t s) {
   hipLaunchKernelGGL(k_clear_flag, dim3(1), dim3(64), 0, s, h->I.b.flag);
   return hipGetLastError() == hipSuccess ? 0 : HEXDYN_E_HIP;
@@ -1349,11 +1350,13 @@ int hexdyn_begin_subcycle(hexdyn_handle *h, int subcycle, void *stream) {
 
 int hexdyn_dyn_tend(hexdyn_handle *h, int stage, void *stream) {
   if (!h || stage < 1 || stage > 3) return HEXDYN_E_INVALID;
+  h->flag_open = 1;
   return NS_CALL(h, dyn_tend, view(h, false), stage, h->cur_sub, (hipStream_t)stream) ? HEXDYN_E_HIP : 0;
 }
 
 int hexdyn_acoustic_substep(hexdyn_handle *h, int stage, int small_step, void *stream) {
   if (!h || stage < 1 || stage > 3 || small_step < 1 || small_step > h->I.k.steps[stage - 1]) return HEXDYN_E_INVALID;
+  h->flag_open = 1;
   return NS_CALL(h, acoustic_substep, view(h, false), stage, small_step, h->cur_sub, 0, (hipStream_t)stream)
              ? HEXDYN_E_HIP
              : 0;
@@ -1368,6 +1371,7 @@ int hexdyn_recover(hexdyn_handle *h, int stage, void *stream) {
   if (!h || stage < 1 || stage > 3) return HEXDYN_E_INVALID;
   // At stage 3 the recovered fluxes are also accumulated into the split-transport
   // sums (copy on the first subcycle, add afterwards: integration.py:27-56).
+  h->flag_open = 1;
   Instance J = view(h, true);
   const int rc = NS_CALL(h, recover, J, stage, h->cur_sub, 0, 0, (hipStream_t)stream);
   recovered(h, stage);
@@ -1388,6 +1392,7 @@ int hexdyn_end_subcycle(hexdyn_handle *h, int subcycle, void *stream) {
 
 int hexdyn_scalars(hexdyn_handle *h, int stage, void *stream) {
   if (!h || stage < 1 || stage > 3) return HEXDYN_E_INVALID;
+  h->flag_open = 1;
   return transport_stage(h, stage, 0, (hipStream_t)stream);
 }
 

@@ -994,3 +994,39 @@ def test_a_refused_step_stays_refused(get_case, by_phases):
     ref, got = o.get_state(), d.get_state()
     for k in ref:
         assert _bits_equal(ref[k], got[k]), f"{k}: {_diff(ref[k], got[k])}"
+
+
+@pytest.mark.parametrize("call", ["recover", "scalars"])
+def test_step_after_a_phase_outside_a_step(get_case, call):
+    """A phase called outside a step on fields that set the validation flag: the
+    next whole step is judged by its own flag and gives the oracle's bits."""
+    import ctypes as ct
+
+    from hexdyn import capi
+    from hexdyn.lib import lib
+
+    print(f"[gpu] x1.162-moist, {call} outside a step, then a step", flush=True)
+    case = get_case("x1.162-moist")
+    good = initial_state_arrays(case)
+    o = Oracle(case, 32)
+    o.set_state(good, rebuild=True)
+    assert o.step(1) == 0
+    name, args = ("RHO_PP", (1,)) if call == "recover" else ("RHO_ZZ", (3,))
+
+    def called_outside():
+        d = _driver(case)
+        d.step_device(1)
+        t = torch.full_like(d.export_field(name), -1e6)
+        assert lib().hexdyn_import_field(d.handle, capi.FIELD_ID[name], ct.c_void_p(t.data_ptr()),
+                                         ct.c_void_p(d.stream_ptr())) == 0
+        d.phase(call, *args)
+        return d
+
+    with pytest.raises(FloatingPointError, match="validation flag"):  # the flag is set
+        called_outside().phase("end_step")
+    d = called_outside()
+    d.set_state(good)
+    d.step_device(1)
+    ref, got = o.get_state(), d.get_state()
+    for k in ref:
+        assert _bits_equal(ref[k], got[k]), f"{k}: {_diff(ref[k], got[k])}"
