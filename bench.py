@@ -430,7 +430,7 @@ def main():
                    "horiz_mixing": args.mixing,
                    "dynamics_split_steps": cfg.config_dynamics_split_steps,
                    "number_of_sub_steps": cfg.config_number_of_sub_steps, "parallelism": "single-gpu",
-                   "launch_tuning": {"waves_per_block": tuning["table"], "default": 4,
+                   "launch_tuning": {"waves_per_block": tuning["table"], "default": tuning.get("default"),
                                      "default_ms_per_step": tuning["default_ms_per_step"],
                                      "tuned_ms_per_step": tuning["tuned_ms_per_step"]}},
         "roofline": roofline,

@@ -1571,11 +1571,12 @@ bool column_kernel(const char *name) {
 int hexdyn_set_launch(hexdyn_handle *h, const char *kernel, int waves_per_block) {
   if (!h || !kernel) return HEXDYN_E_INVALID;
   if (h->in_step) return set_error(h, HEXDYN_E_INVALID, "hexdyn_set_launch inside a step");
+  const bool all = std::strcmp(kernel, "*") == 0;
   if (waves_per_block != 1 && waves_per_block != 2 && waves_per_block != 4 && waves_per_block != 8 &&
-      waves_per_block != 16)
-    return set_error(h, HEXDYN_E_INVALID, "waves_per_block must be 1, 2, 4, 8 or 16");
+      waves_per_block != 16 && !(all && waves_per_block == 0))
+    return set_error(h, HEXDYN_E_INVALID, "waves_per_block must be 1, 2, 4, 8 or 16 (0: \"*\" only)");
   LaunchTune &t = h->tune;
-  if (std::strcmp(kernel, "*") == 0) {
+  if (all) {
     t.n = 0;
     t.def = waves_per_block;
   } else {

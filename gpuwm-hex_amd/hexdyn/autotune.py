@@ -9,10 +9,11 @@ scheduling unit covers (the rows of one block share the CU's L1, and
 consecutive rows on the curve share most of their neighbour rows), and how
 many blocks a CU holds.  The tuner times
 every gather kernel at each tile with HIP events over profiled large steps
-of the handle's own mesh, keeps each kernel's fastest tile, checks that the
-whole step with the chosen tiles is not slower than with the default (4),
-and stores the choice in a JSON file keyed by device, mesh size, levels,
-scalars, mixing and numerics; ``apply_saved`` installs it after ``hexdyn_create``.
+of the handle's own mesh, keeps each kernel's fastest tile where it is not the
+one that an untuned handle of the mesh takes, checks that the whole step with
+the chosen tiles is not slower than the untuned one (and keeps no tile where it
+is), and stores the choice in a JSON file keyed by mesh size, levels, scalars,
+mixing and numerics; ``apply_saved`` installs it after ``hexdyn_create``.
 (The reference tunes the level chunking of its hoisted edge kernels by
 longest-processing-time packing, cuda_edge_hoist.py:63-101.)
 """
@@ -58,7 +59,8 @@ def get_launch(drv, kernel: str) -> int:
 
 
 def apply(drv, table: Dict[str, int]) -> None:
-    set_launch(drv, "*", 4)
+    """The tiles of a table; kernels that it does not list take their defaults."""
+    set_launch(drv, "*", 0)
     for k, w in table.items():
         set_launch(drv, k, w)
 
@@ -90,29 +92,31 @@ def _step_ms(drv, steps: int) -> float:
 
 def tune(drv, steps: int = 2, check_steps: int = 10) -> dict:
     """Pick each gather kernel's wavefronts per block by timing; install and
-    return {"table", "per_kernel_ms", "default_ms_per_step", "tuned_ms_per_step"}."""
+    return {"table", "default", "per_kernel_ms", "default_ms_per_step",
+    "tuned_ms_per_step"}."""
     times = {}
     for w in CANDIDATES:
         set_launch(drv, "*", w)
         _kernel_times(drv, 1)  # warm (graphs are off while profiling; first launches compile nothing)
         times[w] = _kernel_times(drv, steps)
     names = sorted(set().union(*[set(t) for t in times.values()]) - COLUMN_KERNELS)
+    apply(drv, {})
+    default = {n: get_launch(drv, n) for n in names}
     table = {}
     per_kernel = {}
     for n in names:
         best = min(CANDIDATES, key=lambda w: times[w].get(n, float("inf")))
         per_kernel[n] = {str(w): round(times[w].get(n, float("nan")), 5) for w in CANDIDATES}
-        if best != 4:
+        if best != default[n]:
             table[n] = best
-    apply(drv, {})
     default_ms = _step_ms(drv, check_steps)
     apply(drv, table)
     tuned_ms = _step_ms(drv, check_steps)
     if tuned_ms > default_ms:
-        # the whole step decides: 4 everywhere when the per-kernel picks lose
+        # the whole step decides: the defaults when the per-kernel picks lose
         table = {}
         apply(drv, table)
-    return {"table": table, "per_kernel_ms": per_kernel, "default_ms_per_step": round(default_ms, 4),
+    return {"table": table, "default": default, "per_kernel_ms": per_kernel, "default_ms_per_step": round(default_ms, 4),
             "tuned_ms_per_step": round(tuned_ms, 4), "candidates": list(CANDIDATES), "key": tuning_key(drv)}
 
 

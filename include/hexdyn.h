@@ -250,7 +250,8 @@ int hexdyn_graph_count(const hexdyn_handle *h);
 /* Launch shape of the gather kernels (one wavefront per cell, edge or
  * vertex row): wavefronts per block, 1, 2, 4 (the default; on meshes of more than
  * 32768 edges 8 for k_tend_mom_ac, k_sc_edge and k_rec_edge), 8 or 16, by kernel name
- * ("k_diag_edge_flux", ...; "*" resets every kernel to the given value).
+ * ("k_diag_edge_flux", ...; "*" resets every kernel to the given value, and with 0
+ * to its default).
  * The column kernels (k_vcoef, 16 columns per block; k_ac_cell and k_col, 4)
  * and the edge-tiled flux pass (k_diag_edge_flux_t: 8 edges per block
  * through LDS) are refused; setting k_diag_edge_flux selects that pass's

@@ -99,3 +99,46 @@ def test_default_launch_shapes(get_case, name, waves):
         d.close()
     for k in runs[0]:
         assert _bits(runs[0][k], runs[1][k]), k
+
+
+@pytest.mark.parametrize("name,waves", [("x1.10242-moist", 4), ("x1.40962-dry", 8)])
+@pytest.mark.parametrize("picks_win", [False, True])
+def test_tuner_is_judged_by_the_untuned_handle(get_case, tmp_path, monkeypatch, name, waves, picks_win):
+    """The step that the tuner compares with runs every kernel at the shape of a
+    handle without a table; picks that lose leave those shapes, here and in a
+    later handle of the mesh; picks that win are the ones that differ from them."""
+    from hexdyn import autotune
+    from hexdyn.driver import HexDycoreDriver
+
+    print(f"[gpu] tuner against the untuned handle {name}, picks win {picks_win}", flush=True)
+    monkeypatch.setenv("HEXDYN_CACHE", str(tmp_path))
+    passes = ("k_tend_mom_ac", "k_sc_edge", "k_rec_edge", "k_sub_edge")
+    d = HexDycoreDriver.from_host(get_case(name))
+    shapes = {k: autotune.get_launch(d, k) for k in passes}
+    assert shapes == {**dict.fromkeys(passes, waves), "k_sub_edge": 4}
+    seen = []
+
+    def times(drv, steps):  # k_sub_edge is fastest at 16, k_rec_edge at 4, the others at their own shape
+        w = autotune.get_launch(drv, "k_sub_edge")
+        best = {**shapes, "k_sub_edge": 16, "k_rec_edge": 4}
+        return {k: 1.0 + (w != best[k]) for k in passes}
+
+    def step_ms(drv, steps):
+        seen.append({k: autotune.get_launch(drv, k) for k in passes})
+        return 1.0 if len(seen) == 1 else 0.5 if picks_win else 2.0
+
+    monkeypatch.setattr(autotune, "_kernel_times", times)
+    monkeypatch.setattr(autotune, "_step_ms", step_ms)
+    rec = autotune.tune(d)
+    assert seen[0] == shapes
+    want = {"k_sub_edge": 16, **({"k_rec_edge": 4} if waves != 4 else {})}
+    assert seen[1] == {**shapes, **want}
+    assert rec["table"] == (want if picks_win else {})
+    left = {**shapes, **rec["table"]}
+    assert {k: autotune.get_launch(d, k) for k in passes} == left
+    d.close()
+    autotune.save(rec)
+    d = HexDycoreDriver.from_host(get_case(name))
+    assert d.tuning["table"] == rec["table"]
+    assert {k: autotune.get_launch(d, k) for k in passes} == left
+    d.close()
