@@ -22,6 +22,7 @@
 #include <thread>
 #include <sched.h>
 #include <atomic>
+#include <condition_variable>
 #include <system_error>
 #include <vector>
 
@@ -1647,6 +1648,10 @@ constexpr size_t kHalfBytes = (size_t)8 << 20;    // half of the staging
 constexpr size_t kPieceBytes = (size_t)2 << 20;    // a thread's share ends where a huge page of the array does
 constexpr size_t kCarrierBytes = (size_t)4 << 20;  // copied out per thread, at least
 constexpr int kCarriers = 8;
+// Looks of a carrier for the next round before it sleeps: longer than a round's
+// copy takes, since a woken thread comes late (256 looks: x1.10242 1.30 -> 1.36 ms,
+// x1.40962 4.04 -> 4.30; 1024: 1.35 and 4.20; 4096: the same as without sleep).
+constexpr int kLooks = 4096;
 
 struct Piece {
   char *dst;
@@ -1655,11 +1660,15 @@ struct Piece {
 };
 
 // One half of the staging fills from the device while the pieces of the other
-// are copied out by this thread, when it waits, and the carriers.
+// are copied out by this thread, when it waits, and the carriers.  The stream may
+// hold work of any length before the first copy: a carrier with nothing to carry
+// looks for a while, then sleeps.
 // rounds[r]: one past round r's last piece; its pieces lie in half r % 2.
 int download(hexdyn_handle *h, const std::vector<Piece> &pieces, const std::vector<int> &rounds, hipStream_t s) {
   const int n = (int)pieces.size();
   std::atomic<int> issued{0}, next{0}, closed{0};
+  std::mutex board;  // held where issued or closed change, for the carriers that sleep
+  std::condition_variable more;
   std::vector<std::atomic<int>> left(rounds.size());  // pieces of a round still in the staging
   for (size_t r = 0; r < rounds.size(); ++r) left[r].store(rounds[r] - (r ? rounds[r - 1] : 0));
   auto carry_one = [&]() {
@@ -1673,24 +1682,42 @@ int download(hexdyn_handle *h, const std::vector<Piece> &pieces, const std::vect
     left[r].fetch_sub(1, std::memory_order_release);
     return true;
   };
+  auto post = [&](std::atomic<int> &what, int value) {
+    {
+      std::lock_guard<std::mutex> hold(board);
+      what.store(value, std::memory_order_release);
+    }
+    more.notify_all();
+  };
+  auto carry = [&]() {
+    for (int looks = 0; !closed.load();) {
+      if (carry_one()) {
+        looks = 0;
+      } else if (++looks < kLooks) {
+        std::this_thread::yield();
+      } else {
+        std::unique_lock<std::mutex> hold(board);
+        more.wait(hold, [&]() { return closed.load() || next.load() < issued.load(); });
+        looks = 0;
+      }
+    }
+  };
   struct Carriers {
+    decltype(post) &post_closed;
     std::atomic<int> &closed;
     std::vector<std::thread> t;
     ~Carriers() {
-      closed.store(1);
+      post_closed(closed, 1);
       for (auto &x : t) x.join();
     }
-  } carriers{closed, {}};
+  } carriers{post, closed, {}};
   cpu_set_t cpus;
   const int have = sched_getaffinity(0, sizeof cpus, &cpus) == 0 ? CPU_COUNT(&cpus) : 1;
   size_t total = 0;
   for (const Piece &p : pieces) total += p.bytes;
   for (int i = 1; i < std::min({kCarriers, have, (int)std::min<size_t>(total / kCarrierBytes, kCarriers)}); ++i) {
     try {
-      carriers.t.emplace_back([&]() {
-        while (!closed.load())
-          if (!carry_one()) std::this_thread::yield();
-      });
+      carriers.t.emplace_back(carry);
     } catch (const std::system_error &) {
       break;  // no more threads to be had: those there are do it
     }
@@ -1714,7 +1741,7 @@ int download(hexdyn_handle *h, const std::vector<Piece> &pieces, const std::vect
       i = j;
     }
     if (hipStreamSynchronize(s) != hipSuccess) return HEXDYN_E_HIP;
-    issued.store(rounds[r], std::memory_order_release);
+    post(issued, rounds[r]);
   }
   if (rounds.size() > 1) wait_round(rounds.size() - 2);
   wait_round(rounds.size() - 1);

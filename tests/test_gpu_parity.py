@@ -1030,3 +1030,35 @@ def test_step_after_a_phase_outside_a_step(get_case, call):
     ref, got = o.get_state(), d.get_state()
     for k in ref:
         assert _bits_equal(ref[k], got[k]), f"{k}: {_diff(ref[k], got[k])}"
+
+
+def test_download_behind_queued_work_leaves_the_cores_alone(get_case):
+    """A download queued behind work on its stream waits for it without the
+    threads that carry the pieces out: the process's CPU time stays near the one
+    core that a synchronisation may take."""
+    import ctypes as ct
+    import time
+
+    from hexdyn.lib import lib
+
+    print("[gpu] download of 64 MiB behind queued matrix products", flush=True)
+    d = _driver(get_case("x1.162-moist"))
+    x = torch.rand(1 << 24, device="cuda")
+    host = np.empty(x.numel(), dtype=np.float32)
+    m = torch.rand(4096, 4096, device="cuda")
+
+    def download():
+        assert lib().hexdyn_download(d.handle, 1, (ct.c_void_p * 1)(host.ctypes.data), (ct.c_void_p * 1)(x.data_ptr()),
+                                     (ct.c_int64 * 1)(x.numel()), ct.c_void_p(d.stream_ptr())) == 0
+
+    download()
+    torch.cuda.synchronize()
+    for _ in range(400):
+        m @ m
+    w0, c0 = time.perf_counter(), time.process_time()
+    download()
+    wall, cpu = time.perf_counter() - w0, time.process_time() - c0
+    print(f"[gpu] waited {wall:.3f} s, CPU time {cpu:.3f} s", flush=True)
+    assert np.array_equal(host, x.cpu().numpy())
+    assert wall > 0.05, "too little work queued"
+    assert cpu < 2.5 * wall
