@@ -191,6 +191,26 @@ __global__ void __launch_bounds__(256) k_transfer(const XferList x) {
   }
 }
 
+// One field of few rows, a wavefront a row and no LDS: where a tile's chain of
+// steps takes longer than the accesses of 4 bytes that it saves.  A call with its
+// wait: up to 1920 rows 11.9-12.6 us against 13.1-13.7 in tiles; rows to levels at
+// 2562 rows 12.8 against 13.7, at 5120 14.2 against 13.7, at 7680 15.6 against
+// 13.8; levels to rows at 5120 12.9 against 13.5, at 7680 13.5 against 13.6, at
+// 10 242 14.1 against 13.7.
+constexpr int XFER_FEW_IN = 8192, XFER_FEW_OUT = 4096;  // rows (entities x planes) up to which a field goes this way
+template <bool IN>
+__global__ void __launch_bounds__(256) k_transfer_few(const XferField f, int rs) {
+  const int j = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+  const int k = (int)(threadIdx.x & 63), plane = (int)blockIdx.y;
+  if (j >= f.n || k >= rs) return;
+  float *row = f.rows + ((size_t)plane * f.n + f.row_of[j]) * rs;
+  float *logical = f.logical + (size_t)plane * f.nlev * f.n + j;
+  if (IN)
+    row[k] = k < f.nlev ? logical[(size_t)k * f.n] : 0.0f;
+  else if (k < f.nlev)
+    logical[(size_t)k * f.n] = row[k];
+}
+
 struct ProfEntry {
   std::vector<std::pair<hipEvent_t, hipEvent_t>> events;
 };
@@ -1149,6 +1169,15 @@ struct Transfer {
   }
 };
 int transfer(hexdyn_handle *h, const FieldRef &f, float *dev, bool to_internal, hipStream_t s) {
+  if (f.planes > 0 && (long long)f.n * f.planes <= (to_internal ? XFER_FEW_IN : XFER_FEW_OUT)) {
+    const XferField x{f.ptr, dev, f.row_of, f.n, f.nlev, 0};
+    const dim3 grid((f.n + 3) / 4, f.planes);
+    if (to_internal)
+      hipLaunchKernelGGL(k_transfer_few<true>, grid, dim3(256), 0, s, x, h->I.n.RS);
+    else
+      hipLaunchKernelGGL(k_transfer_few<false>, grid, dim3(256), 0, s, x, h->I.n.RS);
+    return hipGetLastError() == hipSuccess ? 0 : HEXDYN_E_HIP;
+  }
   Transfer t;
   t.add(f, dev);
   return t.run(h, to_internal, s);

@@ -1062,3 +1062,30 @@ def test_download_behind_queued_work_leaves_the_cores_alone(get_case):
     assert np.array_equal(host, x.cpu().numpy())
     assert wall > 0.05, "too little work queued"
     assert cpu < 2.5 * wall
+
+
+@pytest.mark.parametrize("name,nlev,species", [("x1.162-moist", 10, 7), ("x1.642-moist", 63, 7), ("x1.2562-moist", 26, 4),
+                                               ("x1.2562-moist", 55, 1)])
+def test_single_fields_by_row_count(get_case, name, nlev, species):
+    """A field alone goes a row at a time up to 4096 rows when exported and 8192 when
+    imported and in tiles above (here 162 to 10 248): the values of the whole state."""
+    import ctypes as ct
+
+    from hexdyn import capi
+    from hexdyn.lib import lib
+
+    print(f"[gpu] fields alone {name} L{nlev} T{species}", flush=True)
+    d = _driver(get_case(name, nlev=nlev, n_scalars=species, moist=True))
+    rng = np.random.default_rng(11)
+    first, second = ({k: rng.uniform(0.5, 2.0, s).astype(np.float32) for k, s in d.shapes.items()} for _ in range(2))
+    d.set_state(first, saved=first)
+    names = {k: k.upper() for k in d.shapes}
+    for k, f in names.items():
+        assert _bits_equal(first[k], d.export_field(f).cpu().numpy()), f
+    for k, f in names.items():
+        t = torch.from_numpy(second[k].reshape(-1, second[k].shape[-1])).cuda()
+        assert lib().hexdyn_import_field(d.handle, capi.FIELD_ID[f], ct.c_void_p(t.data_ptr()),
+                                         ct.c_void_p(d.stream_ptr())) == 0
+    got = d.get_state()
+    for k in names:
+        assert _bits_equal(second[k], got[k]), k
