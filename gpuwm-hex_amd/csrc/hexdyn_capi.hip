@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "../../include/hexdyn.h"
+#include "hexdyn_div.h"
 #include "hexdyn_internal.h"
 #include "hexdyn_powf.h"
 
@@ -460,6 +461,25 @@ float hexdyn_powf(float x, float y) {
   double near_tie = 0.0;
   const std::vector<uint32_t> &ties = gnu_powf_ties(rcv, &why, &near_tie);
   return why.empty() ? hexdyn_gnu_powf_fix(x, r, d, ties.data(), near_tie) : r;
+}
+
+namespace {
+__global__ void __launch_bounds__(256) k_quotient(const float *__restrict__ x, float *__restrict__ q, int64_t n,
+                                                  int count) {
+  const float c = (float)count, rc = 1.0f / c;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    const float v = x[i];
+    q[i] = count ? div_count(v, c, rc) : recip_in_range(v) ? recip(v) : 1.0f / v;
+  }
+}
+}  // namespace
+
+int hexdyn_quotient(const float *x, float *q, int64_t n, int count, void *stream) {
+  if (n < 0 || (n > 0 && (!x || !q)) || (count != 0 && (count < 3 || count > 7))) return HEXDYN_E_INVALID;
+  if (n == 0) return 0;
+  const unsigned blocks = (unsigned)std::min<int64_t>((n + 255) / 256, 4096);
+  hipLaunchKernelGGL(k_quotient, dim3(blocks), dim3(256), 0, (hipStream_t)stream, x, q, n, count);
+  return hipGetLastError() == hipSuccess ? 0 : HEXDYN_E_HIP;
 }
 
 namespace {

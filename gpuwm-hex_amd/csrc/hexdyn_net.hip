@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "../../include/hexdyn.h"
+#include "hexdyn_div.h"
 #include "hexdyn_internal.h"
 
 namespace hexdyn {
@@ -62,19 +63,6 @@ __device__ __forceinline__ int curve_block() {
   const int nb = (int)gridDim.x, b = (int)blockIdx.x;
   const int x = b & 7, i = b >> 3, q = nb >> 3, r = nb & 7;
   return (x < r) ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
-}
-
-// s / n for a neighbour count n in 3..7, rn = RN(1/n): the product with one
-// FMA residual correction is the correctly rounded quotient for quotients in
-// [2^-120, FLT_MAX] and for +0, which a relu leaves often (verified
-// exhaustively for every binary32 s and these n); other inputs take the
-// division.
-__device__ __forceinline__ float div_count(float s, float n, float rn) {
-  const float q0 = s * rn;
-  const float a = fabsf(q0);
-  if ((a >= 0x1p-120f && a <= 0x1.fffffep127f) || __float_as_uint(s) == 0u)
-    return __builtin_fmaf(__builtin_fmaf(-q0, n, s), rn, q0);
-  return s / n;
 }
 
 // ------------------------------------------------------------------ GEMM

@@ -29,6 +29,7 @@
  */
 #include <hip/hip_runtime.h>
 
+#include "hexdyn_div.h"
 #include "hexdyn_internal.h"
 #include "hexdyn_powf.h"
 
@@ -232,19 +233,6 @@ __device__ __forceinline__ void stage_levels(float *s_lev, const float *const (&
 #pragma unroll
   for (int j = 0; j < N; ++j)
     if (w == j) s_lev[j * 64 + k] = rows[j][k];
-}
-
-// 1 / x with IEEE round-to-nearest for |x| in [2^-100, 2^100]: the hardware
-// reciprocal with one FMA correction is the correctly rounded quotient there
-// (verified exhaustively over every binary32 x of that range).  Callers take
-// the division outside it.
-__device__ __forceinline__ bool recip_in_range(float x) {
-  const float a = fabsf(x);
-  return a >= 0x1p-100f && a <= 0x1p100f;
-}
-__device__ __forceinline__ float recip(float x) {
-  const float y0 = __builtin_amdgcn_rcpf(x);
-  return __builtin_fmaf(__builtin_fmaf(-x, y0, 1.0f), y0, y0);
 }
 
 // Value of lane k-1 (lane 0: zero) and k+1 (lane 63: zero): whole-wave DPP

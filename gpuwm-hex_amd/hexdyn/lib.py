@@ -67,6 +67,7 @@ def lib() -> ct.CDLL:
     L.hexdyn_profile_kernels.argtypes = [vp, ct.c_char_p, ct.c_size_t]
     L.hexdyn_powf.argtypes = [ct.c_float, ct.c_float]
     L.hexdyn_powf.restype = ct.c_float
+    L.hexdyn_quotient.argtypes = [vp, vp, ct.c_int64, ct.c_int, vp]
     L.hexdyn_integrals.argtypes = [vp, ct.POINTER(ct.c_double), ct.c_int, vp]
     L.hexdyn_integrals_noalloc.argtypes = [vp, vp, ct.c_int, vp]
     L.hexdyn_copy_state.argtypes = [vp, vp, vp]
@@ -110,7 +111,7 @@ EXPORTED = [
     "hexdyn_profile_kernels", "hexdyn_powf", "hexdyn_integrals", "hexdyn_set_graphs",
     "hexdyn_set_physics_tendencies", "hexdyn_set_post_transport_clamp", "hexdyn_last_create_error",
     "hexdyn_graph_count", "hexdyn_integrals_noalloc", "hexdyn_copy_state", "hexdyn_set_launch",
-    "hexdyn_get_launch", "hexdyn_download",
+    "hexdyn_get_launch", "hexdyn_download", "hexdyn_quotient",
     "hexdyn_net_create", "hexdyn_net_destroy", "hexdyn_net_param_count", "hexdyn_net_set_params",
     "hexdyn_net_get_params", "hexdyn_net_get_grads", "hexdyn_net_set_scales", "hexdyn_net_forward",
     "hexdyn_net_set_target", "hexdyn_net_loss", "hexdyn_net_backward", "hexdyn_net_adam", "hexdyn_net_apply",

@@ -405,6 +405,12 @@ int hexdyn_integrals_noalloc(hexdyn_handle *h, double *out_device, int n_out, vo
  * The first call builds the process's correction bitmap (about 0.7 s). */
 float hexdyn_powf(float x, float y);
 
+/* The kernels' quotients by a corrected product over n values, exposed for their
+ * tests: count 0 gives 1 / x (the column recurrences), count 3..7 gives x / count
+ * (the corrector's neighbour mean), each the bits of the IEEE division.  Device
+ * pointers; enqueued on stream. */
+int hexdyn_quotient(const float *x, float *q, int64_t n, int count, void *stream);
+
 #ifdef __cplusplus
 }
 #endif
