@@ -1089,3 +1089,37 @@ def test_single_fields_by_row_count(get_case, name, nlev, species):
     got = d.get_state()
     for k in names:
         assert _bits_equal(second[k], got[k]), k
+
+
+@pytest.mark.parametrize("splits,substeps", [(1, 4), (3, 2)])
+@pytest.mark.parametrize("field,scale", [("exner", 1e15), ("exner", 1e30), ("exner", np.inf), ("w", np.inf), ("w", np.nan)])
+def test_whole_step_with_a_column_out_of_range(get_case, splits, substeps, field, scale):
+    """One column with a field scaled out of range at its upper half, through the
+    stages' whole column passes: their coefficients take the division (exner), the
+    recurrences carry what is not finite, the step is refused as the oracle's is,
+    and its working fields are the oracle's, NaN where NaN is."""
+    import dataclasses
+
+    print(f"[gpu] x1.2562-moist whole step, {splits} subcycles, {field} x {scale} in one column", flush=True)
+    base = get_case("x1.2562-moist")
+    case = get_case("x1.2562-moist", nlev=26, n_scalars=1, moist=True, config=dataclasses.replace(
+        base.config, config_dt=600.0, config_dynamics_split_steps=splits, config_number_of_sub_steps=substeps))
+    o = Oracle(case, 32)
+    o.set_state(initial_state_arrays(case), rebuild=True)
+    a = o.get_state()
+    a[field][13:, 1234] = (a[field][13:, 1234] + np.float32(1e-3)) * np.float32(scale)
+    o.set_state(a, rebuild=False)
+    d = _driver(case)
+    d.set_state(a, saved=a)
+    assert o.step(1) != 0
+    with pytest.raises(FloatingPointError, match="validation flag"):
+        d.step_device(1)
+    share = []
+    for f in ("TEND_RU", "TEND_RT", "TEND_RW", "TEND_RHO", "RU_P", "RW_P", "RHO_PP", "RTHETA_PP", "RU_AVG", "WW_AVG",
+              "ALPHA_TRI", "GAMMA_TRI", "COFWZ", "COFWT", "COFTZ", "EULER_RU", "EULER_RW"):
+        y = d.export_field(f).cpu().numpy().ravel()
+        x = np.asarray(o.export_field(f)).ravel()
+        share.append(np.isfinite(x).mean())
+        same = (x.view(np.uint32) == y.view(np.uint32)) | (np.isnan(x) & np.isnan(y))
+        assert same.all(), f"{f}: {(~same).sum()} differ"
+    assert 0.2 < min(share) < 1.0
