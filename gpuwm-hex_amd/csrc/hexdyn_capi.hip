@@ -1020,10 +1020,10 @@ static int create_impl(const hexdyn_mesh *m, const hexdyn_vertical *vt, const he
   float **edge_bufs[] = {&B.ru, &B.u, &B.p_u, &B.c_ru, &B.s_ru, &B.cqu, &B.euler_ru, &B.tend_ru, &B.fth,
                          &B.fcorr, &B.fw, &B.ru_p, &B.ru_avg, &B.v, &B.pv_edge, &B.flux_u, &B.split_u};
   for (float **p : edge_bufs) rc |= h->alloc(p, er);
-  float **vert_bufs[] = {&B.vorticity, &B.ke_vertex, &B.pv_vertex};
+  float **vert_bufs[] = {&B.vorticity, &B.pv_vertex};
   for (float **p : vert_bufs) rc |= h->alloc(p, vr);
-  float **scal_bufs[] = {&B.q, &B.q_stage, &B.q_next, &B.fct_mn, &B.fct_mx, &B.fct_mass, &B.fct_sin,
-                         &B.fct_sout, &B.fct_vres};
+  if (!n.VP) rc |= h->alloc(&B.ke_vertex, vr);
+  float **scal_bufs[] = {&B.q, &B.q_stage, &B.q_next, &B.fct_mass, &B.fct_sin, &B.fct_sout, &B.fct_vres};
   for (float **p : scal_bufs) rc |= h->alloc(p, sr);
   float **sedge_bufs[] = {&B.ev, &B.fct_hres};
   for (float **p : sedge_bufs) rc |= h->alloc(p, ser);

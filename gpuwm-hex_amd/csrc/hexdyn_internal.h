@@ -137,12 +137,12 @@ struct Work {
   // acoustic
   float *ru_p, *ru_avg, *rw_p, *ww_avg, *rho_pp, *rtheta_pp, *rtheta_pp_old;
   // diagnostics
-  float *v, *pv_edge, *ke, *divergence, *vorticity, *ke_vertex, *pv_vertex, *pv_cell;
+  float *v, *pv_edge, *ke, *divergence, *vorticity, *pv_vertex, *pv_cell;
+  float *ke_vertex;  // of the vertex pass (Sizes::VP 0 only)
   // fluxes
   float *flux_u, *flux_w, *split_u, *split_w;
   // transport
-  float *q_stage, *q_next, *target, *ev, *fct_mn, *fct_mx, *fct_mass, *fct_sin, *fct_sout, *fct_vres,
-      *fct_hres;
+  float *q_stage, *q_next, *target, *ev, *fct_mass, *fct_sin, *fct_sout, *fct_vres, *fct_hres;
   // horizontal mixing: viscosity, Laplacians and the theta Euler pool
   float *kdiff, *delsq_u, *delsq_div, *delsq_vort, *delsq_theta, *delsq_w, *mix_tw, *euler_theta;
   // held physics tendencies (rows; allocated when first installed)

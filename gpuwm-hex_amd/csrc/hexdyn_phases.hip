@@ -2048,7 +2048,6 @@ __global__ void __launch_bounds__(64 * COLW_AC)
   const int k = lane();
   const int L = I.n.L;
   const int n = I.m.neoc[c];
-  const bool inner = k >= 1 && k < L;
   int e[NE], o[NE];
 #pragma unroll
   for (int s = 0; s < NE; ++s) {
