@@ -803,7 +803,7 @@ static int create_impl(const hexdyn_mesh *m, const hexdyn_vertical *vt, const he
   rc |= h->upload(&M.vdc, vdc); rc |= h->upload(&M.vdcdv, vdcdv);
   rc |= h->upload(&M.ecos, ecos); rc |= h->upload(&M.esin, esin); rc |= h->upload(&M.ocell, ocell);
   n.OCP = ocp;
-  h->tune.large = n.E > 4 * HX_RESIDENT;
+  h->tune.large = n.E > 4 * HX_SMALL;
   if (mixing) {
     // binary32 scalars staged as the reference host does (cuda_horizontal_v841.py:1336-1350)
     const float len = c->config_len_disp, csm = c->config_smagorinsky_coef;
@@ -1467,7 +1467,7 @@ Instance step_view(const hexdyn_handle *h, bool recovery) {
 int enqueue_step(hexdyn_handle *h, hipStream_t s) {
   const hexdyn_config &c = h->cfg;
   const bool transport = c.config_split_dynamics_transport && transported(h);
-  const int w_later = transport && h->I.n.E + h->I.n.C <= HX_RESIDENT ? 1 : 0;  // see k_sc_edge_w
+  const int w_later = transport && h->I.n.E + h->I.n.C <= HX_SMALL ? 1 : 0;  // see k_sc_edge_w
   int rc = run_phase_begin_step(h, s, true);
   for (int sub = 1; rc == 0 && sub <= c.config_dynamics_split_steps; ++sub) {
     h->cur_sub = sub;

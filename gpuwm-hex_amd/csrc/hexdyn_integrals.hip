@@ -71,7 +71,10 @@ constexpr int IQ = 6;
 // the rows a wavefront needs, the species' too, are loaded before the first
 // sum: each sum is a chain of lane exchanges, and a species' load behind the
 // sum before it is one more round trip.  26.9 -> 21.9 us at x1.10242 with six
-// species, 17.8 with the sums' exchanges in registers.
+// species, 17.8 with the sums' exchanges in registers.  A group is summed whole,
+// species past the last one too: a call with its wait takes 33.2, 37.9 and 42.8 us
+// for one, six and seven species there (52.6, 73.8 and 77.1 with one species after
+// another, their exchanges through the permute unit).
 template <int NE>
 __global__ void __launch_bounds__(256) k_integrals(const Instance I, const IntegralArgs a, double *partial) {
   extern __shared__ double s_part[];  // [4 waves][NQ]

@@ -34,11 +34,16 @@ struct Sizes {
   int WPB = 4;
 };
 
+// Wavefronts of a small launch.  The rules that choose a launch's form by it
+// (species_rows, k_sc_edge_w, LaunchTune::large) draw measured lines: below, one
+// wavefront's chain of memory round trips sets the time, above, the chip does.  It
+// is 32 wavefronts on each of 256 CUs, an MI355X's most; a kernel of more than 64
+// registers holds fewer at once.
+constexpr int HX_SMALL = 256 * 32;
+constexpr int HX_VREC = 8;  // values of one vertex in its cell's record (Mesh::vrec)
 // Edge tiles of the staged flux gathers: HX_TILE_E edges per block, at most
 // HX_TILE_U distinct advection cells per tile (larger tiles turn the staged
 // kernels off for the mesh).
-constexpr int HX_RESIDENT = 256 * 32;  // wavefronts the chip holds at once, 32 on each of 256 CUs
-constexpr int HX_VREC = 8;  // values of one vertex in its cell's record (Mesh::vrec)
 constexpr int HX_TILE_E = 8;
 constexpr int HX_TILE_U = 56;
 
@@ -196,7 +201,7 @@ struct LaunchTune {
   static constexpr int kMax = 64;
   int n = 0;
   int def = 0;  // kernels not listed; 0: default_wpb
-  bool large = false;  // a mesh of more edges than four times the wavefronts the chip holds
+  bool large = false;  // a mesh of more than 4 * HX_SMALL edges
   char names[kMax][32];
   int wpb[kMax];
   int find(const char *name) const {
@@ -213,8 +218,9 @@ struct LaunchTune {
   // 62.7 at 8 (x1.40962), k_sc_edge 122.7 and 119.0, k_rec_edge 48.2 and 47.4; a
   // step 5101 -> 5053 us, x1.163842 18.30 -> 18.20 ms, 8 x x1.2562 2492 -> 2469 us.
   // The others lose or are even (k_fct_edge1 158 and 171, k_sub_edge 59.2 and
-  // 61.2), as do all on meshes that fit the chip a few times over (x1.2562 403
-  // and 408 us a step, x1.10242 the same).
+  // 61.2), as do all on smaller meshes (x1.2562 403 and 408 us a step, x1.10242
+  // the same).  The line lies between the 30 720 edges of x1.10242, where nothing
+  // is gained, and the 61 440 of 8 x x1.2562, which gain 1 %.
   int default_wpb(const char *name) const {
     if (large)
       for (const char *k : {"k_tend_mom_ac", "k_sc_edge", "k_rec_edge"})

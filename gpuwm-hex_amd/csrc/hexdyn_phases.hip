@@ -217,12 +217,13 @@ inline int nblocks(int n, int wpb) { return (n + wpb - 1) / wpb; }
 
 // Column kernels: W cells (one wavefront each) per block, which share the
 // per-level coefficient rows in LDS.  The implicit coefficients on their own
-// take 16 columns per block, the acoustic column update (8 columns: the same
-// time, 16: 57 us for 53) and a stage's whole column pass 4.
+// take 16 columns per block, the acoustic column update and a stage's whole column
+// pass 4 (a x1.40962 step with 2, 4 and 8 columns: 5049, 5030 and 5042 us).
 constexpr int COLW_VC = 16;  // k_vcoef
 constexpr int COLW_AC = 4;   // k_ac_cell and k_col
-// The column blocks of a CU need every SIMD to hold 8 wavefronts: the
-// register budget is capped for that (at 7 a CU would hold one block of 16).
+// Registers of k_vcoef and k_ac_cell for 8 wavefronts per SIMD: at 7 a CU would
+// hold one block of 16 columns instead of two, and the acoustic update at 6 takes
+// 87 us for 82 (x1.40962).
 #define KBCOL(W) __global__ void __launch_bounds__(64 * (W)) __attribute__((amdgpu_waves_per_eu(8, 8)))
 
 // Per-level coefficient rows are the same for every column of a block: wave
@@ -2025,11 +2026,11 @@ KBCOL(COLW_AC) k_ac_cell(const Instance I, float dts, int store_old, const RecAr
 // stream of the coefficients gone.
 // The coefficients wait in LDS until the acoustic part, and its rows are loaded
 // when the theta part has freed its registers.  Wavefronts per SIMD: as many as
-// hold the pass without spills, seven (six with coefficients and correction
-// flux, or seven-edge cells); a CU then holds seven or six blocks of four
-// columns, and the chains of some run under the loads of the others.  At eight
-// wavefronts 3-11 registers spill, and their traffic costs more than the
-// occupancy gives: 119 + 166 + 112 us a subcycle's three stages at x1.40962
+// hold the pass without a vector register in memory, seven (six with coefficients
+// and correction flux, or seven-edge cells; up to 34 scalar registers wait in lanes
+// of vector registers); a CU then holds seven or six blocks of four columns, and
+// the chains of some run under the loads of the others.  At eight wavefronts 3-11
+// vector registers spill, and their traffic costs more than the occupancy gives: 119 + 166 + 112 us a subcycle's three stages at x1.40962
 // against 95 + 116 + 93, both with the columns swept out of LDS (blocks of eight
 // columns at six: 103 + 120 + 93).
 template <int NE, bool VC, bool CORR, bool MIX, bool LAST, bool S3>
@@ -2524,10 +2525,11 @@ KB k_sc_edge(const Instance I, const float *__restrict__ qs, float *__restrict__
   if (e < I.n.E) sc_edge<NE>(I, e, lane(), qs, ev);
 }
 // The transport's first edge pass and the recovery of w that ends the dynamics,
-// neither of which reads what the other writes, in one launch where the
-// wavefronts of both are resident at once: a x1.162 step 288 -> 281 us.  Above,
-// the shared launch is slower than the two (174.5 us against 122.2 + 36.8 at
-// x1.40962, 40.6 against 29.5 + 10.2 at x1.10242).
+// neither of which reads what the other writes, in one launch where both
+// together are small (HX_SMALL: meshes of 642 cells take it, 2562 do not): a
+// x1.162 step 288 -> 281 us.  On large meshes the shared launch is slower than
+// the two (174.5 us against 122.2 + 36.8 at x1.40962, 40.6 against 29.5 + 10.2 at
+// x1.10242).
 template <int NE>
 KB k_sc_edge_w(const Instance I, int nb0, const float *__restrict__ qs, float *__restrict__ ev) {
   if ((int)blockIdx.x < nb0) {
@@ -3258,15 +3260,15 @@ int recover(const Instance &I, int stage, int sub, int damp, int w_later, hipStr
 }
 
 // Grid rows of a scalar pass over n entities in batches of g species: a row a
-// batch where every wavefront of all batches is resident at once (32 on each of
-// 256 CUs), so that the batches run side by side instead of one memory round trip
-// after another: a step with six species 280 -> 266 us at x1.162, 341 -> 332 at
-// x1.642, 470 -> 465 at x1.2562.  Above, the batches fill the chip as well one
-// after the other and share the species-independent rows: 1177 us at x1.10242,
-// 1183 with a row a batch.
+// batch where the launch stays small (HX_SMALL), so that the batches run side by
+// side instead of one memory round trip after another: a step with six species
+// 280 -> 266 us at x1.162, 341 -> 332 at x1.642, 470 -> 465 at x1.2562 (there the
+// cell passes alone).  Above, the batches fill the chip as well one after the other
+// and share the species-independent rows: 1177 us at x1.10242, 1183 with a row a
+// batch.
 inline int species_rows(const Instance &I, int n, int g) {
   const int batches = (I.n.NT + g - 1) / g;
-  return (long long)n * batches <= HX_RESIDENT ? batches : 1;
+  return (long long)n * batches <= HX_SMALL ? batches : 1;
 }
 
 int scalars_stage(const Instance &I, int stage, int with_w, hipStream_t s) {
