@@ -3268,7 +3268,7 @@ int recover(const Instance &I, int stage, int sub, int damp, int w_later, hipStr
 // batch.
 inline int species_rows(const Instance &I, int n, int g) {
   const int batches = (I.n.NT + g - 1) / g;
-  return (long long)n * batches <= HX_SMALL ? batches : 1;
+  return batches > 1 && (long long)n * batches <= HX_SMALL ? batches : 1;  // without species a launch of one row
 }
 
 int scalars_stage(const Instance &I, int stage, int with_w, hipStream_t s) {

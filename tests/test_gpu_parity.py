@@ -1123,3 +1123,26 @@ def test_whole_step_with_a_column_out_of_range(get_case, splits, substeps, field
         same = (x.view(np.uint32) == y.view(np.uint32)) | (np.isnan(x) & np.isnan(y))
         assert same.all(), f"{f}: {(~same).sum()} differ"
     assert 0.2 < min(share) < 1.0
+
+
+@pytest.mark.parametrize("monotonic", [False, True])
+def test_transport_phases_without_species(get_case, monotonic):
+    """A host that runs the transport phases whatever the species count: on a dry
+    case they are accepted and change nothing, a step by phases as the whole step."""
+    import dataclasses
+
+    print(f"[gpu] x1.162 dry, transport phases, monotonic {monotonic}", flush=True)
+    base = get_case("x1.162-moist")
+    case = get_case("x1.162-moist", n_scalars=0, moist=False,
+                    config=dataclasses.replace(base.config, config_monotonic=monotonic))
+    assert not _phase_walk(case)
+    o = Oracle(case, 32)
+    o.set_state(initial_state_arrays(case), rebuild=True)
+    assert o.step(1) == 0
+    d = _driver(case)
+    for st in (1, 2, 3):
+        d.phase("scalars", st)
+    d.step_device(1)
+    ref, got = o.get_state(), d.get_state()
+    for k in ref:
+        assert _bits_equal(ref[k], got[k]), f"{k}: {_diff(ref[k], got[k])}"
